@@ -105,7 +105,7 @@ struct PathBuffers
 	float4* shadowPot;     /* contribution.xyz, path slot bits */
 	uint32_t* occluded;
 	float4* pathAcc;       /* per path slot, summed in path order */
-	uint32_t* counters;    /* [0] extension count in, [1] extension out, [2] shadow, [3] trace work counter, [4] second trace counter */
+	uint32_t* counters;    /* [0] extension count in, [2] shadow rays out, [3] extension rays out (one 64-bit atomic adds to both), 8-byte aligned */
 	float2* aux[2];        /* optix7 estimator: postponed bsdf pdf, packed normal of the last vertex */
 };
 
@@ -149,7 +149,7 @@ hipError_t launch_generateF(const CamParams& c, const ShadeParams& p, uint32_t j
 hipError_t launch_shadeF(const ShadeParams& p, const PathBuffers& b, int in, int maxCount, hipStream_t s);
 /* MAXPATHLENGTH of RenderCore_Optix7Filter (core_settings.h:25) */
 static const int MAXPATHLENGTH_FILTER = 7;
-/* counters[0] = counters[1] (next wave size, also logged), counters[1] = counters[2] = 0.
+/* counters[0] = counters[3] (next wave size, also logged), counters[2] = counters[3] = 0.
  * snapshot (if given) receives counters[0..3] as they were before; live (if
  * given, may be pinned host memory) the next wave size. */
 hipError_t launch_advance(uint32_t* counters, uint32_t* logSlot, hipStream_t s, uint32_t* snapshot = nullptr, uint32_t* live = nullptr);
