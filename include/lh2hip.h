@@ -227,6 +227,24 @@ LH2HIP_API int lh2hip_dn_conv3x3_dw(const void* x, int Cin, const void* dy, int 
  * share the array and race; results equal lh2hip_dn_conv3x3_dw's. */
 LH2HIP_API uint64_t lh2hip_dn_dw_scratch_bytes(void);
 LH2HIP_API int lh2hip_dn_conv3x3_dw_noalloc(const void* x, int Cin, const void* dy, int Cout, int H, int W, float* dw, float* db, void* stream);
+/* Weight gradients of several layers in one launch: per layer as
+ * lh2hip_dn_conv3x3_dw; coarse non-NULL: the layer's input is the concatenation
+ * [2x upsample of coarse, x] (Cin 64), read from its two tensors. At most 32
+ * layers, one with Cin 64 counting twice. ws: lh2hip_dn_dw_batch_workspace_bytes
+ * (0: a shape that is not supported). No counterpart in the reference. */
+typedef struct { const void* x; const void* coarse; const void* dy; float* dw; float* db; int Cin, Cout, H, W; } lh2hip_dn_layer;
+LH2HIP_API uint64_t lh2hip_dn_dw_batch_workspace_bytes(const lh2hip_dn_layer* layers, int n);
+LH2HIP_API int lh2hip_dn_conv3x3_dw_batch(const lh2hip_dn_layer* layers, int n, void* ws, uint64_t wsBytes, void* stream);
+/* Input gradients with the next steps of the backward pass in their epilogue
+ * (w: the flipped weights of lh2hip_dn_adam; 16-byte aligned tensors):
+ * dx_relu: gx = act > 0 ? conv3x3(gy, w) : 0 (Cin 16 or 32, Cout 32);
+ * dx_cat: of the convolution of a concatenation (32 to 64 channels), gskip =
+ * channels 32..63, gcoarse = 2x2 sums of channels 0..31 where actCoarse > 0.
+ * pool2_bwd_relu: out = act > 0 ? skip + dy / 4 : 0 (C 8 times a power of two).
+ * Each equals the calls it replaces bit for bit. */
+LH2HIP_API int lh2hip_dn_conv3x3_dx_relu(const void* gy, int Cin, const void* w, const void* act, void* gx, int Cout, int H, int W, void* stream);
+LH2HIP_API int lh2hip_dn_conv3x3_dx_cat(const void* gy, const void* w, const void* actCoarse, void* gcoarse, void* gskip, int H, int W, void* stream);
+LH2HIP_API int lh2hip_dn_pool2_bwd_relu(const void* dy, const void* skip, const void* act, int C, int H, int W, void* out, void* stream);
 LH2HIP_API int lh2hip_dn_relu_bwd(const void* y, const void* dy, void* dyPre, uint64_t n, void* stream);
 LH2HIP_API int lh2hip_dn_pool2(const void* x, int C, int H, int W, void* y, void* stream);
 LH2HIP_API int lh2hip_dn_pool2_bwd(const void* dy, int C, int H, int W, void* dx, int accumulate, void* stream);
@@ -256,6 +274,9 @@ LH2HIP_API int lh2hip_dn_relmse(const float* out, int Cout, const lh2_float4* ta
  * skip): bf16 weights in the forward layout and flipped for the input gradient. */
 LH2HIP_API int lh2hip_dn_adam(float* p, float* m, float* v, const float* g, uint64_t n, float lr, float b1, float b2, float eps, int t,
 	void* wfwd, void* wbwd, int Cout, int Cin, void* stream);
+/* lh2hip_dn_adam on several tensors, one launch per 48. */
+typedef struct { float* p; float* m; float* v; const float* g; void* wfwd; void* wbwd; uint64_t n; int Cout, Cin; } lh2hip_dn_tensor;
+LH2HIP_API int lh2hip_dn_adam_batch(const lh2hip_dn_tensor* tensors, int n, float lr, float b1, float b2, float eps, int t, void* stream);
 
 /* ---- render job server ---------------------------------------------------
  * No counterpart in the reference (its nearest is the asynchronous Render +

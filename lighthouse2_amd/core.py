@@ -64,6 +64,12 @@ _SIGS = {
     "lh2hip_dn_conv3x3_dw": (I, [P, I, P, I, I, I, P, P, P, P]),
     "lh2hip_dn_dw_scratch_bytes": (ctypes.c_uint64, []),
     "lh2hip_dn_conv3x3_dw_noalloc": (I, [P, I, P, I, I, I, P, P, P]),
+    "lh2hip_dn_dw_batch_workspace_bytes": (ctypes.c_uint64, [P, I]),
+    "lh2hip_dn_conv3x3_dw_batch": (I, [P, I, P, ctypes.c_uint64, P]),
+    "lh2hip_dn_conv3x3_dx_relu": (I, [P, I, P, P, P, I, I, I, P]),
+    "lh2hip_dn_conv3x3_dx_cat": (I, [P, P, P, P, P, I, I, P]),
+    "lh2hip_dn_pool2_bwd_relu": (I, [P, P, P, I, I, I, P, P]),
+    "lh2hip_dn_adam_batch": (I, [P, I, ctypes.c_float, ctypes.c_float, ctypes.c_float, ctypes.c_float, I, P]),
     "lh2hip_dn_relu_bwd": (I, [P, P, P, ctypes.c_uint64, P]),
     "lh2hip_dn_pool2": (I, [P, I, I, I, P, P]),
     "lh2hip_dn_pool2_bwd": (I, [P, I, I, I, P, I, P]),

@@ -396,6 +396,42 @@ LH2HIP_API int lh2hip_dn_conv3x3_dw_noalloc(const void* x, int Cin, const void* 
 		"dn_conv3x3_dw_noalloc (Cin x Cout in 16x32, 32x32, 64x32, 32x16, 16x16; W <= 32768)");
 }
 
+static_assert(sizeof(lh2hip_dn_layer) == sizeof(lh::DwLayer) && sizeof(lh2hip_dn_tensor) == sizeof(lh::AdamTensor), "C mirrors of the batch records");
+
+LH2HIP_API uint64_t lh2hip_dn_dw_batch_workspace_bytes(const lh2hip_dn_layer* layers, int n)
+{
+	return lh::dn_dw_batch_workspace_bytes((const lh::DwLayer*)layers, n);
+}
+
+LH2HIP_API int lh2hip_dn_conv3x3_dw_batch(const lh2hip_dn_layer* layers, int n, void* ws, uint64_t wsBytes, void* stream)
+{
+	return dn_status(lh::dn_conv3x3_dw_batch((const lh::DwLayer*)layers, n, ws, (size_t)wsBytes, (hipStream_t)stream),
+		"dn_conv3x3_dw_batch (supported layers, workspace large enough)");
+}
+
+LH2HIP_API int lh2hip_dn_conv3x3_dx_relu(const void* gy, int Cin, const void* w, const void* act, void* gx, int Cout, int H, int W, void* stream)
+{
+	return dn_status(lh::dn_conv3x3_dx_relu((const lh::bf16_t*)gy, Cin, (const lh::bf16_t*)w, (const lh::bf16_t*)act, (lh::bf16_t*)gx, Cout, H, W,
+		(hipStream_t)stream), "dn_conv3x3_dx_relu (16 or 32 to 32 channels, 16-byte aligned)");
+}
+
+LH2HIP_API int lh2hip_dn_conv3x3_dx_cat(const void* gy, const void* w, const void* actCoarse, void* gcoarse, void* gskip, int H, int W, void* stream)
+{
+	return dn_status(lh::dn_conv3x3_dx_cat((const lh::bf16_t*)gy, (const lh::bf16_t*)w, (const lh::bf16_t*)actCoarse, (lh::bf16_t*)gcoarse,
+		(lh::bf16_t*)gskip, H, W, (hipStream_t)stream), "dn_conv3x3_dx_cat (even H, W, 16-byte aligned)");
+}
+
+LH2HIP_API int lh2hip_dn_pool2_bwd_relu(const void* dy, const void* skip, const void* act, int C, int H, int W, void* out, void* stream)
+{
+	return dn_status(lh::dn_pool2_bwd_relu((const lh::bf16_t*)dy, (const lh::bf16_t*)skip, (const lh::bf16_t*)act, C, H, W, (lh::bf16_t*)out,
+		(hipStream_t)stream), "dn_pool2_bwd_relu (even H, W, C 8 times a power of two, 16-byte aligned)");
+}
+
+LH2HIP_API int lh2hip_dn_adam_batch(const lh2hip_dn_tensor* tensors, int n, float lr, float b1, float b2, float eps, int t, void* stream)
+{
+	return dn_status(lh::dn_adam_batch((const lh::AdamTensor*)tensors, n, lr, b1, b2, eps, t, (hipStream_t)stream), "dn_adam_batch");
+}
+
 LH2HIP_API int lh2hip_dn_relu_bwd(const void* y, const void* dy, void* dyPre, uint64_t n, void* stream)
 {
 	return dn_status(lh::dn_relu_bwd((const lh::bf16_t*)y, (const lh::bf16_t*)dy, (lh::bf16_t*)dyPre, (size_t)n, (hipStream_t)stream), "dn_relu_bwd");

@@ -39,6 +39,33 @@ hipError_t dn_conv3x3_dw(const bf16_t* x, int Cin, const bf16_t* dy, int Cout, i
  * dn_dw_scratch_bytes() (no allocation; calls overlapping on one device race). */
 size_t dn_dw_scratch_bytes();
 hipError_t dn_conv3x3_dw_noalloc(const bf16_t* x, int Cin, const bf16_t* dy, int Cout, int H, int W, float* dw, float* db, hipStream_t s);
+/* Weight gradients of several layers in one launch (and one for the partial
+ * sums): per layer as dn_conv3x3_dw; coarse non-null: the layer's input is the
+ * concatenation [2x upsample of coarse, x] (Cin 64) read from its halves. At
+ * most 32 layers, a layer with Cin 64 counting twice. ws: at least
+ * dn_dw_batch_workspace_bytes (0: unsupported). */
+struct DwLayer
+{
+	const bf16_t* x;
+	const bf16_t* coarse;
+	const bf16_t* dy;
+	float* dw;
+	float* db;
+	int Cin, Cout, H, W;
+};
+size_t dn_dw_batch_workspace_bytes(const DwLayer* layers, int n);
+hipError_t dn_conv3x3_dw_batch(const DwLayer* layers, int n, void* ws, size_t wsBytes, hipStream_t s);
+/* Input gradient (w: the flipped weights, Cin channels of gy to 32 of gx) with
+ * the ReLU gradient of the layer below: gx = act > 0 ? conv3x3(gy, w) : 0.
+ * 16-byte aligned tensors. */
+hipError_t dn_conv3x3_dx_relu(const bf16_t* gy, int Cin, const bf16_t* w, const bf16_t* act, bf16_t* gx, int Cout, int H, int W, hipStream_t s);
+/* Input gradient of the convolution of a concatenation (32 channels of gy, 64 of
+ * the input): gskip = channels 32..63, gcoarse = the 2x2 sums of channels
+ * 0..31 where actCoarse > 0, else 0 (dn_conv3x3, dn_upcat_bwd, dn_relu_bwd). */
+hipError_t dn_conv3x3_dx_cat(const bf16_t* gy, const bf16_t* w, const bf16_t* actCoarse, bf16_t* gcoarse, bf16_t* gskip, int H, int W, hipStream_t s);
+/* out = act > 0 ? skip + dy / 4 (dy of the 2x2 average) : 0: dn_pool2_bwd
+ * (accumulating into skip) followed by dn_relu_bwd. */
+hipError_t dn_pool2_bwd_relu(const bf16_t* dy, const bf16_t* skip, const bf16_t* act, int C, int H, int W, bf16_t* out, hipStream_t s);
 hipError_t dn_relu_bwd(const bf16_t* y, const bf16_t* dy, bf16_t* dyPre, size_t n, hipStream_t s);
 /* 2x2 average pool (H, W even) and its gradient (dx = or += dy / 4). */
 hipError_t dn_pool2(const bf16_t* x, int C, int H, int W, bf16_t* y, hipStream_t s);
@@ -57,6 +84,19 @@ hipError_t dn_relmse(const float* out, int Cout, const float4* target, int H, in
  * wbwd[8 - tap][Cin][Cout] used by the input-gradient convolution. */
 hipError_t dn_adam(float* p, float* m, float* v, const float* g, size_t n, float lr, float b1, float b2, float eps, int t,
 	bf16_t* wfwd, bf16_t* wbwd, int Cout, int Cin, hipStream_t s);
+/* dn_adam on several tensors with one launch per 48 (g null: only the bf16 copies). */
+struct AdamTensor
+{
+	float* p;
+	float* m;
+	float* v;
+	const float* g;
+	bf16_t* wfwd;
+	bf16_t* wbwd;
+	size_t n;
+	int Cout, Cin;
+};
+hipError_t dn_adam_batch(const AdamTensor* t, int n, float lr, float b1, float b2, float eps, int step, hipStream_t s);
 
 /* Network input from a filter-estimator frame: radiance = (direct + indirect)
  * sums * invSpp, demodulated by the G-buffer albedo and range-compressed,

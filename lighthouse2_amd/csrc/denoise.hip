@@ -11,12 +11,11 @@
  * output channels, K = 9 taps x input channels; activations are NHWC, so the
  * 4 k-values a lane needs are 4 consecutive channels of one pixel (one 8-byte
  * load) and the weights [tap][n][k] give the same for B.
- * Weight gradient: M = output channels, N = input channels, K = pixels;
- * a 64-pixel tile of dy and the 3 x 66 pixel input halo are staged in LDS
- * channel-major so that both operands read consecutive pixels; each block
- * keeps partial sums for its tiles (the bias gradient from the same staged
- * rows) and a second kernel adds the partials in a fixed order
- * (deterministic).
+ * Weight gradient: M = output channels, N = input channels, K = pixels; a
+ * wave walks down a 32-pixel column segment with its rows staged as they lie
+ * in memory and read through the transposing LDS read, so that both operands
+ * get consecutive pixels; a second kernel adds the blocks' partial sums in a
+ * fixed order (deterministic).
  */
 #include "denoise.h"
 
@@ -35,6 +34,9 @@ __device__ __forceinline__ bf16_t f2bf(float f)
 	if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)((u >> 16) | 0x40u);
 	return (bf16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
 }
+
+static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+static bool aligned16_3(const void* a, const void* b, const void* c) { return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0; }
 
 static const int DW_BLOCKS = 512;
 
@@ -152,12 +154,26 @@ __device__ __forceinline__ float4 frame_display(float o0, float o1, float o2, ui
 }
 
 typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
-enum { IO_NONE = 0, IO_DISPLAY = 1 };
+/* What the epilogue does besides the plain store: IO_DISPLAY writes the display
+ * image of a frame; IO_MASK zeroes outputs whose activation (the tensor `act`,
+ * shaped like y) is not positive, the ReLU gradient of the layer below; IO_SPLIT
+ * (64 outputs) is the gradient of the decoder's concatenation: channels 32..63
+ * to y (the skip tensor), 2 x 2 sums of channels 0..31, masked by `act` (coarse
+ * size), to ypool. */
+enum { IO_NONE = 0, IO_DISPLAY = 1, IO_MASK = 2, IO_SPLIT = 3 };
+
+/* dword of two bf16 gradients, each kept where its activation is positive */
+__device__ __forceinline__ uint32_t relu_mask2(uint32_t act, uint32_t g)
+{
+	return (bf2f((bf16_t)(act & 0xffffu)) > 0.0f ? g & 0xffffu : 0u) | (bf2f((bf16_t)(act >> 16)) > 0.0f ? g & 0xffff0000u : 0u);
+}
+
 template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL = false, int MBW = 4, int ROWS = 4, int IO = IO_NONE>
 __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restrict__ x, const bf16_t* __restrict__ coarse,
 	const bf16_t* __restrict__ w, const float* __restrict__ bias, void* __restrict__ y, int H, int W, bf16_t* __restrict__ ypool,
-	FrameIO io = FrameIO{})
+	FrameIO io = FrameIO{}, const bf16_t* __restrict__ act = nullptr)
 {
+	static_assert(IO != IO_SPLIT || (NB == 4 && !F32OUT && !RELU && !POOL), "the concatenation's gradient has 64 channels");
 	static_assert(IO != IO_DISPLAY || (NB == 1 && F32OUT && !RELU), "the display epilogue reads the first output channels");
 	constexpr int CX = CAT ? 32 : CIN;                  /* channels of x */
 	constexpr int CKX = CX < 32 ? 32 : CX;              /* channels per pixel of the x tile (K, padded) */
@@ -293,7 +309,9 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 		}
 	}
 	const int ry = r0 + wave;
-	float hs[POOL ? MBW : 1][NB][4];                     /* POOL: sums of horizontal pixel pairs */
+	constexpr bool PAIRS = POOL || IO == IO_SPLIT;       /* 2 x 2 sums of the first PNB channel blocks */
+	constexpr int PNB = IO == IO_SPLIT ? 2 : NB;
+	float hs[PAIRS ? MBW : 1][PNB][4];                   /* sums of horizontal pixel pairs */
 	/* bf16 output with channel blocks in pairs: lanes kg and kg ^ 1 swap half
 	 * their fragments so that each lane writes 8 consecutive channels (16 B)
 	 * and one store instruction covers whole 64 B pixel rows; kg even keeps
@@ -333,12 +351,12 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 				else *(uint2*)((bf16_t*)y + o) = make_uint2((uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16,
 					(uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16);
 			}
-			if (POOL)                                     /* the stored (bf16) values, left + right */
+			if (PAIRS && nb < PNB)                        /* the stored (bf16) values, left + right */
 #pragma unroll
 				for (int i = 0; i < 4; i++)
 				{
 					const float r = bf2f(f2bf(v[i]));
-					hs[POOL ? mb : 0][nb][i] = r + __shfl_xor(r, 1);
+					hs[PAIRS ? mb : 0][nb < PNB ? nb : 0][i] = r + __shfl_xor(r, 1);
 				}
 		}
 	}
@@ -350,29 +368,39 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 		{
 			const int px = x0 + mb * 16 + ml;
 #pragma unroll
-			for (int nb = 0; nb < NB; nb += 2)
+			for (int nb = IO == IO_SPLIT ? 2 : 0; nb < NB; nb += 2)
 			{
 				const uint32_t s0 = even ? pk[mb][nb + 1][0] : pk[mb][nb][0], s1 = even ? pk[mb][nb + 1][1] : pk[mb][nb][1];
 				const uint32_t r0 = (uint32_t)__shfl_xor((int)s0, 16), r1 = (uint32_t)__shfl_xor((int)s1, 16);
-				const uint4 q = even ? make_uint4(pk[mb][nb][0], pk[mb][nb][1], r0, r1) : make_uint4(r0, r1, pk[mb][nb + 1][0], pk[mb][nb + 1][1]);
+				uint4 q = even ? make_uint4(pk[mb][nb][0], pk[mb][nb][1], r0, r1) : make_uint4(r0, r1, pk[mb][nb + 1][0], pk[mb][nb + 1][1]);
 				const int ch = even ? nb * 16 + kg * 4 : (nb + 1) * 16 + (kg - 1) * 4;
-				if (ry < H && px < W) *(uint4*)((bf16_t*)y + ((size_t)ry * W + px) * Cout + ch) = q;
+				constexpr int YC = IO == IO_SPLIT ? 32 : Cout;
+				const size_t at = ((size_t)ry * W + px) * YC + ch - (Cout - YC);
+				if (ry < H && px < W)
+				{
+					if (IO == IO_MASK)
+					{
+						const uint4 a = *(const uint4*)(act + at);
+						q = make_uint4(relu_mask2(a.x, q.x), relu_mask2(a.y, q.y), relu_mask2(a.z, q.z), relu_mask2(a.w, q.w));
+					}
+					*(uint4*)((bf16_t*)y + at) = q;
+				}
 			}
 		}
 	}
-	if (POOL)
+	if (PAIRS)
 	{
-		/* 2x2 average: (top pair) + (bottom pair), as dn_pool2 on the stored tensor.
-		 * Odd rows pass their pair sums to the even rows through LDS. */
+		/* 2x2 average, (top pair) + (bottom pair), as dn_pool2 on the stored tensor (IO_SPLIT: the sum, as
+		 * dn_upcat_bwd). Odd rows pass their pair sums to the even rows through LDS. */
 		float* ex = (float*)xs;
 		__syncthreads();                                  /* every wave is done with the staged tile */
 		if (wave & 1)
 #pragma unroll
 			for (int mb = 0; mb < MBW; mb++)
 #pragma unroll
-				for (int nb = 0; nb < NB; nb++)
+				for (int nb = 0; nb < PNB; nb++)
 #pragma unroll
-					for (int i = 0; i < 4; i++) ex[(((wave >> 1) * MBW + mb) * NB * 4 + nb * 4 + i) * 64 + lane] = hs[POOL ? mb : 0][nb][i];
+					for (int i = 0; i < 4; i++) ex[(((wave >> 1) * MBW + mb) * PNB * 4 + nb * 4 + i) * 64 + lane] = hs[PAIRS ? mb : 0][nb][i];
 		__syncthreads();
 		const int Wp = W >> 1, pr = (r0 >> 1) + (wave >> 1);
 		if (!(wave & 1) && ry + 1 < H && !(ml & 1))
@@ -382,14 +410,21 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 				const int px = x0 + mb * 16 + ml;
 				if (px >= W) continue;
 #pragma unroll
-				for (int nb = 0; nb < NB; nb++)
+				for (int nb = 0; nb < PNB; nb++)
 				{
 					bf16_t q[4];
 #pragma unroll
 					for (int i = 0; i < 4; i++)
-						q[i] = f2bf((hs[POOL ? mb : 0][nb][i] + ex[(((wave >> 1) * MBW + mb) * NB * 4 + nb * 4 + i) * 64 + lane]) * 0.25f);
-					*(uint2*)(ypool + ((size_t)pr * Wp + (px >> 1)) * Cout + nb * 16 + kg * 4) =
-						make_uint2((uint32_t)q[0] | (uint32_t)q[1] << 16, (uint32_t)q[2] | (uint32_t)q[3] << 16);
+						q[i] = f2bf((hs[PAIRS ? mb : 0][nb][i] + ex[(((wave >> 1) * MBW + mb) * PNB * 4 + nb * 4 + i) * 64 + lane]) *
+							(IO == IO_SPLIT ? 1.0f : 0.25f));
+					const size_t at = ((size_t)pr * Wp + (px >> 1)) * (PNB * 16) + nb * 16 + kg * 4;
+					uint2 o = make_uint2((uint32_t)q[0] | (uint32_t)q[1] << 16, (uint32_t)q[2] | (uint32_t)q[3] << 16);
+					if (IO == IO_SPLIT)
+					{
+						const uint2 a = *(const uint2*)(act + at);
+						o = make_uint2(relu_mask2(a.x, o.x), relu_mask2(a.y, o.y));
+					}
+					*(uint2*)(ypool + at) = o;
 				}
 			}
 	}
@@ -510,205 +545,380 @@ hipError_t dn_conv3x3_display(const bf16_t* x, const bf16_t* wts, const float* b
 	return hipGetLastError();
 }
 
-/* ---- weight gradient ---------------------------------------------------
- * dW[tap][co][ci] = sum_p dy[p][co] x[p + tap - (1,1)][ci] as a GEMM over
- * pixels on v_mfma_f32_16x16x32_bf16 (M = output channels, N = input
- * channels, K = 32 pixels). Writing q = p + (dx - 1) for the input pixel, a
- * tap pairs input row ty + r - 1 at pixels q with the output-gradient row ty
- * at pixels q + 1 - dx, so a block keeps, per 64-pixel segment of a row:
- * the three input rows (a ring: one new row per step) and the gradient row
- * at its three horizontal shifts, all channel-major ([channel][pixel]) so
- * that every MFMA fragment (8 consecutive pixels of one channel) is one
- * aligned 16-byte LDS read. Staging lanes load 4 pixels x 8 channels with
- * 16-byte global loads and write them transposed as 8 rows of 4 pixels; the
- * next row's loads are in flight while the current row's products run. Nine waves, one per tap, accumulate all Cout x Cin tiles of
- * their tap in registers over a column segment of rows; per-block partial
- * sums are reduced in block order (deterministic). */
-typedef __bf16 bf8v_dw __attribute__((ext_vector_type(8)));
-
-/* Channel c of four pixels: v[p] holds channels 0..7 of pixel p (bf16
- * pairs per dword); the result holds pixels 0..3 of channel c. */
-__device__ __forceinline__ uint2 column4(const uint4 (&v)[4], int c)
+/* Input gradients with what follows them in the backward pass done by the
+ * epilogue: the ReLU gradient of the layer below (dn_conv3x3 + dn_relu_bwd), or
+ * the concatenation's (dn_conv3x3 to 64 channels + dn_upcat_bwd + dn_relu_bwd
+ * of the coarse half), bit for bit. Level 0 at 1088 x 1920: the ReLU pass alone
+ * moved 402 MB (66 us) per layer, the 64-channel tensor 268 MB out and back. */
+template <int CIN, int NB, int IO>
+static void conv_dx(const bf16_t* gy, const bf16_t* w, bf16_t* gx, bf16_t* gcoarse, const bf16_t* act, int H, int W, hipStream_t s)
 {
-	uint32_t d[4];
-#pragma unroll
-	for (int p = 0; p < 4; p++)
-		d[p] = (c >> 1) == 0 ? v[p].x : (c >> 1) == 1 ? v[p].y : (c >> 1) == 2 ? v[p].z : v[p].w;
-	if (c & 1) return make_uint2((d[0] >> 16) | (d[1] & 0xffff0000u), (d[2] >> 16) | (d[3] & 0xffff0000u));
-	return make_uint2((d[0] & 0xffffu) | (d[1] << 16), (d[2] & 0xffffu) | (d[3] << 16));
+	if (small_image(H, W))
+		k_conv3x3_t<CIN, NB, false, false, false, false, 1, 4, IO><<<dim3((W + 15) / 16, (H + 3) / 4), 256, 0, s>>>(gy, nullptr, w, nullptr, gx, H, W,
+			gcoarse, FrameIO{}, act);
+	else
+		k_conv3x3_t<CIN, NB, false, false, false, false, 4, TILE_ROWS, IO><<<dim3((W + 63) / 64, (H + TILE_ROWS - 1) / TILE_ROWS), 64 * TILE_ROWS, 0,
+			s>>>(gy, nullptr, w, nullptr, gx, H, W, gcoarse, FrameIO{}, act);
 }
 
-template <int COUT>
-__device__ __forceinline__ bool tid_in_bias(int tid) { return tid < 16 * COUT; }
-
-template <int CIN, int COUT>
-__global__ void __launch_bounds__(576) k_conv3x3_dw(const bf16_t* __restrict__ x, const bf16_t* __restrict__ dy, int H, int W,
-	int rowsPerChunk, float* __restrict__ partial, float* __restrict__ partialB)
+hipError_t dn_conv3x3_dx_relu(const bf16_t* gy, int Cin, const bf16_t* w, const bf16_t* act, bf16_t* gx, int Cout, int H, int W, hipStream_t s)
 {
-	constexpr int MB = COUT / 16, NB = CIN / 16, KP = 64 + 8;
-	constexpr int XL = 2 * CIN, DL = 6 * COUT;   /* staging lanes: 16 groups of 4 pixels x CIN / 8 channel groups; 3 shifts x 16 x COUT / 8 */
-	__shared__ __attribute__((aligned(16))) bf16_t xs[3][CIN][KP];
-	__shared__ __attribute__((aligned(16))) bf16_t ds[3][COUT][KP];
-	__shared__ float bred[16][COUT];
-	/* bias gradient: lane (channel tid % COUT, pixel group tid / COUT) adds 4 pixels of each row */
-	const bool isB = partialB != nullptr && tid_in_bias<COUT>(threadIdx.x);
-	float bsum = 0.0f;
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	const int r = wave / 3, dxo = wave % 3, sh = 2 - dxo;
-	const int tilesX = (W + 63) / 64;
-	const int x0 = (int)(blockIdx.x % tilesX) * 64, y0 = (int)(blockIdx.x / tilesX) * rowsPerChunk;
-	const int y1 = y0 + rowsPerChunk < H ? y0 + rowsPerChunk : H;
-	/* staging role: x (tid < XL) or dy (XL <= tid < XL + DL) */
-	const bool isX = tid < XL, isD = !isX && tid < XL + DL;
-	const int t = isX ? tid : tid - XL;
-	const int cg = isX ? t % (CIN / 8) : t % (COUT / 8);
-	const int q = isX ? t / (CIN / 8) : (t / (COUT / 8)) % 16;
-	const int shift = isX ? 0 : t / (2 * COUT);    /* dy copy s holds pixels x0 + j + s - 1 */
-	uint4 v[4];
-	const auto load = [&](int row) {
-		const bf16_t* base = isX ? x : dy;
-		const int C = isX ? CIN : COUT;
-		const bool rowOk = row >= 0 && row < H;
+	if (Cout != 32 || (Cin != 16 && Cin != 32) || H <= 0 || W <= 0 || !aligned16_3(gy, act, gx)) return hipErrorInvalidValue;
+	if (Cin == 16) conv_dx<16, 2, IO_MASK>(gy, w, gx, nullptr, act, H, W, s);
+	else conv_dx<32, 2, IO_MASK>(gy, w, gx, nullptr, act, H, W, s);
+	return hipGetLastError();
+}
+
+hipError_t dn_conv3x3_dx_cat(const bf16_t* gy, const bf16_t* w, const bf16_t* actCoarse, bf16_t* gcoarse, bf16_t* gskip, int H, int W, hipStream_t s)
+{
+	if (H <= 0 || W <= 0 || H % 2 || W % 2 || !aligned16_3(gy, actCoarse, gcoarse) || !aligned16(gskip)) return hipErrorInvalidValue;
+	conv_dx<32, 4, IO_SPLIT>(gy, w, gskip, gcoarse, actCoarse, H, W, s);
+	return hipGetLastError();
+}
+
+/* ---- weight gradient ---------------------------------------------------
+ * dW[tap][co][ci] = sum_p dy[p][co] x[p + tap - (1,1)][ci] as a GEMM over
+ * pixels on v_mfma_f32_16x16x32_bf16 (M = output channels, N = input channels,
+ * K = 32 pixels of a row). Writing q = p + (dx - 1) for the input pixel, a tap
+ * pairs input row ty + r - 1 at pixels q with the output-gradient row ty at
+ * pixels q + 1 - dx.
+ *
+ * A wave owns a 32-pixel column segment of a few rows and all nine taps (36
+ * accumulator tiles at 32 x 32 channels), so it needs no barrier while it walks
+ * down: it copies the next input row and gradient row ([pixel][channel], as they
+ * lie in memory) into LDS of its own, and reads fragments with the transposing
+ * LDS read (ds_read_b64_tr_b16: 16 lanes get one channel each of 4 pixels). The
+ * fragments of the last three input rows stay in registers, so every row is
+ * read from memory and from LDS once for its nine uses; the gradient row is read
+ * at its three shifts. Rows are loaded two steps ahead of their use. The block's
+ * 8 waves add their sums in wave order through LDS, and k_dw_reduce adds the
+ * blocks' in a fixed order (deterministic).
+ *
+ * All layers of a network go in one launch (their inputs and gradients are kept
+ * by the backward pass): a layer of a small image fills a fraction of the chip
+ * on its own. The 64 input channels of the decoder's concatenation run as two
+ * halves, the coarse one read from the coarse tensor (row and pixel halved).
+ * The 19 layers of the network at 1088 x 1920 (1.7 GB of inputs and gradients,
+ * 340 us at a copy's rate): 1,034 us and 413 us for partial sums with 9-wave
+ * blocks that transposed while staging and a launch per layer, 471 and 22 us
+ * now; at 256 x 256 362 us in all, now 41. */
+typedef __bf16 bf8v_dw __attribute__((ext_vector_type(8)));
+typedef short s4x __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4x lds_s4x;
+typedef short s8x __attribute__((ext_vector_type(8)));
+
+static constexpr int DWW = 8;                       /* waves per block */
+static constexpr int DW_SEG = 32;                   /* pixels of a wave's segment */
+static constexpr int DW_MAXJOBS = 32;
+static constexpr int DW_ROWSTRIDE = 40;             /* bf16 per LDS pixel: 32 channels and padding */
+static constexpr int DW_STAGE = (DW_SEG + DW_SEG + 2) * DW_ROWSTRIDE;
+
+struct DwJob
+{
+	const bf16_t* x;
+	const bf16_t* dy;
+	float* dw;
+	float* db;          /* null: no bias gradient from this job */
+	uint32_t part;      /* its partial sums in the workspace: blocks x n floats from here */
+	int H, W;
+	int16_t cx, cy;     /* channels of x and dy: 16 or 32 */
+	int16_t up;         /* 1: x is the coarse tensor [H/2][W/2][cx], upsampled */
+	int16_t ldw, off;   /* dw row length and first column of this job's channels */
+	int16_t sx;         /* channels per pixel of x in memory */
+	int rows, tilesX, chunks, block0, blocks;
+	int out0;           /* first output of the job in the reduction's grid, in groups of 32 */
+};
+struct DwBatch { DwJob j[DW_MAXJOBS]; int n; };
+static_assert(sizeof(DwBatch) <= 4000, "kernel argument size");
+
+__device__ __forceinline__ bf8v_dw tr_frag(const bf16_t* lds, int firstPixel, int ch, int lane)
+{
+	const bf16_t* p = lds + (firstPixel + 8 * (lane >> 4) + ((lane & 15) >> 2)) * DW_ROWSTRIDE + ch + (lane & 3) * 4;
+	const s4x a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4x*)p);
+	const s4x b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4x*)(p + 4 * DW_ROWSTRIDE));
+	const s8x v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+	return __builtin_bit_cast(bf8v_dw, v);
+}
+
+/* One chunk (a segment of J.rows rows) into acc[tap][mb][nb], accb[mb] (column 0.. of sum dy). */
+template <int CX, int CY>
+__device__ __forceinline__ void dw_chunk(const DwJob& J, int chunk, bf16_t* lx, f4v (&acc)[9][2][2], f4v (&accb)[2])
+{
+	constexpr int MB = CY / 16, NB = CX / 16, XG = CX / 8, DG = CY / 8;           /* 16-byte groups per pixel */
+	constexpr int XI = DW_SEG * XG / 64, DI = ((DW_SEG + 2) * DG + 63) / 64;      /* loads per lane and row */
+	bf16_t* ld = lx + DW_SEG * DW_ROWSTRIDE;
+	const int lane = threadIdx.x & 63, H = J.H, W = J.W;
+	const int x0 = (chunk % J.tilesX) * DW_SEG, y0 = (chunk / J.tilesX) * J.rows, y1 = min(y0 + J.rows, H);
+	const auto loadX = [&](uint4 (&v)[XI], int row) {
 #pragma unroll
-		for (int p = 0; p < 4; p++)
+		for (int j = 0; j < XI; j++)
 		{
-			const int px = x0 + 4 * q + p + (isX ? 0 : shift - 1);
-			v[p] = (rowOk && px >= 0 && px < W) ? *(const uint4*)(base + ((size_t)row * W + px) * C + cg * 8) : make_uint4(0, 0, 0, 0);
+			const int i = lane + 64 * j, g = i % XG, px = x0 + i / XG;
+			const size_t at = J.up ? (size_t)(row >> 1) * (W >> 1) + (px >> 1) : (size_t)row * W + px;
+			v[j] = row >= 0 && row < H && row <= y1 && px < W ? *(const uint4*)(J.x + at * J.sx + g * 8) : make_uint4(0, 0, 0, 0);
 		}
 	};
-	const auto store = [&](int slot) {
+	const auto loadD = [&](uint4 (&v)[DI], int row) {    /* pixels x0 - 1 .. x0 + 32 */
 #pragma unroll
-		for (int c = 0; c < 8; c++)
+		for (int j = 0; j < DI; j++)
 		{
-			bf16_t* dst = isX ? &xs[slot][cg * 8 + c][4 * q] : &ds[shift][cg * 8 + c][4 * q];
-			*(uint2*)dst = column4(v, c);
+			const int i = lane + 64 * j, g = i % DG, k = i / DG, px = x0 - 1 + k;
+			v[j] = k < DW_SEG + 2 && row < y1 && px >= 0 && px < W ? *(const uint4*)(J.dy + ((size_t)row * W + px) * CY + g * 8) : make_uint4(0, 0, 0, 0);
 		}
 	};
-	const auto slotOf = [](int row) { return (row % 3 + 3) % 3; };
-	f4v acc[MB][NB];
+	const auto storeX = [&](const uint4 (&v)[XI]) {
 #pragma unroll
-	for (int mb = 0; mb < MB; mb++)
+		for (int j = 0; j < XI; j++)
+		{
+			const int i = lane + 64 * j;
+			*(uint4*)(lx + (i / XG) * DW_ROWSTRIDE + (i % XG) * 8) = v[j];
+		}
+	};
+	const auto storeD = [&](const uint4 (&v)[DI]) {
 #pragma unroll
-		for (int nb = 0; nb < NB; nb++) acc[mb][nb] = (f4v){ 0.0f, 0.0f, 0.0f, 0.0f };
-	if (y0 < y1)
+		for (int j = 0; j < DI; j++)
+		{
+			const int i = lane + 64 * j;
+			if (i < (DW_SEG + 2) * DG) *(uint4*)(ld + (i / DG) * DW_ROWSTRIDE + (i % DG) * 8) = v[j];
+		}
+	};
+	bf8v_dw ring[3][NB];                                 /* input rows ty - 1, ty, ty + 1 */
+	uint4 xv[2][XI], dv[2][DI];
 	{
-		if (isX)
-		{	/* the two rows above the first step's new row */
-			load(y0 - 1), store(slotOf(y0 - 1));
-			load(y0), store(slotOf(y0));
-		}
-		if (isX) load(y0 + 1);
-		else if (isD) load(y0);
-		for (int ty = y0; ty < y1; ty++)
+		uint4 a[XI], b[XI];
+		loadX(a, y0 - 1), loadX(b, y0);
+		loadX(xv[0], y0 + 1), loadD(dv[0], y0);
+		loadX(xv[1], y0 + 2), loadD(dv[1], y0 + 1);
+		storeX(a);
+#pragma unroll
+		for (int nb = 0; nb < NB; nb++) ring[0][nb] = tr_frag(lx, 0, nb * 16, lane);
+		storeX(b);
+#pragma unroll
+		for (int nb = 0; nb < NB; nb++) ring[1][nb] = tr_frag(lx, 0, nb * 16, lane);
+	}
+	const bf8v_dw ones = { (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f, (__bf16)1.0f };
+	const auto step = [&](uint4 (&xs)[XI], uint4 (&dsv)[DI], int ty) {
+		storeX(xs), storeD(dsv);
+		loadX(xs, ty + 3), loadD(dsv, ty + 2);
+#pragma unroll
+		for (int nb = 0; nb < NB; nb++) ring[2][nb] = tr_frag(lx, 0, nb * 16, lane);
+#pragma unroll
+		for (int dx = 0; dx < 3; dx++)
 		{
-			if (isX) store(slotOf(ty + 1));
-			else if (isD) store(0);
-			__syncthreads();
-			if (ty + 1 < y1)
-			{	/* the next step's rows, in flight during this step's products */
-				if (isX) load(ty + 2);
-				else if (isD) load(ty + 1);
-			}
-			if (isB)
-			{	/* the unshifted copy holds row ty at pixels x0 .. x0 + 63 (zero beyond W) */
-				const uint2 v = *(const uint2*)&ds[1][tid % COUT][(tid / COUT) * 4];
-				bsum += bf2f((bf16_t)(v.x & 0xffffu)), bsum += bf2f((bf16_t)(v.x >> 16));
-				bsum += bf2f((bf16_t)(v.y & 0xffffu)), bsum += bf2f((bf16_t)(v.y >> 16));
-			}
-			const int xslot = slotOf(ty - 1 + r);
+			bf8v_dw A[MB];
 #pragma unroll
-			for (int kc = 0; kc < 2; kc++)
-			{
-				const int koff = kc * 32 + (lane >> 4) * 8;
-				bf8v_dw A[MB], B[NB];
+			for (int mb = 0; mb < MB; mb++) A[mb] = tr_frag(ld, 2 - dx, mb * 16, lane);
 #pragma unroll
-				for (int mb = 0; mb < MB; mb++) A[mb] = *(const bf8v_dw*)&ds[sh][mb * 16 + (lane & 15)][koff];
-#pragma unroll
-				for (int nb = 0; nb < NB; nb++) B[nb] = *(const bf8v_dw*)&xs[xslot][nb * 16 + (lane & 15)][koff];
+			for (int r = 0; r < 3; r++)
 #pragma unroll
 				for (int mb = 0; mb < MB; mb++)
 #pragma unroll
-					for (int nb = 0; nb < NB; nb++) acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mb], B[nb], acc[mb][nb], 0, 0, 0);
-			}
-			__syncthreads();
+					for (int nb = 0; nb < NB; nb++)
+						acc[3 * r + dx][mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mb], ring[r][nb], acc[3 * r + dx][mb][nb], 0, 0, 0);
+			if (dx == 1)
+#pragma unroll
+				for (int mb = 0; mb < MB; mb++) accb[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mb], ones, accb[mb], 0, 0, 0);
 		}
+#pragma unroll
+		for (int nb = 0; nb < NB; nb++) ring[0][nb] = ring[1][nb], ring[1][nb] = ring[2][nb];
+	};
+	for (int ty = y0; ty < y1; ty += 2)
+	{
+		step(xv[0], dv[0], ty);
+		if (ty + 1 < y1) step(xv[1], dv[1], ty + 1);
 	}
-	if (partialB)
-	{	/* this block's bias partial: the 16 pixel groups of each channel added in group order */
-		if (isB) bred[tid / COUT][tid % COUT] = bsum;
-		__syncthreads();
-		if (tid < COUT)
-		{
-			float t = 0.0f;
-			for (int g = 0; g < 16; g++) t += bred[g][tid];
-			partialB[(size_t)blockIdx.x * COUT + tid] = t;
-		}
-	}
-	/* D layout: lane holds rows 4 (lane / 16) + i, column lane % 16 */
-	float* out = partial + (size_t)blockIdx.x * 9 * COUT * CIN;
-	const int tap = wave;
-#pragma unroll
-	for (int mb = 0; mb < MB; mb++)
-#pragma unroll
-		for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-			for (int i = 0; i < 4; i++)
-				out[((size_t)tap * COUT + mb * 16 + (lane >> 4) * 4 + i) * CIN + nb * 16 + (lane & 15)] = acc[mb][nb][i];
 }
 
-/* out[i] = sum over b < blocks of partial[b][i] in a fixed order: 8 lanes
- * per output each add every 8th block partial (32 consecutive outputs per
- * block row, coalesced), then the 8 sums are added in lane order. */
-__global__ void __launch_bounds__(256) k_reduce_partials(const float* __restrict__ partial, int blocks, int n, float* __restrict__ out)
+/* Sums of the block's waves, in wave order, to partial[9][CY][CX] and bias[CY]:
+ * in four rounds, each wave laying a quarter of its tiles into LDS. */
+template <int CX, int CY>
+__device__ __forceinline__ void dw_store(float* lds, const f4v (&acc)[9][2][2], const f4v (&accb)[2], float* out)
+{
+	constexpr int MB = CY / 16, NB = CX / 16;
+	constexpr int TILES = 9 * MB * NB;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	f4v t[TILES];
+#pragma unroll
+	for (int tap = 0; tap < 9; tap++)
+#pragma unroll
+		for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+			for (int nb = 0; nb < NB; nb++) t[(tap * MB + mb) * NB + nb] = acc[tap][mb][nb];
+	constexpr int PER = (TILES + 3) / 4;
+#pragma unroll
+	for (int round = 0; round < 4; round++)
+	{
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < PER; k++)
+			if (round * PER + k < TILES) *(f4v*)(lds + ((wave * PER + k) * 64 + lane) * 4) = t[round * PER + k < TILES ? round * PER + k : 0];
+		__syncthreads();
+		for (int e = threadIdx.x; e < PER * 64; e += 64 * DWW)
+		{
+			const int tile = round * PER + e / 64, l = e % 64;
+			if (tile >= TILES) continue;
+			f4v sum = *(const f4v*)(lds + e * 4);
+#pragma unroll
+			for (int w = 1; w < DWW; w++) sum += *(const f4v*)(lds + (w * PER * 64 + e) * 4);
+			const int tap = tile / (MB * NB), mb = (tile / NB) % MB, nb = tile % NB;
+			/* D layout: lane holds rows 4 (lane / 16) + i, column lane % 16 */
+#pragma unroll
+			for (int i = 0; i < 4; i++) out[(tap * CY + mb * 16 + (l >> 4) * 4 + i) * CX + nb * 16 + (l & 15)] = sum[i];
+		}
+	}
+	__syncthreads();
+	if ((lane & 15) == 0)
+#pragma unroll
+		for (int mb = 0; mb < MB; mb++) *(f4v*)(lds + (wave * 2 + mb) * 16 + (lane >> 4) * 4) = accb[mb];
+	__syncthreads();
+	if ((int)threadIdx.x < CY)
+	{
+		float sum = 0.0f;
+		for (int w = 0; w < DWW; w++) sum += lds[(w * 2 + (int)threadIdx.x / 16) * 16 + (int)threadIdx.x % 16];
+		out[9 * CY * CX + threadIdx.x] = sum;
+	}
+}
+
+template <int CX, int CY>
+__device__ __forceinline__ void dw_job(const DwJob& J, float* lds, float* ws)
+{
+	const int wave = threadIdx.x >> 6, b = (int)blockIdx.x - J.block0, chunk = b * DWW + wave;
+	f4v acc[9][2][2], accb[2];
+#pragma unroll
+	for (int k = 0; k < 9; k++)
+#pragma unroll
+		for (int m = 0; m < 4; m++) acc[k][m >> 1][m & 1] = (f4v){ 0.0f, 0.0f, 0.0f, 0.0f };
+	accb[0] = accb[1] = (f4v){ 0.0f, 0.0f, 0.0f, 0.0f };
+	if (chunk < J.chunks) dw_chunk<CX, CY>(J, chunk, (bf16_t*)lds + wave * DW_STAGE, acc, accb);
+	dw_store<CX, CY>(lds, acc, accb, ws + J.part + (size_t)b * (9 * CX * CY + CY));
+}
+
+__global__ void __launch_bounds__(64 * DWW, 2) k_conv3x3_dw(const DwBatch B, float* __restrict__ ws)
+{
+	constexpr int SUMS = DWW * 9 * 64 * 4 * 4, STAGE = DWW * DW_STAGE * 2;
+	__shared__ __attribute__((aligned(16))) char lds[SUMS > STAGE ? SUMS : STAGE];
+	int k = 0;
+	while (k + 1 < B.n && B.j[k + 1].block0 <= (int)blockIdx.x) k++;
+	const DwJob& J = B.j[k];
+	if (J.cx == 32 && J.cy == 32) dw_job<32, 32>(J, (float*)lds, ws);
+	else if (J.cx == 16 && J.cy == 32) dw_job<16, 32>(J, (float*)lds, ws);
+	else if (J.cx == 32) dw_job<32, 16>(J, (float*)lds, ws);
+	else dw_job<16, 16>(J, (float*)lds, ws);
+}
+
+/* Sums of every job's blocks in a fixed order: 8 lanes per output each add
+ * every 8th block partial (32 consecutive outputs per block row, coalesced),
+ * then the 8 sums are added in lane order. */
+__global__ void __launch_bounds__(256) k_dw_reduce(const DwBatch B, const float* __restrict__ ws)
 {
 	__shared__ float red[8][33];
-	const int lane = threadIdx.x & 31, part = threadIdx.x >> 5;
-	const int i = blockIdx.x * 32 + lane;
+	int k = 0;
+	while (k + 1 < B.n && B.j[k + 1].out0 <= (int)blockIdx.x) k++;
+	const DwJob& J = B.j[k];
+	const int lane = threadIdx.x & 31, part = threadIdx.x >> 5, nw = 9 * J.cx * J.cy, n = nw + J.cy;
+	const int i = ((int)blockIdx.x - J.out0) * 32 + lane;
 	float s = 0.0f;
 	if (i < n)
-		for (int b = part; b < blocks; b += 8) s += partial[(size_t)b * n + i];
+		for (int b = part; b < J.blocks; b += 8) s += ws[J.part + (size_t)b * n + i];
 	red[part][lane] = s;
 	__syncthreads();
-	if (part == 0 && i < n)
-	{
-		float t = 0.0f;
+	if (part != 0 || i >= n) return;
+	float t = 0.0f;
 #pragma unroll
-		for (int k = 0; k < 8; k++) t += red[k][lane];
-		out[i] = t;
+	for (int q = 0; q < 8; q++) t += red[q][lane];
+	if (i < nw) J.dw[(size_t)(i / J.cx) * J.ldw + J.off + i % J.cx] = t;
+	else if (J.db) J.db[i - nw] = t;
+}
+
+/* Jobs of a list of layers: chunk heights (the same for all layers: enough
+ * chunks for 8,192 waves, each at least 8 rows: fewer waves leave compute units
+ * idle at the end, shorter chunks re-read two rows of their neighbours' input),
+ * block and workspace ranges; taller chunks where the partial sums would exceed
+ * maxFloats. false: a shape that is not supported. */
+static bool dw_plan(const DwLayer* L, int layers, size_t maxFloats, DwBatch& B, size_t& floats, int& blocks, int& outs)
+{
+	B.n = 0;
+	int64_t steps = 0;
+	int tallest = 1;
+	if (!L || layers <= 0) return false;
+	for (int i = 0; i < layers; i++)
+	{
+		const DwLayer& l = L[i];
+		const bool ok = (l.Cout == 32 && (l.Cin == 16 || l.Cin == 32 || l.Cin == 64)) || (l.Cout == 16 && (l.Cin == 16 || l.Cin == 32));
+		if (!ok || !l.x || !l.dy || !l.dw || l.H <= 0 || l.W <= 0 || (l.W + 63) / 64 > DW_BLOCKS) return false;   /* W beyond DW_BLOCKS * 64 pixels */
+		if (l.coarse && (l.Cin != 64 || l.H % 2 || l.W % 2)) return false;
+		const int parts = l.Cin == 64 ? 2 : 1;
+		if (B.n + parts > DW_MAXJOBS) return false;
+		for (int p = 0; p < parts; p++)
+		{
+			DwJob& J = B.j[B.n++];
+			J = DwJob{};
+			J.dy = l.dy, J.dw = l.dw, J.db = p == 0 ? l.db : nullptr;
+			J.H = l.H, J.W = l.W, J.cy = (int16_t)l.Cout, J.ldw = (int16_t)l.Cin, J.off = (int16_t)(32 * p);
+			J.cx = (int16_t)(l.Cin == 64 ? 32 : l.Cin);
+			J.sx = (int16_t)(l.Cin == 64 && !l.coarse ? 64 : J.cx);
+			J.up = (int16_t)(l.coarse && p == 0 ? 1 : 0);
+			J.x = l.coarse ? (p == 0 ? l.coarse : l.x) : l.x + 32 * p;
+			J.tilesX = (l.W + DW_SEG - 1) / DW_SEG;
+			steps += (int64_t)J.tilesX * l.H;
+			tallest = tallest > l.H ? tallest : l.H;
+		}
 	}
+	int rows = (int)(steps / 8192 < 8 ? 8 : steps / 8192 < tallest ? steps / 8192 : tallest);
+	while (true)
+	{
+		blocks = outs = 0, floats = 0;
+		for (int k = 0; k < B.n; k++)
+		{
+			DwJob& J = B.j[k];
+			const int n = 9 * J.cx * J.cy + J.cy;
+			J.rows = rows < J.H ? rows : J.H;
+			J.chunks = J.tilesX * ((J.H + J.rows - 1) / J.rows), J.blocks = (J.chunks + DWW - 1) / DWW;
+			J.block0 = blocks, J.out0 = outs, J.part = (uint32_t)floats;
+			blocks += J.blocks, outs += (n + 31) / 32, floats += (size_t)J.blocks * n;
+		}
+		if (floats <= maxFloats) return true;
+		if (rows >= tallest) return false;
+		rows += (rows + 7) / 8;
+	}
+}
+
+static hipError_t dw_launch(const DwBatch& B, int blocks, int outs, void* ws, hipStream_t s)
+{
+	k_conv3x3_dw<<<blocks, 64 * DWW, 0, s>>>(B, (float*)ws);
+	k_dw_reduce<<<outs, 256, 0, s>>>(B, (const float*)ws);
+	return hipGetLastError();
 }
 
 size_t dn_dw_workspace_bytes(int Cin, int Cout) { return (size_t)DW_BLOCKS * (9 * Cout * Cin + Cout) * sizeof(float); }
 
-template <int CIN, int COUT>
-static void launch_dw(const bf16_t* x, const bf16_t* dy, int H, int W, int rowsPerChunk, float* partial, float* partialB, int blocks, hipStream_t s)
-{
-	k_conv3x3_dw<CIN, COUT><<<blocks, 576, 0, s>>>(x, dy, H, W, rowsPerChunk, partial, partialB);
-}
-
 hipError_t dn_conv3x3_dw(const bf16_t* x, int Cin, const bf16_t* dy, int Cout, int H, int W, float* dw, float* db, void* ws, hipStream_t s)
 {
-	if (H <= 0 || W <= 0 || !ws) return hipErrorInvalidValue;
-	/* blocks = 64-pixel column segments x row chunks (at least 8 rows each), at most DW_BLOCKS */
-	const int tilesX = (W + 63) / 64;
-	int chunks = DW_BLOCKS / tilesX;
-	if (chunks < 1) chunks = 1;
-	if (chunks > (H + 7) / 8) chunks = (H + 7) / 8;
-	const int rowsPerChunk = (H + chunks - 1) / chunks;
-	const int blocks = tilesX * ((H + rowsPerChunk - 1) / rowsPerChunk);
-	if (blocks > DW_BLOCKS) return hipErrorInvalidValue;   /* W beyond DW_BLOCKS * 64 pixels */
-	float* partial = (float*)ws;
-	const int n = 9 * Cout * Cin;
-	float* bp = db ? partial + (size_t)DW_BLOCKS * n : nullptr;   /* bias partials of the same blocks */
-	if (Cin == 16 && Cout == 32) launch_dw<16, 32>(x, dy, H, W, rowsPerChunk, partial, bp, blocks, s);
-	else if (Cin == 32 && Cout == 32) launch_dw<32, 32>(x, dy, H, W, rowsPerChunk, partial, bp, blocks, s);
-	else if (Cin == 64 && Cout == 32) launch_dw<64, 32>(x, dy, H, W, rowsPerChunk, partial, bp, blocks, s);
-	else if (Cin == 32 && Cout == 16) launch_dw<32, 16>(x, dy, H, W, rowsPerChunk, partial, bp, blocks, s);
-	else if (Cin == 16 && Cout == 16) launch_dw<16, 16>(x, dy, H, W, rowsPerChunk, partial, bp, blocks, s);
-	else return hipErrorInvalidValue;
-	k_reduce_partials<<<(n + 31) / 32, 256, 0, s>>>(partial, blocks, n, dw);
-	if (db) k_reduce_partials<<<(Cout + 31) / 32, 256, 0, s>>>(bp, blocks, Cout, db);
-	return hipGetLastError();
+	DwLayer l = { x, nullptr, dy, dw, db, Cin, Cout, H, W };
+	DwBatch B;
+	size_t floats;
+	int blocks, outs;
+	if (!ws || !dw_plan(&l, 1, dn_dw_workspace_bytes(Cin, Cout) / sizeof(float), B, floats, blocks, outs)) return hipErrorInvalidValue;
+	return dw_launch(B, blocks, outs, ws, s);
+}
+
+static const size_t DW_BATCH_FLOATS = (size_t)1 << 30;
+
+size_t dn_dw_batch_workspace_bytes(const DwLayer* layers, int n)
+{
+	DwBatch B;
+	size_t floats;
+	int blocks, outs;
+	return dw_plan(layers, n, DW_BATCH_FLOATS, B, floats, blocks, outs) ? floats * sizeof(float) : 0;
+}
+
+hipError_t dn_conv3x3_dw_batch(const DwLayer* layers, int n, void* ws, size_t wsBytes, hipStream_t s)
+{
+	DwBatch B;
+	size_t floats;
+	int blocks, outs;
+	if (!ws || !dw_plan(layers, n, DW_BATCH_FLOATS, B, floats, blocks, outs) || floats * sizeof(float) > wsBytes) return hipErrorInvalidValue;
+	return dw_launch(B, blocks, outs, ws, s);
 }
 
 /* ---- weight gradient without allocation --------------------------------
@@ -793,6 +1003,27 @@ __global__ void k_pool2_bwd8(const bf16_t* __restrict__ dy, int gs, int W, bf16_
 	st8(o, r);
 }
 
+/* the gradient of an encoder level's second activation: the skip connection's gradient plus a
+ * quarter of the pooled tensor's (k_pool2_bwd8, accumulating), then the ReLU gradient, in one pass */
+__global__ void k_pool2_bwd_relu8(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ skip, const bf16_t* __restrict__ act, int gs, int W,
+	bf16_t* __restrict__ out)
+{
+	const int j = blockIdx.x * blockDim.x + threadIdx.x, G = 1 << gs, py = blockIdx.y;
+	if (j >= W * G) return;
+	const int px = j >> gs, c8 = j & (G - 1);
+	const size_t at = ((size_t)py * W + px) * (8 * G) + 8 * c8;
+	const u16x8 d = ld8(dy + ((size_t)(py >> 1) * (W >> 1) + (px >> 1)) * (8 * G) + 8 * c8), prev = ld8(skip + at), a = ld8(act + at);
+	u16x8 r;
+#pragma unroll
+	for (int k = 0; k < 8; k++)
+	{
+		float v = bf2f(d[k]) * 0.25f;
+		v += bf2f(prev[k]);
+		r[k] = bf2f(a[k]) > 0.0f ? f2bf(v) : (unsigned short)0;
+	}
+	st8(out + at, r);
+}
+
 __global__ void k_pool2_8(const bf16_t* __restrict__ x, int gs, int W, bf16_t* __restrict__ y)
 {
 	const int w2 = W >> 1, j = blockIdx.x * blockDim.x + threadIdx.x, G = 1 << gs, py = blockIdx.y;
@@ -838,7 +1069,6 @@ __global__ void k_upcat_bwd_skip8(const bf16_t* __restrict__ dcat, int G0, int G
 	st8(dskip + ((size_t)py * W + px) * (8 * G1) + 8 * g, ld8(dcat + ((size_t)py * W + px) * (8 * G) + 8 * (G0 + g)));
 }
 
-static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 static int log2_exact(int v) { int k = 0; while ((1 << k) < v) k++; return (1 << k) == v ? k : -1; }
 static dim3 row_grid(int perRow, int rows) { return dim3((unsigned)((perRow + 255) / 256), (unsigned)rows); }
 
@@ -848,7 +1078,6 @@ __global__ void k_relu_bwd(const bf16_t* __restrict__ y, const bf16_t* __restric
 		out[i] = bf2f(y[i]) > 0.0f ? dy[i] : (bf16_t)0;
 }
 
-static bool aligned16_3(const void* a, const void* b, const void* c) { return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0; }
 
 hipError_t dn_relu_bwd(const bf16_t* y, const bf16_t* dy, bf16_t* dyPre, size_t n, hipStream_t s)
 {
@@ -950,6 +1179,15 @@ hipError_t dn_pool2_bwd(const bf16_t* dy, int C, int H, int W, bf16_t* dx, int a
 	if (gs >= 0 && aligned16(dy) && aligned16(dx) && H <= 65535)
 		k_pool2_bwd8<<<row_grid(W << gs, H), 256, 0, s>>>(dy, gs, W, dx, accumulate);
 	else k_pool2_bwd<<<grid_for((size_t)H * W * C), 256, 0, s>>>(dy, C, H, W, dx, accumulate);
+	return hipGetLastError();
+}
+
+hipError_t dn_pool2_bwd_relu(const bf16_t* dy, const bf16_t* skip, const bf16_t* act, int C, int H, int W, bf16_t* out, hipStream_t s)
+{
+	if (H % 2 || W % 2 || H <= 0 || W <= 0 || H > 65535) return hipErrorInvalidValue;
+	const int gs = C <= 0 || C % 8 ? -1 : log2_exact(C / 8);
+	if (gs < 0 || !aligned16_3(dy, skip, act) || !aligned16(out)) return hipErrorInvalidValue;
+	k_pool2_bwd_relu8<<<row_grid(W << gs, H), 256, 0, s>>>(dy, skip, act, gs, W, out);
 	return hipGetLastError();
 }
 
@@ -1090,35 +1328,86 @@ __global__ void k_relmse(const float* __restrict__ out, int Cout, const float4* 
 	if (threadIdx.x == 0) atomicAdd(loss, red[0] * invN);
 }
 
+/* The network's 16 output channels: one 16-byte read and two 16-byte writes per
+ * pixel in place of 3 + 16 element accesses at a 64-byte stride; the same
+ * per-pixel arithmetic and order of sums. 1088 x 1920: 89 -> 42 us. */
+__global__ void __launch_bounds__(256) k_relmse16(const float4* __restrict__ out, const float4* __restrict__ target, size_t pixels, float invN,
+	uint4* __restrict__ dout, float* __restrict__ loss)
+{
+	__shared__ float red[256];
+	float l = 0.0f;
+	for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < pixels; p += (size_t)gridDim.x * blockDim.x)
+	{
+		const float4 t4 = target[p], o4 = out[4 * p];
+		const float t[3] = { t4.x, t4.y, t4.z }, o[3] = { o4.x, o4.y, o4.z };
+		uint32_t g[3];
+#pragma unroll
+		for (int c = 0; c < 3; c++)
+		{
+			const float d = o[c] - t[c], den = t[c] * t[c] + 0.01f;
+			l += d * d / den;
+			g[c] = f2bf(2.0f * d / den * invN);
+		}
+		dout[2 * p] = make_uint4(g[0] | g[1] << 16, g[2], 0, 0);
+		dout[2 * p + 1] = make_uint4(0, 0, 0, 0);
+	}
+	red[threadIdx.x] = l;
+	__syncthreads();
+	for (int k = 128; k > 0; k >>= 1)
+	{
+		if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+		__syncthreads();
+	}
+	if (threadIdx.x == 0) atomicAdd(loss, red[0] * invN);
+}
+
 hipError_t dn_relmse(const float* out, int Cout, const float4* target, int H, int W, bf16_t* dout, float* loss, hipStream_t s)
 {
 	const size_t pixels = (size_t)H * W;
 	const int blocks = grid_for(pixels) < 1024 ? grid_for(pixels) : 1024;
-	k_relmse<<<blocks, 256, 0, s>>>(out, Cout, target, pixels, 1.0f / (3.0f * (float)pixels), dout, loss);
+	const float invN = 1.0f / (3.0f * (float)pixels);
+	if (Cout == 16 && aligned16_3(out, target, dout)) k_relmse16<<<blocks, 256, 0, s>>>((const float4*)out, target, pixels, invN, (uint4*)dout, loss);
+	else k_relmse<<<blocks, 256, 0, s>>>(out, Cout, target, pixels, invN, dout, loss);
 	return hipGetLastError();
 }
 
-__global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v, const float* __restrict__ g, size_t n,
-	float lr, float b1, float b2, float eps, float c1, float c2, bf16_t* __restrict__ wfwd, bf16_t* __restrict__ wbwd, int Cout, int Cin)
+__device__ __forceinline__ void adam_element(const AdamTensor& T, size_t i, float lr, float b1, float b2, float eps, float c1, float c2)
 {
-	for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
+	float w = T.p[i];
+	if (T.g)
 	{
-		float w = p[i];
-		if (g)
-		{
-			const float gi = g[i];
-			const float mi = b1 * m[i] + (1.0f - b1) * gi, vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-			m[i] = mi, v[i] = vi;
-			w -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-			p[i] = w;
-		}
-		if (wfwd) wfwd[i] = f2bf(w);
-		if (wbwd)
-		{
-			const int ci = (int)(i % Cin), co = (int)((i / Cin) % Cout), tap = (int)(i / ((size_t)Cin * Cout));
-			wbwd[((size_t)(8 - tap) * Cin + ci) * Cout + co] = f2bf(w);
-		}
+		const float gi = T.g[i];
+		const float mi = b1 * T.m[i] + (1.0f - b1) * gi, vi = b2 * T.v[i] + (1.0f - b2) * gi * gi;
+		T.m[i] = mi, T.v[i] = vi;
+		w -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+		T.p[i] = w;
 	}
+	if (T.wfwd) T.wfwd[i] = f2bf(w);
+	if (T.wbwd)
+	{
+		const int ci = (int)(i % T.Cin), co = (int)((i / T.Cin) % T.Cout), tap = (int)(i / ((size_t)T.Cin * T.Cout));
+		T.wbwd[((size_t)(8 - tap) * T.Cin + ci) * T.Cout + co] = f2bf(w);
+	}
+}
+
+__global__ void k_adam(const AdamTensor T, float lr, float b1, float b2, float eps, float c1, float c2)
+{
+	for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < T.n; i += (size_t)gridDim.x * blockDim.x) adam_element(T, i, lr, b1, b2, eps, c1, c2);
+}
+
+/* All tensors of a network in one launch, a block of 256 elements each within
+ * one tensor: 38 launches of 2.4-3.4 us became one of 7. */
+static constexpr int ADAM_MAX = 48;
+struct AdamBatch { AdamTensor t[ADAM_MAX]; uint32_t block0[ADAM_MAX]; int n; };
+static_assert(sizeof(AdamBatch) <= 4000, "kernel argument size");
+
+__global__ void __launch_bounds__(256) k_adam_batch(const AdamBatch B, float lr, float b1, float b2, float eps, float c1, float c2)
+{
+	int k = 0;
+	while (k + 1 < B.n && B.block0[k + 1] <= blockIdx.x) k++;
+	const AdamTensor& T = B.t[k];
+	const size_t i = (size_t)(blockIdx.x - B.block0[k]) * 256 + threadIdx.x;
+	if (i < T.n) adam_element(T, i, lr, b1, b2, eps, c1, c2);
 }
 
 hipError_t dn_adam(float* p, float* m, float* v, const float* g, size_t n, float lr, float b1, float b2, float eps, int t,
@@ -1126,7 +1415,26 @@ hipError_t dn_adam(float* p, float* m, float* v, const float* g, size_t n, float
 {
 	if (wbwd && (Cout <= 0 || Cin <= 0 || n != (size_t)9 * Cout * Cin)) return hipErrorInvalidValue;
 	const float c1 = 1.0f - powf(b1, (float)t), c2 = 1.0f - powf(b2, (float)t);
-	k_adam<<<grid_for(n), 256, 0, s>>>(p, m, v, g, n, lr, b1, b2, eps, c1, c2, wfwd, wbwd, Cout, Cin);
+	const AdamTensor T = { p, m, v, g, wfwd, wbwd, n, Cout, Cin };
+	k_adam<<<grid_for(n), 256, 0, s>>>(T, lr, b1, b2, eps, c1, c2);
+	return hipGetLastError();
+}
+
+hipError_t dn_adam_batch(const AdamTensor* t, int n, float lr, float b1, float b2, float eps, int step, hipStream_t s)
+{
+	if (!t || n < 0) return hipErrorInvalidValue;
+	for (int i = 0; i < n; i++)
+		if (!t[i].p || !t[i].m || !t[i].v || t[i].n > ((size_t)1 << 31) ||
+			(t[i].wbwd && (t[i].Cout <= 0 || t[i].Cin <= 0 || t[i].n != (size_t)9 * t[i].Cout * t[i].Cin))) return hipErrorInvalidValue;
+	const float c1 = 1.0f - powf(b1, (float)step), c2 = 1.0f - powf(b2, (float)step);
+	for (int i = 0; i < n;)
+	{
+		AdamBatch B;
+		uint32_t blocks = 0;
+		for (B.n = 0; i < n && B.n < ADAM_MAX && blocks < (1u << 30); i++)
+			if (t[i].n) B.t[B.n] = t[i], B.block0[B.n++] = blocks, blocks += (uint32_t)((t[i].n + 255) / 256);
+		if (blocks) k_adam_batch<<<blocks, 256, 0, s>>>(B, lr, b1, b2, eps, c1, c2);
+	}
 	return hipGetLastError();
 }
 

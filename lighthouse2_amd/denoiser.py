@@ -7,8 +7,7 @@ Network (channels): input 16 = [radiance 3, albedo 3, normal 3, depth 1, 0 x 6]
   encoder level l = 0..3: a = relu(conv(in)), b = relu(conv(a)), in_{l+1} = avgpool2(b)
   bottleneck (level 4):   a = relu(conv(in)), b = relu(conv(a))
   decoder level l = 3..0: cat = [upsample2(prev), b_l], c = relu(conv(cat)), d = relu(conv(c))
-                          (the forward reads cat from its two halves; the backward
-                          pass materialises it for the weight gradient)
+                          (read from its two halves, forward and backward: never materialised)
   output: conv(d_0) -> 16 channels fp32, the first 3 are the denoised radiance.
 Loss: relMSE over the 3 output channels. Optimiser: Adam on fp32 master weights.
 Torch tensors serve as device buffers only; every operation is a kernel of
@@ -24,6 +23,17 @@ LEVELS = 5
 CH = 32
 CIN = 16
 COUT = 16
+
+
+class _Layer(ctypes.Structure):
+    """lh2hip_dn_layer: one convolution's weight gradient."""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "coarse", "dy", "dw", "db")] + [(n, ctypes.c_int) for n in ("Cin", "Cout", "H", "W")]
+
+
+class _Tensor(ctypes.Structure):
+    """lh2hip_dn_tensor: one parameter tensor of an Adam step."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("p", "m", "v", "g", "wfwd", "wbwd")] + [("n", ctypes.c_uint64)]
+                + [(n, ctypes.c_int) for n in ("Cout", "Cin")])
 
 
 def layer_specs():
@@ -77,51 +87,75 @@ class UNetDenoiser:
             d["wf"] = torch.zeros(9 * co * ci, **bf)
             d["wb"] = torch.zeros(9 * co * ci, **bf)
             self.p[name] = d
+        self._tensors = self._tensor_table(grads=True)
         self._cast()
-        self.ws = torch.zeros(int(library().lh2hip_dn_dw_workspace_bytes(2 * CH, CH)) // 4 + 64, **f32)
-        # activations per level (kept for the backward pass) and their gradients
+        # activations per level (kept for the backward pass) and the gradients of
+        # what each layer adds up before its ReLU (kept for the weight gradients)
         self.a, self.g = {}, {}
         for lvl in range(LEVELS):
             h, w = H >> lvl, W >> lvl
             self.a[f"in_{lvl}"] = torch.zeros(h * w * (CIN if lvl == 0 else CH), **bf)
-            for k in ("a", "b"):
+            if lvl > 0:
+                self.g[f"in_{lvl}"] = torch.zeros(h * w * CH, **bf)
+            for k in ("a", "b") + (("c", "d") if lvl < LEVELS - 1 else ()):
                 self.a[f"{k}_{lvl}"] = torch.zeros(h * w * CH, **bf)
                 self.g[f"{k}_{lvl}"] = torch.zeros(h * w * CH, **bf)
-            self.g[f"in_{lvl}"] = torch.zeros(h * w * CH, **bf)
             if lvl < LEVELS - 1:
-                for k in ("c", "d"):
-                    self.a[f"{k}_{lvl}"] = torch.zeros(h * w * CH, **bf)
-                    self.g[f"{k}_{lvl}"] = torch.zeros(h * w * CH, **bf)
-                self.a[f"cat_{lvl}"] = torch.zeros(h * w * 2 * CH, **bf)
-                self.g[f"cat_{lvl}"] = torch.zeros(h * w * 2 * CH, **bf)
+                self.g[f"skip_{lvl}"] = torch.zeros(h * w * CH, **bf)
         self.out = torch.zeros(H * W * COUT, **f32)
         self.dout = torch.zeros(H * W * COUT, **bf)
-        self.tmp = torch.zeros(H * W * 2 * CH, **bf)
         self.loss = torch.zeros(1, **f32)
+        self._layers = self._layer_table()
+        need = int(library().lh2hip_dn_dw_batch_workspace_bytes(self._layers, len(self._layers)))
+        self.ws = torch.zeros(need // 4, **f32)    # empty (and the backward pass refused) beyond the weight gradient's sizes
 
     # ---- helpers --------------------------------------------------------
-    def _cast(self):
-        L = library()
+    def _tensor_table(self, grads):
+        """Every weight and bias for one Adam launch; without gradients: the weights' bf16 copies only."""
+        rows = []
         for d in self.p.values():
-            _check(L.lh2hip_dn_adam(d["w"].data_ptr(), d["mw"].data_ptr(), d["vw"].data_ptr(), None, d["w"].numel(),
-                                    0.0, 0.9, 0.999, 1e-8, 1, d["wf"].data_ptr(), d["wb"].data_ptr(), d["co"], d["ci"], self.sh))
+            for k in ("w", "b") if grads else ("w",):
+                rows.append(_Tensor(d[k].data_ptr(), d["m" + k].data_ptr(), d["v" + k].data_ptr(), d["g" + k].data_ptr() if grads else None,
+                                    d["wf"].data_ptr() if k == "w" else None, d["wb"].data_ptr() if k == "w" else None, d[k].numel(),
+                                    d["co"], d["ci"]))
+        return (_Tensor * len(rows))(*rows)
+
+    def _layer_table(self):
+        """Inputs and output gradients of the 19 convolutions, for one weight-gradient launch."""
+        rows = []
+        for name, ci, co in layer_specs():
+            lvl = 0 if name == "out" else int(name[-1])
+            coarse = None
+            if name == "out":
+                x, gy = self.a["d_0"], self.dout
+            else:
+                x = self.a[{"e1": "in", "e2": "a", "d1": "b", "d2": "c"}[name[:2]] + f"_{lvl}"]
+                gy = self.g[{"e1": "a", "e2": "b", "d1": "c", "d2": "d"}[name[:2]] + f"_{lvl}"]
+                if name[:2] == "d1":
+                    coarse = self._below(lvl).data_ptr()
+            d = self.p[name]
+            rows.append(_Layer(x.data_ptr(), coarse, gy.data_ptr(), d["gw"].data_ptr(), d["gb"].data_ptr(), ci, co, self.H >> lvl, self.W >> lvl))
+        return (_Layer * len(rows))(*rows)
+
+    def _below(self, lvl, grad=False):
+        """The tensor a decoder level upsamples (or its gradient)."""
+        t = self.g if grad else self.a
+        return t[f"d_{lvl + 1}"] if lvl + 1 < LEVELS - 1 else t[f"b_{LEVELS - 1}"]
+
+    def _cast(self):
+        t = self._tensor_table(grads=False)
+        _check(library().lh2hip_dn_adam_batch(t, len(t), 0.0, 0.9, 0.999, 1e-8, 1, self.sh))
 
     def _conv(self, x, name, y, h, w, flags):
         d = self.p[name]
         _check(library().lh2hip_dn_conv3x3(x.data_ptr(), d["ci"], d["wf"].data_ptr(), d["b"].data_ptr(), y.data_ptr(), d["co"],
                                            h, w, flags, self.sh))
 
-    def _conv_dx(self, gy, name, gx, h, w):
+    def _dx_relu(self, gy, name, act, gx, h, w):
+        """Gradient of a layer's input, through the ReLU that made the input."""
         d = self.p[name]
-        _check(library().lh2hip_dn_conv3x3(gy.data_ptr(), d["co"], d["wb"].data_ptr(), None, gx.data_ptr(), d["ci"], h, w, 0, self.sh))
-
-    def _conv_dw(self, x, name, gy, h, w):
-        d = self.p[name]
-        _check(library().lh2hip_dn_conv3x3_dw(x.data_ptr(), d["ci"], gy.data_ptr(), d["co"], h, w, d["gw"].data_ptr(),
-                                              d["gb"].data_ptr(), self.ws.data_ptr(), self.sh))
-
-    def _relu_bwd(self, y, gy, out):
-        _check(library().lh2hip_dn_relu_bwd(y.data_ptr(), gy.data_ptr(), out.data_ptr(), y.numel(), self.sh))
+        _check(library().lh2hip_dn_conv3x3_dx_relu(gy.data_ptr(), d["co"], d["wb"].data_ptr(), act.data_ptr(), gx.data_ptr(), d["ci"],
+                                                   h, w, self.sh))
 
     # ---- public API -----------------------------------------------------
     def set_input(self, radiance, albedo, normal, depth):
@@ -169,43 +203,29 @@ class UNetDenoiser:
         H, W = self.H, self.W
         self.loss.zero_()
         _check(L.lh2hip_dn_relmse(self.out.data_ptr(), COUT, target.data_ptr(), H, W, self.dout.data_ptr(), self.loss.data_ptr(), self.sh))
-        g, a, tmp = self.g, self.a, self.tmp
-        self._conv_dw(a["d_0"], "out", self.dout, H, W)
-        self._conv_dx(self.dout, "out", g["d_0"], H, W)
+        g, a = self.g, self.a
+        self._dx_relu(self.dout, "out", a["d_0"], g["d_0"], H, W)
         for lvl in range(0, LEVELS - 1):
             h, w = H >> lvl, W >> lvl
-            self._relu_bwd(a[f"d_{lvl}"], g[f"d_{lvl}"], tmp[:h * w * CH])
-            self._conv_dw(a[f"c_{lvl}"], f"d2_{lvl}", tmp, h, w)
-            self._conv_dx(tmp, f"d2_{lvl}", g[f"c_{lvl}"], h, w)
-            self._relu_bwd(a[f"c_{lvl}"], g[f"c_{lvl}"], tmp[:h * w * CH])
-            prev = a[f"d_{lvl + 1}"] if lvl + 1 < LEVELS - 1 else a[f"b_{LEVELS - 1}"]
-            _check(L.lh2hip_dn_upcat(prev.data_ptr(), CH, a[f"b_{lvl}"].data_ptr(), CH, h, w, a[f"cat_{lvl}"].data_ptr(), self.sh))
-            self._conv_dw(a[f"cat_{lvl}"], f"d1_{lvl}", tmp, h, w)
-            self._conv_dx(tmp, f"d1_{lvl}", g[f"cat_{lvl}"], h, w)
-            coarse = g[f"d_{lvl + 1}"] if lvl + 1 < LEVELS - 1 else g[f"b_{LEVELS - 1}"]
-            _check(L.lh2hip_dn_upcat_bwd(g[f"cat_{lvl}"].data_ptr(), CH, CH, h, w, coarse.data_ptr(), g[f"b_{lvl}"].data_ptr(), self.sh))
+            self._dx_relu(g[f"d_{lvl}"], f"d2_{lvl}", a[f"c_{lvl}"], g[f"c_{lvl}"], h, w)
+            _check(L.lh2hip_dn_conv3x3_dx_cat(g[f"c_{lvl}"].data_ptr(), self.p[f"d1_{lvl}"]["wb"].data_ptr(), self._below(lvl).data_ptr(),
+                                              self._below(lvl, grad=True).data_ptr(), g[f"skip_{lvl}"].data_ptr(), h, w, self.sh))
         for lvl in range(LEVELS - 1, -1, -1):
             h, w = H >> lvl, W >> lvl
             if lvl < LEVELS - 1:
-                _check(L.lh2hip_dn_pool2_bwd(g[f"in_{lvl + 1}"].data_ptr(), CH, h, w, g[f"b_{lvl}"].data_ptr(), 1, self.sh))
-            self._relu_bwd(a[f"b_{lvl}"], g[f"b_{lvl}"], tmp[:h * w * CH])
-            self._conv_dw(a[f"a_{lvl}"], f"e2_{lvl}", tmp, h, w)
-            self._conv_dx(tmp, f"e2_{lvl}", g[f"a_{lvl}"], h, w)
-            self._relu_bwd(a[f"a_{lvl}"], g[f"a_{lvl}"], tmp[:h * w * CH])
-            self._conv_dw(a[f"in_{lvl}"], f"e1_{lvl}", tmp, h, w)
+                _check(L.lh2hip_dn_pool2_bwd_relu(g[f"in_{lvl + 1}"].data_ptr(), g[f"skip_{lvl}"].data_ptr(), a[f"b_{lvl}"].data_ptr(), CH, h, w,
+                                                  g[f"b_{lvl}"].data_ptr(), self.sh))
+            self._dx_relu(g[f"b_{lvl}"], f"e2_{lvl}", a[f"a_{lvl}"], g[f"a_{lvl}"], h, w)
             if lvl > 0:
-                self._conv_dx(tmp, f"e1_{lvl}", g[f"in_{lvl}"], h, w)
+                d = self.p[f"e1_{lvl}"]
+                _check(L.lh2hip_dn_conv3x3(g[f"a_{lvl}"].data_ptr(), CH, d["wb"].data_ptr(), None, g[f"in_{lvl}"].data_ptr(), CH, h, w, 0, self.sh))
+        _check(L.lh2hip_dn_conv3x3_dw_batch(self._layers, len(self._layers), self.ws.data_ptr(), self.ws.numel() * 4, self.sh))
         return self.loss
 
     def step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         """One Adam step on every parameter (also refreshes the bf16 copies)."""
-        L = library()
         self.t += 1
-        for d in self.p.values():
-            _check(L.lh2hip_dn_adam(d["w"].data_ptr(), d["mw"].data_ptr(), d["vw"].data_ptr(), d["gw"].data_ptr(), d["w"].numel(),
-                                    lr, b1, b2, eps, self.t, d["wf"].data_ptr(), d["wb"].data_ptr(), d["co"], d["ci"], self.sh))
-            _check(L.lh2hip_dn_adam(d["b"].data_ptr(), d["mb"].data_ptr(), d["vb"].data_ptr(), d["gb"].data_ptr(), d["b"].numel(),
-                                    lr, b1, b2, eps, self.t, None, None, 0, 0, self.sh))
+        _check(library().lh2hip_dn_adam_batch(self._tensors, len(self._tensors), lr, b1, b2, eps, self.t, self.sh))
 
     def weights_blob(self):
         """The network's inference weights as one blob (the job server's

@@ -1,0 +1,151 @@
+"""The backward pass's fused and batched kernels against the separate calls they
+replace (bit for bit) and the weight gradient against FP64, at the edges of
+their tiles: 32-pixel segments and 8-row chunks of the weight gradient, 16- and
+64-pixel tiles of the convolutions, 256-element blocks of the Adam step."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import lighthouse2_amd as lh
+from lighthouse2_amd import denoiser as D
+import denoiser_ref as R
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(torch, a):
+    return torch.from_numpy(D.bf16_bits(a).reshape(-1).copy()).cuda()
+
+
+def empty(torch, n):
+    return torch.full((n,), 0x7f7f, dtype=torch.int16, device="cuda")
+
+
+def check_dw(torch, x, gy, gw, gb, terms):
+    """fp32 sums of `terms` exact products: within 1e-5 of the largest sum (as the unbatched entry point's test)."""
+    rgw, rgb = R.conv_dw(x, gy)
+    assert np.max(np.abs(gw.cpu().numpy().reshape(rgw.shape) - rgw)) <= 1e-5 * np.max(np.abs(rgw)), terms
+    assert np.max(np.abs(gb.cpu().numpy() - rgb)) <= 1e-5 * np.max(np.abs(rgb)) + 1e-6, terms
+
+
+@pytest.mark.parametrize("H,W", [(1, 1), (2, 31), (7, 32), (8, 33), (9, 64), (17, 65), (70, 34)])
+def test_weight_gradient_tile_edges(torch_cuda, H, W):
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(H * 100 + W)
+    for cin, cout in ((16, 32), (32, 32), (64, 32), (32, 16), (16, 16)):
+        x, gy = R.bf16(rng.standard_normal((H, W, cin))), R.bf16(rng.standard_normal((H, W, cout)))
+        dx, dgy = dev(torch, x), dev(torch, gy)
+        ws = torch.zeros(int(L.lh2hip_dn_dw_workspace_bytes(cin, cout)) // 4, device="cuda")
+        gw, gb = torch.full((9 * cout * cin,), 7.0, device="cuda"), torch.full((cout,), 7.0, device="cuda")
+        assert L.lh2hip_dn_conv3x3_dw(dx.data_ptr(), cin, dgy.data_ptr(), cout, H, W, gw.data_ptr(), gb.data_ptr(), ws.data_ptr(), sh) == 0
+        torch.cuda.synchronize()
+        check_dw(torch, x, gy, gw, gb, (cin, cout, H, W))
+
+
+def test_weight_gradient_batch_with_concatenation(torch_cuda):
+    """A list of layers of different sizes; one reads its 64 inputs from the two halves of a concatenation."""
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(3)
+    rows, keep, checks = [], [], []
+    for cin, cout, H, W, cat in ((16, 32, 40, 70, False), (64, 32, 22, 70, True), (32, 16, 8, 32, False), (64, 32, 6, 34, False), (32, 32, 1, 5, False)):
+        gy = R.bf16(rng.standard_normal((H, W, cout)))
+        coarse = None
+        if cat:
+            c, k = R.bf16(rng.standard_normal((H // 2, W // 2, 32))), R.bf16(rng.standard_normal((H, W, 32)))
+            x, coarse, dx = R.upcat(c, k), dev(torch, c), dev(torch, k)
+        else:
+            x = R.bf16(rng.standard_normal((H, W, cin)))
+            dx = dev(torch, x)
+        dgy, gw, gb = dev(torch, gy), torch.full((9 * cout * cin,), 7.0, device="cuda"), torch.full((cout,), 7.0, device="cuda")
+        keep += [dx, dgy, coarse]
+        rows.append(D._Layer(dx.data_ptr(), coarse.data_ptr() if cat else None, dgy.data_ptr(), gw.data_ptr(), gb.data_ptr(), cin, cout, H, W))
+        checks.append((x, gy, gw, gb))
+    t = (D._Layer * len(rows))(*rows)
+    need = int(L.lh2hip_dn_dw_batch_workspace_bytes(t, len(rows)))
+    ws = torch.zeros(need // 4, device="cuda")
+    assert L.lh2hip_dn_conv3x3_dw_batch(t, len(rows), ws.data_ptr(), need - 4, sh) != 0      # too small: refused on the host
+    assert L.lh2hip_dn_conv3x3_dw_batch(t, len(rows), ws.data_ptr(), need, sh) == 0
+    torch.cuda.synchronize()
+    for k, (x, gy, gw, gb) in enumerate(checks):
+        check_dw(torch, x, gy, gw, gb, k)
+    t[0].Cin = 48
+    assert int(L.lh2hip_dn_dw_batch_workspace_bytes(t, len(rows))) == 0
+
+
+@pytest.mark.parametrize("H,W", [(2, 2), (6, 18), (22, 70), (202, 1930)])
+def test_input_gradients_equal_their_parts(torch_cuda, H, W):
+    """dx_relu, dx_cat and pool2_bwd_relu; 202 x 1930 runs the 8 x 64 tiles, ragged both ways."""
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(W)
+    bf = lambda *s: R.bf16(rng.standard_normal(s))
+    n = H * W
+    act = bf(H, W, 32)
+    act[rng.random(act.shape) < 0.3] = 0
+    dact = dev(torch, act)
+    for cin in (16, 32):
+        gy, w = dev(torch, bf(H, W, cin)), dev(torch, bf(9, 32, cin) * 0.2)
+        want, got = empty(torch, n * 32), empty(torch, n * 32)
+        assert L.lh2hip_dn_conv3x3(gy.data_ptr(), cin, w.data_ptr(), None, want.data_ptr(), 32, H, W, 0, sh) == 0
+        assert L.lh2hip_dn_relu_bwd(dact.data_ptr(), want.data_ptr(), want.data_ptr(), n * 32, sh) == 0
+        assert L.lh2hip_dn_conv3x3_dx_relu(gy.data_ptr(), cin, w.data_ptr(), dact.data_ptr(), got.data_ptr(), 32, H, W, sh) == 0
+        assert torch.equal(want, got), cin
+    w64, ac = dev(torch, bf(9, 64, 32) * 0.2), dev(torch, bf(H // 2, W // 2, 32))
+    cat, skip, coarse = empty(torch, n * 64), empty(torch, n * 32), empty(torch, n * 8)
+    assert L.lh2hip_dn_conv3x3(gy.data_ptr(), 32, w64.data_ptr(), None, cat.data_ptr(), 64, H, W, 0, sh) == 0
+    assert L.lh2hip_dn_upcat_bwd(cat.data_ptr(), 32, 32, H, W, coarse.data_ptr(), skip.data_ptr(), sh) == 0
+    assert L.lh2hip_dn_relu_bwd(ac.data_ptr(), coarse.data_ptr(), coarse.data_ptr(), n * 8, sh) == 0
+    skip2, coarse2 = empty(torch, n * 32), empty(torch, n * 8)
+    assert L.lh2hip_dn_conv3x3_dx_cat(gy.data_ptr(), w64.data_ptr(), ac.data_ptr(), coarse2.data_ptr(), skip2.data_ptr(), H, W, sh) == 0
+    assert torch.equal(skip, skip2) and torch.equal(coarse, coarse2)
+    out = empty(torch, n * 32)
+    assert L.lh2hip_dn_pool2_bwd_relu(coarse.data_ptr(), skip.data_ptr(), dact.data_ptr(), 32, H, W, out.data_ptr(), sh) == 0
+    assert L.lh2hip_dn_pool2_bwd(coarse.data_ptr(), 32, H, W, skip.data_ptr(), 1, sh) == 0
+    assert L.lh2hip_dn_relu_bwd(dact.data_ptr(), skip.data_ptr(), skip.data_ptr(), n * 32, sh) == 0
+    assert torch.equal(skip, out)
+    assert L.lh2hip_dn_conv3x3_dx_relu(gy.data_ptr() + 2, 32, w64.data_ptr(), dact.data_ptr(), got.data_ptr(), 32, H, W, sh) != 0
+
+
+def test_adam_batch_and_vector_loss_equal_the_single_calls(torch_cuda):
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(9)
+    f = lambda n: torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()
+    rows, single = [], []
+    for n, co, ci in ((9 * 16 * 16, 16, 16), (1, 0, 0), (255, 0, 0), (257, 0, 0), (9 * 32 * 64, 32, 64)) + ((32, 0, 0),) * 50:
+        p, m, v, g = f(n), f(n), f(n).abs(), f(n)
+        wf, wb = empty(torch, n), empty(torch, n)
+        q = [t.clone() for t in (p, m, v, wf, wb)]
+        rows.append((p, m, v, g, wf, wb, n, co, ci))
+        conv = co > 0
+        assert L.lh2hip_dn_adam(q[0].data_ptr(), q[1].data_ptr(), q[2].data_ptr(), g.data_ptr(), n, 1e-3, 0.9, 0.999, 1e-8, 3,
+                                q[3].data_ptr() if conv else None, q[4].data_ptr() if conv else None, co, ci, sh) == 0
+        single.append(q)
+    t = (D._Tensor * len(rows))(*[D._Tensor(p.data_ptr(), m.data_ptr(), v.data_ptr(), g.data_ptr(), wf.data_ptr() if co else None,
+                                            wb.data_ptr() if co else None, n, co, ci) for p, m, v, g, wf, wb, n, co, ci in rows])
+    assert L.lh2hip_dn_adam_batch(t, len(rows), 1e-3, 0.9, 0.999, 1e-8, 3, sh) == 0
+    torch.cuda.synchronize()
+    for (p, m, v, g, wf, wb, n, co, ci), q in zip(rows, single):
+        assert all(torch.equal(a, b) for a, b in zip((p, m, v, wf, wb), q)), n
+    # the loss of 16 channels: aligned (vector) against one element off (scalar kernel); the sum over blocks is an atomic
+    H, W = 33, 70
+    o, tgt = rng.standard_normal((H * W * 16 + 1,)).astype(np.float32), f(H * W * 4)
+    res = []
+    for off in (0, 1):
+        buf = torch.zeros(H * W * 16 + 4, device="cuda")
+        buf[off:off + H * W * 16] = torch.from_numpy(o[:H * W * 16]).cuda()
+        dout, loss = empty(torch, H * W * 16), torch.zeros(1, device="cuda")
+        assert L.lh2hip_dn_relmse(buf.data_ptr() + 4 * off, 16, tgt.data_ptr(), H, W, dout.data_ptr(), loss.data_ptr(), sh) == 0
+        res.append((dout.clone(), float(loss.item())))
+    assert torch.equal(res[0][0], res[1][0]) and abs(res[0][1] - res[1][1]) <= 1e-5 * res[0][1]   # 10 block sums in any order
+
+
+def test_batch_records_match_the_header():
+    assert ctypes.sizeof(D._Layer) == 56 and ctypes.sizeof(D._Tensor) == 64
