@@ -369,7 +369,7 @@ void RenderCore::buildMesh(MeshData& m)
 	L.order = m.dOrder.as<uint32_t>(), L.last = m.dLast.as<uint8_t>();
 	int counts[3];
 	hipCheck(layout_device(m.dBuildNodes.as<BuildNode>(), m.dBuildPrims.as<uint32_t>(), b.nodeCount, b.levelStart, nullptr, L, counts, stream), "bvh layout");
-	m.tris.ensure(sizeof(float4) * 3 * (size_t)n);
+	m.tris.ensure(sizeof(float4) * 3 * ((size_t)n + TRACE_TRI_PAD));
 	hipCheck(gather_tris(m.verts.as<float4>(), m.dOrder.as<uint32_t>(), m.dLast.as<uint8_t>(), n, m.tris.as<float4>(), stream), "gather_tris");
 	BuildNode root;
 	hipCheck(hipMemcpyAsync(&root, m.dBuildNodes.p, sizeof(BuildNode), hipMemcpyDeviceToHost, stream), "D2H root");

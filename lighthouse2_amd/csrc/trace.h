@@ -48,6 +48,7 @@ hipError_t launch_trace_dev(const TraceScene& s, int mode, const float4* rays, v
 	uint32_t* queue, uint32_t* overflow, int persistentBlocks, hipStream_t stream, TraceStats* statsDev = nullptr);
 size_t trace_overflow_bytes(int persistentBlocks);
 
+static const int TRACE_TRI_PAD = 3;                 /* records that may be read (and are ignored) past a mesh's last leaf triangle */
 static const int TRACE_BLOCK = 256;
 static const int TRACE_LDS_STACK = 16;
 static const int TRACE_OVF_STACK = 112;

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include "lh_math.h"
 
 namespace lh {
@@ -183,6 +184,24 @@ __device__ __forceinline__ void visit_f32(const NodeF32& n, const Lane& L, Stack
 	else ref = st.sp ? st.pop() : REF_DONE;
 }
 
+/* Object-space ray and BLAS root of an instance. */
+__device__ __forceinline__ void enter_instance(const TraceScene& sc, int id, Lane& L, uint32_t& ref)
+{
+	const InstanceRec& I = sc.inst[id];
+	if (!(I.flags & 1u))
+	{
+		const float4 a = I.inv0, b = I.inv1, c = I.inv2;
+		const v3 wO = L.wO, wD = L.wD;
+		L.O = mk3(a.x * wO.x + a.y * wO.y + a.z * wO.z + a.w, b.x * wO.x + b.y * wO.y + b.z * wO.z + b.w, c.x * wO.x + c.y * wO.y + c.z * wO.z + c.w);
+		L.D = mk3(a.x * wD.x + a.y * wD.y + a.z * wD.z, b.x * wD.x + b.y * wD.y + b.z * wD.z, c.x * wD.x + c.y * wD.y + c.z * wD.z);
+		L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
+	}
+	L.rp = ray_setup(L.D);
+	L.inst = id;
+	L.nodes = I.nodes, L.tris = I.tris;
+	ref = I.root;
+}
+
 /* A top-level entry: restore the world ray if a BLAS was being walked, then
  * either enter an instance (object-space ray, BLAS root) or walk a TLAS node. */
 template <int BLOCK>
@@ -195,23 +214,7 @@ __device__ __forceinline__ void visit_top(const TraceScene& sc, Lane& L, Stack<B
 		L.inst = -1;
 	}
 	const uint32_t r = ref & ~REF_TLAS;
-	if (r & REF_LEAF)
-	{
-		const int id = (int)(r & REF_MASK);
-		const InstanceRec& I = sc.inst[id];
-		if (!(I.flags & 1u))
-		{
-			const float4 a = I.inv0, b = I.inv1, c = I.inv2;
-			const v3 wO = L.wO, wD = L.wD;
-			L.O = mk3(a.x * wO.x + a.y * wO.y + a.z * wO.z + a.w, b.x * wO.x + b.y * wO.y + b.z * wO.z + b.w, c.x * wO.x + c.y * wO.y + c.z * wO.z + c.w);
-			L.D = mk3(a.x * wD.x + a.y * wD.y + a.z * wD.z, b.x * wD.x + b.y * wD.y + b.z * wD.z, c.x * wD.x + c.y * wD.y + c.z * wD.z);
-			L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
-		}
-		L.rp = ray_setup(L.D);
-		L.inst = id;
-		L.nodes = I.nodes, L.tris = I.tris;
-		ref = I.root;
-	}
+	if (r & REF_LEAF) enter_instance(sc, (int)(r & REF_MASK), L, ref);
 	else visit_f32(sc.tlas[r], L, st, ref, REF_TLAS);
 }
 
@@ -622,6 +625,196 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 6 : 8) k_trace_ww(const Tra
 	}
 }
 
+/* ---- four lanes per ray ---------------------------------------------------
+ * A launch of few rays is one dependent chain per ray: with a lane per ray the
+ * chip holds a wave or less per SIMD, every step issues the node visit and the
+ * triangle test of 64 rays' worth of divergence, and the launch lasts as long as
+ * its longest ray (4,096 rays over 20k triangles: 181 us). Here the four lanes of
+ * a quad share a ray. A lane tests one of the node's four children (it loads 16 of
+ * the node's 64 bytes, the quad passes them round with quad_perm moves, which
+ * cost an ALU slot and no memory) and one of a leaf's triangles, so a step has
+ * half the instructions and a leaf of up to four triangles takes one. Children
+ * are ordered by ranking unique keys (the near distance's bits with the child in
+ * the two lowest), no sort. Waves hold `perWave` rays, as few as keep every SIMD
+ * busy: the fewer rays, the seldomer a wave runs the triangle test for one of
+ * them. No ray feed: quad i traces ray i, so the launch needs no counters cleared.
+ * Each lane keeps the best hit of its own triangles under the shared distance;
+ * the quad's best is picked by (t, instance, primitive) at the end, so hits equal
+ * the other loops' bit for bit. 4,096 rays: 183 -> 76 us over 20k triangles, 222 -> 99
+ * over 1,000 instances; a 256 x 256 wave of the Cornell box 151 -> 49 us. */
+static const int QUAD_BLOCK = 64;
+static const int QUAD_LDS_STACK = 32;
+
+template <int CTRL> __device__ __forceinline__ uint32_t quad_u(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
+template <int CTRL> __device__ __forceinline__ float quad_f(float v) { return bitsf(quad_u<CTRL>(fbits(v))); }
+enum { QUAD_0 = 0x00, QUAD_1 = 0x55, QUAD_2 = 0xaa, QUAD_3 = 0xff, QUAD_X1 = 0xb1, QUAD_X2 = 0x4e, QUAD_X3 = 0x1b };
+
+/* the quad's four bits of a wave ballot */
+__device__ __forceinline__ uint32_t quad_bits(uint64_t m, int lane)
+{
+	return ((lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32)) >> (lane & 28)) & 15u;
+}
+
+/* One stack per ray, entries written by the quad's lanes. */
+struct QuadStack
+{
+	lds_u32* lds;       /* QUAD_LDS_STACK x 16 rays */
+	uint32_t* ovf;      /* this ray's overflow area */
+	int ray, sp;
+	__device__ __forceinline__ void put(int at, uint32_t v)
+	{
+		if (at < QUAD_LDS_STACK) lds[at * 16 + ray] = v;
+		else if (at < TRACE_MAX_STACK) ovf[at - QUAD_LDS_STACK] = v;
+	}
+	__device__ __forceinline__ uint32_t pop()
+	{
+		sp--;
+		uint32_t v = lds[min(sp, QUAD_LDS_STACK - 1) * 16 + ray];
+		if (sp >= QUAD_LDS_STACK) v = ovf[sp - QUAD_LDS_STACK];
+		return v;
+	}
+};
+
+/* visit_q8 with a child per lane: the same planes, widening and tests. */
+__device__ __forceinline__ void visit_quad(const NodeQ8* node, int c, int lane, const Lane& L, QuadStack& st, uint32_t& ref)
+{
+	const float4 mine = ((const float4*)node)[c];
+	const uint32_t child = ((const uint32_t*)&node->refs)[c];
+	const float ox = quad_f<QUAD_0>(mine.x), oy = quad_f<QUAD_0>(mine.y), oz = quad_f<QUAD_0>(mine.z), stepz = quad_f<QUAD_0>(mine.w);
+	const uint32_t ax = quad_u<QUAD_1>(fbits(mine.x)), ay = quad_u<QUAD_1>(fbits(mine.y)), az = quad_u<QUAD_1>(fbits(mine.z)), aw = quad_u<QUAD_1>(fbits(mine.w));
+	const uint32_t bx_ = quad_u<QUAD_2>(fbits(mine.x)), by_ = quad_u<QUAD_2>(fbits(mine.y));
+	const float stepx = quad_f<QUAD_2>(mine.z), stepy = quad_f<QUAD_2>(mine.w);
+	const float dx = stepx * L.inv.x, dy = stepy * L.inv.y, dz = stepz * L.inv.z;
+	const float bx = (ox - L.O.x) * L.inv.x, by = (oy - L.O.y) * L.inv.y, bz = (oz - L.O.z) * L.inv.z;
+	const float ex = fmaf(fabsf(dx), 2.43186950683593750e-4f, fabsf(bx) * 9.5367431640625e-7f);   /* 255 * 2^-20, 2^-20 */
+	const float ey = fmaf(fabsf(dy), 2.43186950683593750e-4f, fabsf(by) * 9.5367431640625e-7f);
+	const float ez = fmaf(fabsf(dz), 2.43186950683593750e-4f, fabsf(bz) * 9.5367431640625e-7f);
+	const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
+	const int sh = 8 * c;
+	const auto plane = [&](uint32_t w) { return (float)((w >> sh) & 255u); };
+	const float qax = plane(ax), qay = plane(ay), qaz = plane(az), qbx = plane(aw), qby = plane(bx_), qbz = plane(by_);
+	const float tn = fmaxf(fmaxf(fmaf(px ? qax : qbx, dx, bx - ex), fmaf(py ? qay : qby, dy, by - ey)), fmaxf(fmaf(pz ? qaz : qbz, dz, bz - ez), L.tmin));
+	const float tf = fminf(fminf(fmaf(px ? qbx : qax, dx, bx + ex), fmaf(py ? qby : qay, dy, by + ey)), fminf(fmaf(pz ? qbz : qaz, dz, bz + ez), L.tbest));
+	const bool hit = child != Q8_EMPTY && tn <= tf;
+	const uint32_t hits = quad_bits(__ballot(hit), lane);
+	if (hits == 0)
+	{
+		ref = st.sp ? st.pop() : REF_DONE;
+		return;
+	}
+	/* order by near distance (its bits: any order is right, this one is near first for tn >= 0) */
+	const uint32_t key = ((hit ? fbits(fmaxf(tn, 0.0f)) : 0x7fffffffu) & ~3u) | (uint32_t)c;
+	const uint32_t k1 = quad_u<QUAD_X1>(key), k2 = quad_u<QUAD_X2>(key), k3 = quad_u<QUAD_X3>(key);
+	const int rank = (k1 < key) + (k2 < key) + (k3 < key), n = __popc(hits) - 1;
+	const uint32_t first = min(min(key, k1), min(k2, k3)) & 3u, far = first ^ (uint32_t)c;
+	const uint32_t r1 = quad_u<QUAD_X1>(child), r2 = quad_u<QUAD_X2>(child), r3 = quad_u<QUAD_X3>(child);
+	if (hit && rank > 0) st.put(st.sp + n - rank, child);
+	st.sp += n;
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* another lane of the quad may pop it */
+	ref = far < 2 ? (far == 0 ? child : r1) : (far == 2 ? r2 : r3);
+}
+
+template <int MODE, bool TWO>
+__global__ void __launch_bounds__(QUAD_BLOCK, 6) k_trace_quad(const TraceScene sc, const float4* __restrict__ rays, void* __restrict__ out,
+	int maxCount, const uint32_t* __restrict__ countDev, int perWave, uint32_t* __restrict__ overflow)
+{
+	__shared__ uint32_t sstack[QUAD_LDS_STACK * 16];
+	const int count = countDev ? min((int)*countDev, maxCount) : maxCount;
+	const int lane = threadIdx.x, c = lane & 3, quad = lane >> 2;
+	const int idx = (int)blockIdx.x * perWave + quad;
+	if (quad >= perWave || idx >= count) return;
+	QuadStack st;
+	st.lds = (lds_u32*)sstack, st.ovf = overflow + (size_t)idx * TRACE_OVF_STACK, st.ray = quad, st.sp = 0;
+	Lane L;
+	L.inst = -1;
+	L.nodes = sc.nodes, L.tris = sc.tris;
+	uint32_t ref = REF_DONE, pend = REF_DONE, steps = 0;
+	start_ray<TWO>(sc, rays, (uint32_t)idx, L, ref);
+	float best = L.tbest;                    /* this lane's own hit; L.tbest is the quad's nearest distance */
+	if (is_blas_leaf(ref)) pend = ref & REF_MASK, ref = REF_DONE;
+	bool any = false;
+	while (true)
+	{
+		const bool doTri = pend != REF_DONE;
+		const bool top = TWO && is_top(ref);
+		const bool doNode = is_inner(ref) || (top && !doTri);
+		if (doTri)
+		{
+			/* lane c: triangle pend + c; the ones past the leaf's last are another leaf's, or the array's padding */
+			const float4 ta = L.tris[3 * (pend + c)], tb = L.tris[3 * (pend + c) + 1], tc = L.tris[3 * (pend + c) + 2];
+			const uint32_t ends = quad_bits(__ballot((fbits(ta.w) & TRI_LAST) != 0), lane);
+			if ((ends & ((1u << c) - 1u)) == 0)
+			{
+				const int prim = (int)(fbits(ta.w) & 0x7fffffffu), instId = TWO ? L.inst : 0;
+				float t, U, V, det;
+				if (tri_intersect(L.rp, L.O, mk3(ta.x, ta.y, ta.z), mk3(tb.x, tb.y, tb.z), mk3(tc.x, tc.y, tc.z), t, U, V, det) && t > L.tmin)
+				{
+					if (MODE != MODE_CLOSEST) any = t < L.tbest;
+					else if (better_hit(t, instId, prim, best, L.binst, L.bprim))
+						best = t, L.binst = instId, L.bprim = prim, L.bU = U, L.bV = V, L.bdet = det;
+				}
+			}
+			if (MODE != MODE_CLOSEST)
+			{
+				if (quad_bits(__ballot(any), lane)) { any = true; break; }
+			}
+			else
+			{
+				const float m = fminf(best, quad_f<QUAD_X1>(best));
+				L.tbest = fminf(m, quad_f<QUAD_X2>(m));
+			}
+			pend = ends ? REF_DONE : pend + 4;
+		}
+		if (doNode)
+		{
+			if (++steps > TRACE_MAX_STEPS) ref = REF_DONE, st.sp = 0;
+			else if (!top) visit_quad((const NodeQ8*)L.nodes + ref, c, lane, L, st, ref);
+			else
+			{	/* top level: the four lanes do the same */
+				if (L.inst >= 0)
+				{
+					L.O = L.wO, L.D = L.wD;
+					L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
+					L.inst = -1;
+				}
+				const uint32_t r = ref & ~REF_TLAS;
+				if (r & REF_LEAF) enter_instance(sc, (int)(r & REF_MASK), L, ref);
+				else
+				{
+					const NodeF32 nd = sc.tlas[r];
+					float tl, tr;
+					const bool hl = slab(nd.lxy.x, nd.lxy.y, nd.lxy.z, nd.lxy.w, nd.lrz.x, nd.lrz.y, L.O, L.inv, L.tmin, L.tbest, tl);
+					const bool hr = slab(nd.rxy.x, nd.rxy.y, nd.rxy.z, nd.rxy.w, nd.lrz.z, nd.lrz.w, L.O, L.inv, L.tmin, L.tbest, tr);
+					const uint32_t rl = nd.refs.x | REF_TLAS, rr = nd.refs.y | REF_TLAS;
+					if (hl && hr)
+					{
+						st.put(st.sp, tr < tl ? rl : rr), st.sp++;
+						ref = tr < tl ? rr : rl;
+					}
+					else ref = hl ? rl : hr ? rr : st.sp ? st.pop() : REF_DONE;
+				}
+			}
+		}
+		if (pend == REF_DONE && is_blas_leaf(ref)) pend = ref & REF_MASK, ref = st.sp ? st.pop() : REF_DONE;
+		if (pend == REF_DONE && ref == REF_DONE) break;
+	}
+	if (MODE == MODE_CLOSEST)
+	{	/* the quad's best hit: two exchanges */
+		const auto take = [&](auto x) {
+			constexpr int CTRL = decltype(x)::value;
+			const float t = quad_f<CTRL>(best), U = quad_f<CTRL>(L.bU), V = quad_f<CTRL>(L.bV), det = quad_f<CTRL>(L.bdet);
+			const int inst = (int)quad_u<CTRL>((uint32_t)L.binst), prim = (int)quad_u<CTRL>((uint32_t)L.bprim);
+			if (prim >= 0 && (L.bprim < 0 || better_hit(t, inst, prim, best, L.binst, L.bprim)))
+				best = t, L.binst = inst, L.bprim = prim, L.bU = U, L.bV = V, L.bdet = det;
+		};
+		take(std::integral_constant<int, QUAD_X1>());
+		take(std::integral_constant<int, QUAD_X2>());
+		L.tbest = best;
+	}
+	else L.bprim = any ? 0 : -1;
+	if (c == 0) write_result<MODE>(L, out, idx);
+}
+
 size_t trace_overflow_bytes(int persistentBlocks)
 {
 	return (size_t)persistentBlocks * TRACE_BLOCK * TRACE_OVF_STACK * sizeof(uint32_t);
@@ -697,11 +890,39 @@ static void launch1(const TraceScene& s, int mode, const float4* rays, void* out
 	else launch2<FMT, MODE_ANY_FLAG>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
 }
 
+/* Launches of at most this many rays take four lanes per ray. Incoherent
+ * closest hits, us, a lane per ray / four lanes:
+ *   rays      20k triangles   1M triangles   1,000 instances
+ *   1,024        172 / 72        208 / 104       202 / 79
+ *   16,384       212 / 106       259 / 161       245 / 130
+ *   131,072      260 / 188       301 / 238       328 / 255
+ *   262,144      278 / 266       340 / 355       323 / 400
+ *   524,288      301 / 452       413 / 608       465 / 699 */
+static const int QUAD_MAX_RAYS = 1 << 17;
+
+template <int MODE>
+static void launch_quad(const TraceScene& s, const float4* rays, void* out, int maxCount, const uint32_t* countDev, uint32_t* overflow, hipStream_t stream)
+{
+	/* 1 to 16 rays per wave: at least as many waves as the chip has SIMDs (1,024) */
+	int perWave = 1;
+	while (perWave < 16 && maxCount / (2 * perWave) >= 1024) perWave *= 2;
+	const int blocks = (maxCount + perWave - 1) / perWave;
+	if (s.twoLevel) k_trace_quad<MODE, true><<<blocks, QUAD_BLOCK, 0, stream>>>(s, rays, out, maxCount, countDev, perWave, overflow);
+	else k_trace_quad<MODE, false><<<blocks, QUAD_BLOCK, 0, stream>>>(s, rays, out, maxCount, countDev, perWave, overflow);
+}
+
 hipError_t launch_trace_dev(const TraceScene& s, int mode, const float4* rays, void* out, int maxCount, const uint32_t* countDev,
 	uint32_t* queue, uint32_t* overflow, int blocks, hipStream_t stream, TraceStats* stats)
 {
 	if (maxCount <= 0) return hipSuccess;
 	if (s.maxStack > TRACE_MAX_STACK) return hipErrorInvalidValue;
+	if (s.format == FMT_Q8 && s.loop == LOOP_MERGED && !stats && maxCount <= QUAD_MAX_RAYS && maxCount <= blocks * TRACE_BLOCK)
+	{	/* overflow areas: one per ray */
+		if (mode == MODE_CLOSEST) launch_quad<MODE_CLOSEST>(s, rays, out, maxCount, countDev, overflow, stream);
+		else if (mode == MODE_ANY_MASK) launch_quad<MODE_ANY_MASK>(s, rays, out, maxCount, countDev, overflow, stream);
+		else launch_quad<MODE_ANY_FLAG>(s, rays, out, maxCount, countDev, overflow, stream);
+		return hipGetLastError();
+	}
 	k_reset_queue<<<1, 256, 0, stream>>>(queue);
 	if (s.format == FMT_Q8) launch1<FMT_Q8>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats);
 	else launch1<FMT_F32>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats);
