@@ -327,6 +327,187 @@ __device__ __forceinline__ void start_ray(const TraceScene& sc, const float4* ra
 #define COUNT_WAVE(pred, iters, lanes) do { if (COUNT) { const uint64_t m_ = __ballot(pred); \
 	if (m_ && __lane_id() == __ffsll((unsigned long long)m_) - 1) iters++, lanes += __popcll(m_); } } while (0)
 
+/* ---- four lanes per ray ---------------------------------------------------
+ * A launch of few rays is one dependent chain per ray: with a lane per ray the
+ * chip holds a wave or less per SIMD, every step issues the node visit and the
+ * triangle test of 64 rays' worth of divergence, and the launch lasts as long as
+ * its longest ray (4,096 rays over 20k triangles: 181 us). Here the four lanes of
+ * a quad share a ray. A lane tests one of the node's four children (it loads 16 of
+ * the node's 64 bytes, the quad passes them round with quad_perm moves, which
+ * cost an ALU slot and no memory) and one of a leaf's triangles, so a step has
+ * half the instructions and a leaf of up to four triangles takes one. Children
+ * are ordered by ranking unique keys (the near distance's bits with the child in
+ * the two lowest), no sort. Waves hold `perWave` rays, as few as keep every SIMD
+ * busy: the fewer rays, the seldomer a wave runs the triangle test for one of
+ * them. No ray feed: quad i traces ray i, so the launch needs no counters cleared.
+ * Each lane keeps the best hit of its own triangles under the shared distance;
+ * the quad's best is picked by (t, instance, primitive) at the end, so hits equal
+ * the other loops' bit for bit. 4,096 rays: 183 -> 76 us over 20k triangles, 222 -> 99
+ * over 1,000 instances; a 256 x 256 wave of the Cornell box 151 -> 49 us. */
+static const int QUAD_BLOCK = 64;
+static const int QUAD_LDS_STACK = 32;
+static const int TAIL_RAYS = 16;   /* merged loop: rays of a wave that continue with four lanes each once the feed is dry */
+
+template <int CTRL> __device__ __forceinline__ uint32_t quad_u(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
+template <int CTRL> __device__ __forceinline__ float quad_f(float v) { return bitsf(quad_u<CTRL>(fbits(v))); }
+enum { QUAD_0 = 0x00, QUAD_1 = 0x55, QUAD_2 = 0xaa, QUAD_3 = 0xff, QUAD_X1 = 0xb1, QUAD_X2 = 0x4e, QUAD_X3 = 0x1b };
+
+/* the quad's four bits of a wave ballot */
+__device__ __forceinline__ uint32_t quad_bits(uint64_t m, int lane)
+{
+	return ((lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32)) >> (lane & 28)) & 15u;
+}
+
+/* One stack per ray, entries written by the quad's lanes: DEPTH in LDS
+ * (interleaved over STRIDE rays), the others in the ray's overflow area. */
+template <int DEPTH, int STRIDE>
+struct QuadStack
+{
+	lds_u32* lds;
+	uint32_t* ovf;
+	int col, sp;
+	__device__ __forceinline__ void put(int at, uint32_t v)
+	{
+		if (at < DEPTH) lds[at * STRIDE + col] = v;
+		else if (at < TRACE_MAX_STACK) ovf[at - DEPTH] = v;
+	}
+	__device__ __forceinline__ uint32_t pop()
+	{
+		sp--;
+		uint32_t v = lds[min(sp, DEPTH - 1) * STRIDE + col];
+		if (sp >= DEPTH) v = ovf[sp - DEPTH];
+		return v;
+	}
+};
+
+/* visit_q8 with a child per lane: the same planes, widening and tests. */
+template <typename STACK>
+__device__ __forceinline__ void visit_quad(const NodeQ8* node, int c, int lane, const Lane& L, STACK& st, uint32_t& ref)
+{
+	const float4 mine = ((const float4*)node)[c];
+	const uint32_t child = ((const uint32_t*)&node->refs)[c];
+	const float ox = quad_f<QUAD_0>(mine.x), oy = quad_f<QUAD_0>(mine.y), oz = quad_f<QUAD_0>(mine.z), stepz = quad_f<QUAD_0>(mine.w);
+	const uint32_t ax = quad_u<QUAD_1>(fbits(mine.x)), ay = quad_u<QUAD_1>(fbits(mine.y)), az = quad_u<QUAD_1>(fbits(mine.z)), aw = quad_u<QUAD_1>(fbits(mine.w));
+	const uint32_t bx_ = quad_u<QUAD_2>(fbits(mine.x)), by_ = quad_u<QUAD_2>(fbits(mine.y));
+	const float stepx = quad_f<QUAD_2>(mine.z), stepy = quad_f<QUAD_2>(mine.w);
+	const float dx = stepx * L.inv.x, dy = stepy * L.inv.y, dz = stepz * L.inv.z;
+	const float bx = (ox - L.O.x) * L.inv.x, by = (oy - L.O.y) * L.inv.y, bz = (oz - L.O.z) * L.inv.z;
+	const float ex = fmaf(fabsf(dx), 2.43186950683593750e-4f, fabsf(bx) * 9.5367431640625e-7f);   /* 255 * 2^-20, 2^-20 */
+	const float ey = fmaf(fabsf(dy), 2.43186950683593750e-4f, fabsf(by) * 9.5367431640625e-7f);
+	const float ez = fmaf(fabsf(dz), 2.43186950683593750e-4f, fabsf(bz) * 9.5367431640625e-7f);
+	const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
+	const int sh = 8 * c;
+	const auto plane = [&](uint32_t w) { return (float)((w >> sh) & 255u); };
+	const float qax = plane(ax), qay = plane(ay), qaz = plane(az), qbx = plane(aw), qby = plane(bx_), qbz = plane(by_);
+	const float tn = fmaxf(fmaxf(fmaf(px ? qax : qbx, dx, bx - ex), fmaf(py ? qay : qby, dy, by - ey)), fmaxf(fmaf(pz ? qaz : qbz, dz, bz - ez), L.tmin));
+	const float tf = fminf(fminf(fmaf(px ? qbx : qax, dx, bx + ex), fmaf(py ? qby : qay, dy, by + ey)), fminf(fmaf(pz ? qbz : qaz, dz, bz + ez), L.tbest));
+	const bool hit = child != Q8_EMPTY && tn <= tf;
+	const uint32_t hits = quad_bits(__ballot(hit), lane);
+	if (hits == 0)
+	{
+		ref = st.sp ? st.pop() : REF_DONE;
+		return;
+	}
+	/* order by near distance (its bits: any order is right, this one is near first for tn >= 0) */
+	const uint32_t key = ((hit ? fbits(fmaxf(tn, 0.0f)) : 0x7fffffffu) & ~3u) | (uint32_t)c;
+	const uint32_t k1 = quad_u<QUAD_X1>(key), k2 = quad_u<QUAD_X2>(key), k3 = quad_u<QUAD_X3>(key);
+	const int rank = (k1 < key) + (k2 < key) + (k3 < key), n = __popc(hits) - 1;
+	const uint32_t first = min(min(key, k1), min(k2, k3)) & 3u, far = first ^ (uint32_t)c;
+	const uint32_t r1 = quad_u<QUAD_X1>(child), r2 = quad_u<QUAD_X2>(child), r3 = quad_u<QUAD_X3>(child);
+	if (hit && rank > 0) st.put(st.sp + n - rank, child);
+	st.sp += n;
+	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* another lane of the quad may pop it */
+	ref = far < 2 ? (far == 0 ? child : r1) : (far == 2 ? r2 : r3);
+}
+
+/* Walks a quad's ray from (ref, pend, stack) to its end; the result is in L of
+ * every lane. best: this lane's own hit (with L's hit fields), L.tbest the
+ * quad's nearest distance. */
+template <int MODE, bool TWO, typename STACK>
+__device__ __forceinline__ void quad_walk(const TraceScene& sc, Lane& L, STACK& st, uint32_t ref, uint32_t pend, uint32_t steps, int c, int lane, float best)
+{
+	bool any = false;
+	while (true)
+	{
+		const bool doTri = pend != REF_DONE;
+		const bool top = TWO && is_top(ref);
+		const bool doNode = is_inner(ref) || (top && !doTri);
+		if (doTri)
+		{
+			/* lane c: triangle pend + c; the ones past the leaf's last are another leaf's, or the array's padding */
+			const float4 ta = L.tris[3 * (pend + c)], tb = L.tris[3 * (pend + c) + 1], tc = L.tris[3 * (pend + c) + 2];
+			const uint32_t ends = quad_bits(__ballot((fbits(ta.w) & TRI_LAST) != 0), lane);
+			if ((ends & ((1u << c) - 1u)) == 0)
+			{
+				const int prim = (int)(fbits(ta.w) & 0x7fffffffu), instId = TWO ? L.inst : 0;
+				float t, U, V, det;
+				if (tri_intersect(L.rp, L.O, mk3(ta.x, ta.y, ta.z), mk3(tb.x, tb.y, tb.z), mk3(tc.x, tc.y, tc.z), t, U, V, det) && t > L.tmin)
+				{
+					if (MODE != MODE_CLOSEST) any = t < L.tbest;
+					else if (better_hit(t, instId, prim, best, L.binst, L.bprim))
+						best = t, L.binst = instId, L.bprim = prim, L.bU = U, L.bV = V, L.bdet = det;
+				}
+			}
+			if (MODE != MODE_CLOSEST)
+			{
+				if (quad_bits(__ballot(any), lane)) { any = true; break; }
+			}
+			else
+			{
+				const float m = fminf(best, quad_f<QUAD_X1>(best));
+				L.tbest = fminf(m, quad_f<QUAD_X2>(m));
+			}
+			pend = ends ? REF_DONE : pend + 4;
+		}
+		if (doNode)
+		{
+			if (++steps > TRACE_MAX_STEPS) ref = REF_DONE, st.sp = 0;
+			else if (!top) visit_quad((const NodeQ8*)L.nodes + ref, c, lane, L, st, ref);
+			else
+			{	/* top level: the four lanes do the same */
+				if (L.inst >= 0)
+				{
+					L.O = L.wO, L.D = L.wD;
+					L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
+					L.inst = -1;
+				}
+				const uint32_t r = ref & ~REF_TLAS;
+				if (r & REF_LEAF) enter_instance(sc, (int)(r & REF_MASK), L, ref);
+				else
+				{
+					const NodeF32 nd = sc.tlas[r];
+					float tl, tr;
+					const bool hl = slab(nd.lxy.x, nd.lxy.y, nd.lxy.z, nd.lxy.w, nd.lrz.x, nd.lrz.y, L.O, L.inv, L.tmin, L.tbest, tl);
+					const bool hr = slab(nd.rxy.x, nd.rxy.y, nd.rxy.z, nd.rxy.w, nd.lrz.z, nd.lrz.w, L.O, L.inv, L.tmin, L.tbest, tr);
+					const uint32_t rl = nd.refs.x | REF_TLAS, rr = nd.refs.y | REF_TLAS;
+					if (hl && hr)
+					{
+						st.put(st.sp, tr < tl ? rl : rr), st.sp++;
+						ref = tr < tl ? rr : rl;
+					}
+					else ref = hl ? rl : hr ? rr : st.sp ? st.pop() : REF_DONE;
+				}
+			}
+		}
+		if (pend == REF_DONE && is_blas_leaf(ref)) pend = ref & REF_MASK, ref = st.sp ? st.pop() : REF_DONE;
+		if (pend == REF_DONE && ref == REF_DONE) break;
+	}
+	if (MODE == MODE_CLOSEST)
+	{	/* the quad's best hit: two exchanges */
+		const auto take = [&](auto x) {
+			constexpr int CTRL = decltype(x)::value;
+			const float t = quad_f<CTRL>(best), U = quad_f<CTRL>(L.bU), V = quad_f<CTRL>(L.bV), det = quad_f<CTRL>(L.bdet);
+			const int inst = (int)quad_u<CTRL>((uint32_t)L.binst), prim = (int)quad_u<CTRL>((uint32_t)L.bprim);
+			if (prim >= 0 && (L.bprim < 0 || better_hit(t, inst, prim, best, L.binst, L.bprim)))
+				best = t, L.binst = inst, L.bprim = prim, L.bU = U, L.bV = V, L.bdet = det;
+		};
+		take(std::integral_constant<int, QUAD_X1>());
+		take(std::integral_constant<int, QUAD_X2>());
+		L.tbest = best;
+	}
+	else L.bprim = any ? 0 : -1;
+}
+
 /* Merged loop (default): every iteration each lane tests one pending leaf
  * triangle and visits one node, both predicated, with both loads issued at
  * the top of the iteration. Lanes never wait for one another between a node
@@ -346,6 +527,7 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 	bool active = false, exhausted = false;
 	uint32_t ref = REF_DONE, pend = REF_DONE, steps = 0;
 	unsigned long long cn = 0, ct = 0, wn = 0, wl = 0, fn = 0, fl = 0, li = 0, ll = 0, ti = 0, tl = 0;
+	constexpr bool TAIL = FMT == FMT_Q8 && !COUNT;
 	Feed feed;
 	feed_init(feed);
 	if (COUNT && threadIdx.x == 0) atomicMin(&stats->tStart, (unsigned long long)wall_clock64());
@@ -366,6 +548,7 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 				active = true;
 			}
 		}
+		if (TAIL && exhausted && __popcll(__ballot(active)) <= TAIL_RAYS) break;
 		if (!__any(active))
 		{
 			if (exhausted) break;
@@ -375,7 +558,8 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 		bool finished = false;
 		while (true)
 		{
-			if (!exhausted && __popcll(__ballot(true)) <= 64 - sc.refillLanes) break;
+			if (TAIL ? __popcll(__ballot(true)) <= (exhausted ? TAIL_RAYS : 64 - sc.refillLanes) : !exhausted && __popcll(__ballot(true)) <= 64 - sc.refillLanes)
+				break;
 			if (exhausted) COUNT_WAVE(true, ti, tl); else COUNT_WAVE(true, li, ll);
 			const bool doTri = pend != REF_DONE;
 			const bool doNode = is_inner(ref) || (TWO && is_top(ref) && !doTri);
@@ -416,6 +600,33 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 		if (!finished) continue;
 		write_result<MODE>(L, out, rayIdx);
 		active = false;
+	}
+	if (TAIL)
+	{	/* The wave's last rays (at most 16), four lanes each: quad q takes the q-th lane that still holds one. With
+		 * the feed dry a launch lasts until its longest rays end, and a step costs a wave the same for one ray as
+		 * for 64; the quads' steps have half the instructions. 1 M rays towards area lights over 1,000 instances
+		 * 764 -> 689 us, 2 M incoherent rays over 4 M triangles 1,100 -> 1,068 us (12 rays instead of 16: the
+		 * same within 2%; the ray's state moves by lane shuffles and the LDS stack stays where it is, so the
+		 * main loop keeps its registers). */
+		uint64_t m = __ballot(active);
+		const int lane = threadIdx.x & 63, c = lane & 3;
+		for (int q = lane >> 2; q > 0; q--) m &= m - 1;
+		const bool mine = m != 0;
+		const int src = mine ? __ffsll((unsigned long long)m) - 1 : 0;
+		rayIdx = __shfl(rayIdx, src), ref = (uint32_t)__shfl((int)ref, src), pend = (uint32_t)__shfl((int)pend, src), steps = (uint32_t)__shfl((int)steps, src);
+		const float tbest = __shfl(L.tbest, src), U = __shfl(L.bU, src), V = __shfl(L.bV, src), det = __shfl(L.bdet, src);
+		const int binst = __shfl(L.binst, src), bprim = __shfl(L.bprim, src), inst = TWO ? __shfl(L.inst, src) : -1;
+		QuadStack<TRACE_LDS_STACK, TRACE_BLOCK> qs;
+		qs.sp = __shfl(st.sp, src), qs.lds = st.lds, qs.col = (int)(threadIdx.x & ~63u) + src;
+		qs.ovf = overflow + ((size_t)blockIdx.x * TRACE_BLOCK + qs.col) * TRACE_OVF_STACK;
+		__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+		if (!mine) return;
+		uint32_t root;
+		start_ray<TWO>(sc, rays, (uint32_t)rayIdx, L, root);
+		if (TWO && inst >= 0) enter_instance(sc, inst, L, root);
+		L.tbest = tbest, L.bU = U, L.bV = V, L.bdet = det, L.binst = binst, L.bprim = bprim;
+		quad_walk<MODE, TWO>(sc, L, qs, ref, pend, steps, c, lane, tbest);
+		if (c == 0) write_result<MODE>(L, out, rayIdx);
 	}
 	if (COUNT)
 	{
@@ -625,95 +836,6 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 6 : 8) k_trace_ww(const Tra
 	}
 }
 
-/* ---- four lanes per ray ---------------------------------------------------
- * A launch of few rays is one dependent chain per ray: with a lane per ray the
- * chip holds a wave or less per SIMD, every step issues the node visit and the
- * triangle test of 64 rays' worth of divergence, and the launch lasts as long as
- * its longest ray (4,096 rays over 20k triangles: 181 us). Here the four lanes of
- * a quad share a ray. A lane tests one of the node's four children (it loads 16 of
- * the node's 64 bytes, the quad passes them round with quad_perm moves, which
- * cost an ALU slot and no memory) and one of a leaf's triangles, so a step has
- * half the instructions and a leaf of up to four triangles takes one. Children
- * are ordered by ranking unique keys (the near distance's bits with the child in
- * the two lowest), no sort. Waves hold `perWave` rays, as few as keep every SIMD
- * busy: the fewer rays, the seldomer a wave runs the triangle test for one of
- * them. No ray feed: quad i traces ray i, so the launch needs no counters cleared.
- * Each lane keeps the best hit of its own triangles under the shared distance;
- * the quad's best is picked by (t, instance, primitive) at the end, so hits equal
- * the other loops' bit for bit. 4,096 rays: 183 -> 76 us over 20k triangles, 222 -> 99
- * over 1,000 instances; a 256 x 256 wave of the Cornell box 151 -> 49 us. */
-static const int QUAD_BLOCK = 64;
-static const int QUAD_LDS_STACK = 32;
-
-template <int CTRL> __device__ __forceinline__ uint32_t quad_u(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true); }
-template <int CTRL> __device__ __forceinline__ float quad_f(float v) { return bitsf(quad_u<CTRL>(fbits(v))); }
-enum { QUAD_0 = 0x00, QUAD_1 = 0x55, QUAD_2 = 0xaa, QUAD_3 = 0xff, QUAD_X1 = 0xb1, QUAD_X2 = 0x4e, QUAD_X3 = 0x1b };
-
-/* the quad's four bits of a wave ballot */
-__device__ __forceinline__ uint32_t quad_bits(uint64_t m, int lane)
-{
-	return ((lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32)) >> (lane & 28)) & 15u;
-}
-
-/* One stack per ray, entries written by the quad's lanes. */
-struct QuadStack
-{
-	lds_u32* lds;       /* QUAD_LDS_STACK x 16 rays */
-	uint32_t* ovf;      /* this ray's overflow area */
-	int ray, sp;
-	__device__ __forceinline__ void put(int at, uint32_t v)
-	{
-		if (at < QUAD_LDS_STACK) lds[at * 16 + ray] = v;
-		else if (at < TRACE_MAX_STACK) ovf[at - QUAD_LDS_STACK] = v;
-	}
-	__device__ __forceinline__ uint32_t pop()
-	{
-		sp--;
-		uint32_t v = lds[min(sp, QUAD_LDS_STACK - 1) * 16 + ray];
-		if (sp >= QUAD_LDS_STACK) v = ovf[sp - QUAD_LDS_STACK];
-		return v;
-	}
-};
-
-/* visit_q8 with a child per lane: the same planes, widening and tests. */
-__device__ __forceinline__ void visit_quad(const NodeQ8* node, int c, int lane, const Lane& L, QuadStack& st, uint32_t& ref)
-{
-	const float4 mine = ((const float4*)node)[c];
-	const uint32_t child = ((const uint32_t*)&node->refs)[c];
-	const float ox = quad_f<QUAD_0>(mine.x), oy = quad_f<QUAD_0>(mine.y), oz = quad_f<QUAD_0>(mine.z), stepz = quad_f<QUAD_0>(mine.w);
-	const uint32_t ax = quad_u<QUAD_1>(fbits(mine.x)), ay = quad_u<QUAD_1>(fbits(mine.y)), az = quad_u<QUAD_1>(fbits(mine.z)), aw = quad_u<QUAD_1>(fbits(mine.w));
-	const uint32_t bx_ = quad_u<QUAD_2>(fbits(mine.x)), by_ = quad_u<QUAD_2>(fbits(mine.y));
-	const float stepx = quad_f<QUAD_2>(mine.z), stepy = quad_f<QUAD_2>(mine.w);
-	const float dx = stepx * L.inv.x, dy = stepy * L.inv.y, dz = stepz * L.inv.z;
-	const float bx = (ox - L.O.x) * L.inv.x, by = (oy - L.O.y) * L.inv.y, bz = (oz - L.O.z) * L.inv.z;
-	const float ex = fmaf(fabsf(dx), 2.43186950683593750e-4f, fabsf(bx) * 9.5367431640625e-7f);   /* 255 * 2^-20, 2^-20 */
-	const float ey = fmaf(fabsf(dy), 2.43186950683593750e-4f, fabsf(by) * 9.5367431640625e-7f);
-	const float ez = fmaf(fabsf(dz), 2.43186950683593750e-4f, fabsf(bz) * 9.5367431640625e-7f);
-	const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
-	const int sh = 8 * c;
-	const auto plane = [&](uint32_t w) { return (float)((w >> sh) & 255u); };
-	const float qax = plane(ax), qay = plane(ay), qaz = plane(az), qbx = plane(aw), qby = plane(bx_), qbz = plane(by_);
-	const float tn = fmaxf(fmaxf(fmaf(px ? qax : qbx, dx, bx - ex), fmaf(py ? qay : qby, dy, by - ey)), fmaxf(fmaf(pz ? qaz : qbz, dz, bz - ez), L.tmin));
-	const float tf = fminf(fminf(fmaf(px ? qbx : qax, dx, bx + ex), fmaf(py ? qby : qay, dy, by + ey)), fminf(fmaf(pz ? qbz : qaz, dz, bz + ez), L.tbest));
-	const bool hit = child != Q8_EMPTY && tn <= tf;
-	const uint32_t hits = quad_bits(__ballot(hit), lane);
-	if (hits == 0)
-	{
-		ref = st.sp ? st.pop() : REF_DONE;
-		return;
-	}
-	/* order by near distance (its bits: any order is right, this one is near first for tn >= 0) */
-	const uint32_t key = ((hit ? fbits(fmaxf(tn, 0.0f)) : 0x7fffffffu) & ~3u) | (uint32_t)c;
-	const uint32_t k1 = quad_u<QUAD_X1>(key), k2 = quad_u<QUAD_X2>(key), k3 = quad_u<QUAD_X3>(key);
-	const int rank = (k1 < key) + (k2 < key) + (k3 < key), n = __popc(hits) - 1;
-	const uint32_t first = min(min(key, k1), min(k2, k3)) & 3u, far = first ^ (uint32_t)c;
-	const uint32_t r1 = quad_u<QUAD_X1>(child), r2 = quad_u<QUAD_X2>(child), r3 = quad_u<QUAD_X3>(child);
-	if (hit && rank > 0) st.put(st.sp + n - rank, child);
-	st.sp += n;
-	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* another lane of the quad may pop it */
-	ref = far < 2 ? (far == 0 ? child : r1) : (far == 2 ? r2 : r3);
-}
-
 template <int MODE, bool TWO>
 __global__ void __launch_bounds__(QUAD_BLOCK, 6) k_trace_quad(const TraceScene sc, const float4* __restrict__ rays, void* __restrict__ out,
 	int maxCount, const uint32_t* __restrict__ countDev, int perWave, uint32_t* __restrict__ overflow)
@@ -723,8 +845,8 @@ __global__ void __launch_bounds__(QUAD_BLOCK, 6) k_trace_quad(const TraceScene s
 	const int lane = threadIdx.x, c = lane & 3, quad = lane >> 2;
 	const int idx = (int)blockIdx.x * perWave + quad;
 	if (quad >= perWave || idx >= count) return;
-	QuadStack st;
-	st.lds = (lds_u32*)sstack, st.ovf = overflow + (size_t)idx * TRACE_OVF_STACK, st.ray = quad, st.sp = 0;
+	QuadStack<QUAD_LDS_STACK, 16> st;
+	st.lds = (lds_u32*)sstack, st.ovf = overflow + (size_t)idx * TRACE_OVF_STACK, st.col = quad, st.sp = 0;
 	Lane L;
 	L.inst = -1;
 	L.nodes = sc.nodes, L.tris = sc.tris;
@@ -732,86 +854,7 @@ __global__ void __launch_bounds__(QUAD_BLOCK, 6) k_trace_quad(const TraceScene s
 	start_ray<TWO>(sc, rays, (uint32_t)idx, L, ref);
 	float best = L.tbest;                    /* this lane's own hit; L.tbest is the quad's nearest distance */
 	if (is_blas_leaf(ref)) pend = ref & REF_MASK, ref = REF_DONE;
-	bool any = false;
-	while (true)
-	{
-		const bool doTri = pend != REF_DONE;
-		const bool top = TWO && is_top(ref);
-		const bool doNode = is_inner(ref) || (top && !doTri);
-		if (doTri)
-		{
-			/* lane c: triangle pend + c; the ones past the leaf's last are another leaf's, or the array's padding */
-			const float4 ta = L.tris[3 * (pend + c)], tb = L.tris[3 * (pend + c) + 1], tc = L.tris[3 * (pend + c) + 2];
-			const uint32_t ends = quad_bits(__ballot((fbits(ta.w) & TRI_LAST) != 0), lane);
-			if ((ends & ((1u << c) - 1u)) == 0)
-			{
-				const int prim = (int)(fbits(ta.w) & 0x7fffffffu), instId = TWO ? L.inst : 0;
-				float t, U, V, det;
-				if (tri_intersect(L.rp, L.O, mk3(ta.x, ta.y, ta.z), mk3(tb.x, tb.y, tb.z), mk3(tc.x, tc.y, tc.z), t, U, V, det) && t > L.tmin)
-				{
-					if (MODE != MODE_CLOSEST) any = t < L.tbest;
-					else if (better_hit(t, instId, prim, best, L.binst, L.bprim))
-						best = t, L.binst = instId, L.bprim = prim, L.bU = U, L.bV = V, L.bdet = det;
-				}
-			}
-			if (MODE != MODE_CLOSEST)
-			{
-				if (quad_bits(__ballot(any), lane)) { any = true; break; }
-			}
-			else
-			{
-				const float m = fminf(best, quad_f<QUAD_X1>(best));
-				L.tbest = fminf(m, quad_f<QUAD_X2>(m));
-			}
-			pend = ends ? REF_DONE : pend + 4;
-		}
-		if (doNode)
-		{
-			if (++steps > TRACE_MAX_STEPS) ref = REF_DONE, st.sp = 0;
-			else if (!top) visit_quad((const NodeQ8*)L.nodes + ref, c, lane, L, st, ref);
-			else
-			{	/* top level: the four lanes do the same */
-				if (L.inst >= 0)
-				{
-					L.O = L.wO, L.D = L.wD;
-					L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
-					L.inst = -1;
-				}
-				const uint32_t r = ref & ~REF_TLAS;
-				if (r & REF_LEAF) enter_instance(sc, (int)(r & REF_MASK), L, ref);
-				else
-				{
-					const NodeF32 nd = sc.tlas[r];
-					float tl, tr;
-					const bool hl = slab(nd.lxy.x, nd.lxy.y, nd.lxy.z, nd.lxy.w, nd.lrz.x, nd.lrz.y, L.O, L.inv, L.tmin, L.tbest, tl);
-					const bool hr = slab(nd.rxy.x, nd.rxy.y, nd.rxy.z, nd.rxy.w, nd.lrz.z, nd.lrz.w, L.O, L.inv, L.tmin, L.tbest, tr);
-					const uint32_t rl = nd.refs.x | REF_TLAS, rr = nd.refs.y | REF_TLAS;
-					if (hl && hr)
-					{
-						st.put(st.sp, tr < tl ? rl : rr), st.sp++;
-						ref = tr < tl ? rr : rl;
-					}
-					else ref = hl ? rl : hr ? rr : st.sp ? st.pop() : REF_DONE;
-				}
-			}
-		}
-		if (pend == REF_DONE && is_blas_leaf(ref)) pend = ref & REF_MASK, ref = st.sp ? st.pop() : REF_DONE;
-		if (pend == REF_DONE && ref == REF_DONE) break;
-	}
-	if (MODE == MODE_CLOSEST)
-	{	/* the quad's best hit: two exchanges */
-		const auto take = [&](auto x) {
-			constexpr int CTRL = decltype(x)::value;
-			const float t = quad_f<CTRL>(best), U = quad_f<CTRL>(L.bU), V = quad_f<CTRL>(L.bV), det = quad_f<CTRL>(L.bdet);
-			const int inst = (int)quad_u<CTRL>((uint32_t)L.binst), prim = (int)quad_u<CTRL>((uint32_t)L.bprim);
-			if (prim >= 0 && (L.bprim < 0 || better_hit(t, inst, prim, best, L.binst, L.bprim)))
-				best = t, L.binst = inst, L.bprim = prim, L.bU = U, L.bV = V, L.bdet = det;
-		};
-		take(std::integral_constant<int, QUAD_X1>());
-		take(std::integral_constant<int, QUAD_X2>());
-		L.tbest = best;
-	}
-	else L.bprim = any ? 0 : -1;
+	quad_walk<MODE, TWO>(sc, L, st, ref, pend, steps, c, lane, best);
 	if (c == 0) write_result<MODE>(L, out, idx);
 }
 
