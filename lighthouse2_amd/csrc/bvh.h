@@ -61,7 +61,8 @@ struct InstanceRec
 	uint32_t flags;            /* bit 0: identity transform */
 };
 
-/* Result of a GPU build: device arrays (owned by the caller). */
+/* A GPU build: the caller's device arrays (2 n nodes, n primitives) and what
+ * the build found. */
 struct DeviceBuild
 {
 	BuildNode* nodes = nullptr;
@@ -72,17 +73,38 @@ struct DeviceBuild
 
 /* Binned SAH (16 bins) over primitive boxes lo[i].xyz / hi[i].xyz on the GPU.
  * maxLeaf: largest SAH leaf; maxDegenerateLeaf: largest leaf when all
- * centroids coincide (beyond it the range is halved). Returns hipSuccess or an error. */
+ * centroids coincide (beyond it the range is halved). ws: device memory of
+ * gpu_build_workspace_bytes(n), free for other use once the stream has passed
+ * the build. Returns hipSuccess or an error. */
+size_t gpu_build_workspace_bytes(int n);
 hipError_t gpu_build(const float4* dLo, const float4* dHi, int n, int maxLeaf, int maxDegenerateLeaf,
-	DeviceBuild& out, hipStream_t stream);
-void free_build(DeviceBuild& b);
+	DeviceBuild& out, void* ws, size_t wsBytes, hipStream_t stream);
 
-/* Refit on the device, topology unchanged. Boxes of the build nodes
- * first .. first+count-1 (one tree level: leaves take the min / max of their
- * triangles' vertices, interior nodes the union of their two children, which
- * must already be refitted); then the laid-out f32 / q8 nodes are rewritten
- * from the refitted build boxes through the layout maps (refs unchanged). */
-hipError_t refit_level(BuildNode* dNodes, const uint32_t* dPrims, const float4* dVerts, int first, int count, hipStream_t stream);
+/* Passes over a tree level by level are launch-bound where levels are small: up
+ * to 64 consecutive levels of at most 2,048 nodes run in one block, a barrier
+ * between two (a launch of its own costs a level 4-5 us, a barrier and a round
+ * of loads 1-2 us). s[0] .. s[n]: their build ids, by depth. */
+static const int LEVELS_BLOCK = 1024, LEVELS_NODES = 2048;
+struct LevelRange { int n; int s[65]; };
+/* The levels from depth `at` down (down true), or ending above depth `at`. */
+inline LevelRange small_levels(const std::vector<int>& levelStart, int at, bool down)
+{
+	const int levels = (int)levelStart.size() - 1;
+	const auto small = [&](int d) { return d >= 0 && d < levels && levelStart[d + 1] - levelStart[d] <= LEVELS_NODES; };
+	LevelRange r;
+	r.n = 0;
+	while (r.n < 64 && small(down ? at + r.n : at - 1 - r.n)) r.n++;
+	const int d0 = down ? at : at - r.n;
+	for (int k = 0; k <= r.n; k++) r.s[k] = levelStart[d0 + k];
+	return r;
+}
+
+/* Refit on the device, topology unchanged. Boxes of the build nodes, deepest
+ * level first (leaves take the min / max of their triangles' vertices, interior
+ * nodes the union of their two children); then the laid-out f32 / q8 nodes are
+ * rewritten from the refitted build boxes through the layout maps (refs
+ * unchanged). */
+hipError_t refit_levels(BuildNode* dNodes, const uint32_t* dPrims, const float4* dVerts, const std::vector<int>& levelStart, hipStream_t stream);
 hipError_t refit_layout(const BuildNode* dNodes, NodeF32* dF32, const int32_t* dF32Kids, int nF32, NodeQ8* dQ8, const int32_t* dQ8Map, int nQ8, hipStream_t stream);
 
 /* Triangle soup (3 float4 per triangle) -> primitive boxes. */
@@ -106,10 +128,14 @@ struct LayoutOut
 /* levelStart[d]..levelStart[d+1]: the build ids of depth d (gpu_build's breadth-first
  * order). leafRefMap non-null (top level, one primitive per leaf): leaf refs are
  * REF_LEAF | leafRefMap[primitive] and no triangle order is written.
- * countsOut (host, may be null; the call then waits for the stream): [0] f32
- * nodes, [1] q8 nodes, [2] q8 tree depth. */
+ * ws: device memory of layout_workspace_bytes(nodeCount, q8 wanted), needed
+ * until layout_counts (or, without it, until the stream has passed the layout). */
+size_t layout_workspace_bytes(int nodeCount, bool q8);
 hipError_t layout_device(const BuildNode* dNodes, const uint32_t* dPrims, int nodeCount, const std::vector<int>& levelStart,
-	const uint32_t* leafRefMap, const LayoutOut& out, int* countsOut, hipStream_t stream);
+	const uint32_t* leafRefMap, const LayoutOut& out, void* ws, size_t wsBytes, hipStream_t stream);
+/* What the layout found, read back from its workspace (waits for the stream). */
+struct LayoutCounts { int nF32, nQ8, depthQ8, pad; BuildNode root; };
+hipError_t layout_counts(const void* ws, LayoutCounts& out, hipStream_t stream);
 
 /* Gathers leaf triangles: tris[3*i+k] = verts[3*order[i]+k], v0.w = prim | last bit. */
 hipError_t gather_tris(const float4* dVerts, const uint32_t* dOrder, const uint8_t* dLast, int n, float4* dTris, hipStream_t stream);

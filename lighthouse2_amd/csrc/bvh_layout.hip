@@ -22,12 +22,13 @@
  *
  * The build tree is breadth-first: the nodes of depth d are the id range
  * [levelStart[d], levelStart[d+1]) and children lie one level below their
- * parent. Every pass is one launch per level, one thread per node:
+ * parent. Every pass goes level by level, one thread per node (a launch per
+ * level, small levels together in one block, see bvh.h):
  *   up1   subtree triangle count and interior-node count (deepest level first);
  *   down1 leaf bases, f32 slots and nodes, the leaf triangle order, and which
  *         binary nodes head a 4-wide node (with their children);
  *   up2   4-wide subtree sizes;
- *   down2 4-wide slots and quantised nodes.
+ *   down2 4-wide slots and child refs; the boxes are quantised afterwards, all at once.
  */
 #include "bvh.h"
 #include "lh_math.h"
@@ -54,7 +55,7 @@ struct LayoutArgs
 	int32_t* q8Map;
 	uint32_t* order;
 	uint8_t* last;
-	int* info;                    /* [0] = 4-wide depth */
+	LayoutCounts* info;
 };
 
 __device__ __forceinline__ int& fld(const LayoutArgs& a, int field, int x) { return a.f[(size_t)field * a.nodeCount + x]; }
@@ -65,28 +66,23 @@ __device__ __forceinline__ float node_half_area(const BuildNode& b)
 	return dx * dy + dy * dz + dz * dx;
 }
 
-__global__ void k_lay_root(LayoutArgs a)
+/* The root's fields; WLEV = -1 for every node below it. */
+__global__ void k_lay_clear(LayoutArgs a)
 {
-	if (threadIdx.x != 0) return;
+	const int x = blockIdx.x * blockDim.x + threadIdx.x;
+	if (x >= a.nodeCount) return;
+	fld(a, F_WLEV, x) = -1;
+	if (x != 0) return;
 	fld(a, F_BASE, 0) = 0;
 	fld(a, F_S32, 0) = 0, fld(a, F_A32, 0) = 1;
 	const bool interior = a.nodes[0].count == 0;
 	fld(a, F_WLEV, 0) = (a.q8 && interior) ? 0 : -1;
 	fld(a, F_SQ8, 0) = 0, fld(a, F_AQ8, 0) = 1;
-	a.info[0] = a.q8 ? 1 : 0;   /* a root leaf counts as one level, as the traversal stack sizing assumes */
+	a.info->depthQ8 = a.q8 ? 1 : 0;   /* a root leaf counts as one level, as the traversal stack sizing assumes */
 }
 
-/* WLEV = -1 for every node below the root (the root kernel sets node 0 after). */
-__global__ void k_lay_clear(LayoutArgs a)
+__device__ __forceinline__ void lay_up1(const LayoutArgs& a, int x)
 {
-	const int x = blockIdx.x * blockDim.x + threadIdx.x;
-	if (x < a.nodeCount) fld(a, F_WLEV, x) = -1;
-}
-
-__global__ void __launch_bounds__(LBLOCK) k_lay_up1(LayoutArgs a, int b, int e)
-{
-	const int x = b + blockIdx.x * LBLOCK + threadIdx.x;
-	if (x >= e) return;
 	const BuildNode N = a.nodes[x];
 	if (N.count > 0) fld(a, F_TRI, x) = N.count, fld(a, F_N32, x) = 0;
 	else
@@ -102,10 +98,8 @@ __device__ __forceinline__ uint32_t leaf_ref(const LayoutArgs& a, const BuildNod
 	return a.leafRefMap ? (REF_LEAF | a.leafRefMap[a.prims[leaf.leftFirst]]) : (REF_LEAF | (uint32_t)base);
 }
 
-__global__ void __launch_bounds__(LBLOCK) k_lay_down1(LayoutArgs a, int b, int e)
+__device__ __forceinline__ void lay_down1(const LayoutArgs& a, int x)
 {
-	const int x = b + blockIdx.x * LBLOCK + threadIdx.x;
-	if (x >= e) return;
 	const BuildNode N = a.nodes[x];
 	const int base = fld(a, F_BASE, x);
 	if (N.count > 0)
@@ -172,13 +166,12 @@ __global__ void __launch_bounds__(LBLOCK) k_lay_down1(LayoutArgs a, int b, int e
 	bool any = false;
 	for (int j = 0; j < cnt; j++)
 		if (a.nodes[k[j]].count == 0) fld(a, F_WLEV, k[j]) = wl + 1, any = true;
-	if (any) atomicMax(&a.info[0], wl + 2);
+	if (any) atomicMax(&a.info->depthQ8, wl + 2);
 }
 
-__global__ void __launch_bounds__(LBLOCK) k_lay_up2(LayoutArgs a, int b, int e)
+__device__ __forceinline__ void lay_up2(const LayoutArgs& a, int x)
 {
-	const int x = b + blockIdx.x * LBLOCK + threadIdx.x;
-	if (x >= e || fld(a, F_WLEV, x) < 0) return;
+	if (fld(a, F_WLEV, x) < 0) return;
 	const int4 kv = a.kids[x];
 	const int k[4] = { kv.x, kv.y, kv.z, kv.w };
 	int size = 1;
@@ -258,10 +251,9 @@ hipError_t refit_layout(const BuildNode* dNodes, NodeF32* dF32, const int32_t* d
 	return hipGetLastError();
 }
 
-__global__ void __launch_bounds__(LBLOCK) k_lay_down2(LayoutArgs a, int b, int e)
+__device__ __forceinline__ void lay_down2(const LayoutArgs& a, int x)
 {
-	const int x = b + blockIdx.x * LBLOCK + threadIdx.x;
-	if (x >= e || fld(a, F_WLEV, x) < 0) return;
+	if (fld(a, F_WLEV, x) < 0) return;
 	const int4 kv = a.kids[x];
 	const int k[4] = { kv.x, kv.y, kv.z, kv.w };
 	int cnt = 0, ik = 0;
@@ -282,6 +274,26 @@ __global__ void __launch_bounds__(LBLOCK) k_lay_down2(LayoutArgs a, int b, int e
 		}
 		else refs[j] = REF_LEAF | (uint32_t)fld(a, F_BASE, k[j]);
 	}
+	a.q8[s].refs = make_uint4(refs[0], refs[1], refs[2], refs[3]);
+	if (a.q8Map)
+	{
+		a.q8Map[5 * s] = x;
+		for (int c = 0; c < 4; c++) a.q8Map[5 * s + 1 + c] = c < cnt ? k[c] : -1;
+	}
+}
+
+/* Quantised boxes of every 4-wide node, once their slots are known: no order
+ * between nodes, so one launch (inside the last pass, the double-precision
+ * rounding search of a few nodes per level set the pace of each level). */
+__global__ void __launch_bounds__(LBLOCK) k_lay_quantise(LayoutArgs a)
+{
+	const int x = blockIdx.x * LBLOCK + threadIdx.x;
+	if (x >= a.nodeCount || fld(a, F_WLEV, x) < 0) return;
+	const int4 kv = a.kids[x];
+	const int k[4] = { kv.x, kv.y, kv.z, kv.w };
+	int cnt = 0;
+	for (int j = 0; j < 4; j++)
+		if (k[j] >= 0) cnt = j + 1;
 	const BuildNode B = a.nodes[x];
 	uint32_t ex[3], q[6][4] = {};
 	for (int ax = 0; ax < 3; ax++)
@@ -291,16 +303,54 @@ __global__ void __launch_bounds__(LBLOCK) k_lay_down2(LayoutArgs a, int b, int e
 		ex[ax] = quantise_axis_dev(B.lo[ax], B.hi[ax], clo, chi, cnt, q[ax], q[3 + ax]);
 	}
 	auto pack = [](const uint32_t* v) { return v[0] | (v[1] << 8) | (v[2] << 16) | (v[3] << 24); };
-	NodeQ8 o;
+	NodeQ8& o = a.q8[fld(a, F_SQ8, x)];
 	o.origin = make_float4(B.lo[0], B.lo[1], B.lo[2], __uint_as_float(q8_step_bits(ex[2])));
 	o.qa = make_uint4(pack(q[0]), pack(q[1]), pack(q[2]), pack(q[3]));
 	o.qb = make_uint4(pack(q[4]), pack(q[5]), q8_step_bits(ex[0]), q8_step_bits(ex[1]));
-	o.refs = make_uint4(refs[0], refs[1], refs[2], refs[3]);
-	a.q8[s] = o;
-	if (a.q8Map)
+}
+
+enum { UP1, DOWN1, UP2, DOWN2 };
+template <int PASS> __device__ __forceinline__ void lay_node(const LayoutArgs& a, int x)
+{
+	if (PASS == UP1) lay_up1(a, x);
+	else if (PASS == DOWN1) lay_down1(a, x);
+	else if (PASS == UP2) lay_up2(a, x);
+	else lay_down2(a, x);
+}
+
+template <int PASS>
+__global__ void __launch_bounds__(LBLOCK) k_lay_level(LayoutArgs a, int b, int e)
+{
+	const int x = b + blockIdx.x * LBLOCK + threadIdx.x;
+	if (x < e) lay_node<PASS>(a, x);
+}
+
+template <int PASS>
+__global__ void __launch_bounds__(LEVELS_BLOCK) k_lay_levels(LayoutArgs a, LevelRange r)
+{
+	constexpr bool UP = PASS == UP1 || PASS == UP2;
+	for (int k = 0; k < r.n; k++)
 	{
-		a.q8Map[5 * s] = x;
-		for (int c = 0; c < 4; c++) a.q8Map[5 * s + 1 + c] = c < cnt ? k[c] : -1;
+		const int d = UP ? r.n - 1 - k : k;
+		for (int x = r.s[d] + (int)threadIdx.x; x < r.s[d + 1]; x += LEVELS_BLOCK) lay_node<PASS>(a, x);
+		__syncthreads();
+	}
+}
+
+template <int PASS>
+static void lay_pass(const LayoutArgs& a, const std::vector<int>& levelStart, hipStream_t stream)
+{
+	constexpr bool UP = PASS == UP1 || PASS == UP2;
+	const int levels = (int)levelStart.size() - 1;
+	for (int done = 0; done < levels;)
+	{
+		const LevelRange r = small_levels(levelStart, UP ? levels - done : done, !UP);
+		if (r.n > 1) k_lay_levels<PASS><<<1, LEVELS_BLOCK, 0, stream>>>(a, r), done += r.n;
+		else
+		{
+			const int d = UP ? levels - 1 - done : done, b = levelStart[d], e = levelStart[d + 1];
+			k_lay_level<PASS><<<(e - b + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a, b, e), done++;
+		}
 	}
 }
 
@@ -308,71 +358,46 @@ __global__ void k_lay_counts(LayoutArgs a)
 {
 	if (threadIdx.x != 0) return;
 	const bool interior = a.nodes[0].count == 0;
-	a.info[1] = interior ? fld(a, F_N32, 0) : 0;
-	a.info[2] = (interior && a.q8) ? fld(a, F_NQ8, 0) : 0;
+	a.info->nF32 = interior ? fld(a, F_N32, 0) : 0;
+	a.info->nQ8 = (interior && a.q8) ? fld(a, F_NQ8, 0) : 0;
+	a.info->root = a.nodes[0];
 }
 
-#define LCK(x) do { hipError_t e_ = (x); if (e_ != hipSuccess) { err = e_; goto done; } } while (0)
+/* Workspace: the counts first, then the per-node fields and the 4-wide children. */
+static const size_t LAY_HEAD = 256;
+size_t layout_workspace_bytes(int nodeCount, bool q8)
+{
+	return LAY_HEAD + (size_t)nodeCount * (sizeof(int) * F_COUNT + (q8 ? sizeof(int4) : 0)) + 64;
+}
 
 hipError_t layout_device(const BuildNode* dNodes, const uint32_t* dPrims, int nodeCount, const std::vector<int>& levelStart,
-	const uint32_t* leafRefMap, const LayoutOut& out, int* countsOut, hipStream_t stream)
+	const uint32_t* leafRefMap, const LayoutOut& out, void* ws, size_t wsBytes, hipStream_t stream)
 {
-	hipError_t err = hipSuccess;
-	int* f = nullptr;
-	int4* kids = nullptr;
-	int* info = nullptr;
-	const int levels = (int)levelStart.size() - 1;
-	if (nodeCount <= 0 || levels <= 0) return hipSuccess;
+	if (nodeCount <= 0 || levelStart.size() < 2) return hipSuccess;
+	if (!ws || wsBytes < layout_workspace_bytes(nodeCount, out.q8 != nullptr)) return hipErrorInvalidValue;
 	LayoutArgs a;
-	LCK(hipMalloc((void**)&f, sizeof(int) * (size_t)F_COUNT * nodeCount));
-	LCK(hipMalloc((void**)&info, sizeof(int) * 4));
-	if (out.q8) LCK(hipMalloc((void**)&kids, sizeof(int4) * (size_t)nodeCount));
-	a.nodes = dNodes, a.prims = dPrims, a.leafRefMap = leafRefMap, a.f = f, a.kids = kids, a.nodeCount = nodeCount;
-	a.f32 = out.f32, a.f32Kids = out.f32Kids, a.q8 = out.q8, a.q8Map = out.q8Map, a.order = out.order, a.last = out.last, a.info = info;
+	a.info = (LayoutCounts*)ws;
+	a.kids = out.q8 ? (int4*)((char*)ws + LAY_HEAD) : nullptr;
+	a.f = (int*)((char*)ws + LAY_HEAD + (out.q8 ? sizeof(int4) * (size_t)nodeCount : 0));
+	a.nodes = dNodes, a.prims = dPrims, a.leafRefMap = leafRefMap, a.nodeCount = nodeCount;
+	a.f32 = out.f32, a.f32Kids = out.f32Kids, a.q8 = out.q8, a.q8Map = out.q8Map, a.order = out.order, a.last = out.last;
 	k_lay_clear<<<(nodeCount + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a);
-	k_lay_root<<<1, 64, 0, stream>>>(a);
-	for (int d = levels - 1; d >= 0; d--)
-	{
-		const int b = levelStart[d], e = levelStart[d + 1];
-		k_lay_up1<<<(e - b + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a, b, e);
-	}
-	for (int d = 0; d < levels; d++)
-	{
-		const int b = levelStart[d], e = levelStart[d + 1];
-		k_lay_down1<<<(e - b + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a, b, e);
-	}
+	lay_pass<UP1>(a, levelStart, stream);
+	lay_pass<DOWN1>(a, levelStart, stream);
 	if (out.q8)
 	{
-		for (int d = levels - 1; d >= 0; d--)
-		{
-			const int b = levelStart[d], e = levelStart[d + 1];
-			k_lay_up2<<<(e - b + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a, b, e);
-		}
-		for (int d = 0; d < levels; d++)
-		{
-			const int b = levelStart[d], e = levelStart[d + 1];
-			k_lay_down2<<<(e - b + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a, b, e);
-		}
+		lay_pass<UP2>(a, levelStart, stream);
+		lay_pass<DOWN2>(a, levelStart, stream);
+		k_lay_quantise<<<(nodeCount + LBLOCK - 1) / LBLOCK, LBLOCK, 0, stream>>>(a);
 	}
 	k_lay_counts<<<1, 64, 0, stream>>>(a);
-	LCK(hipGetLastError());
-	if (countsOut)
-	{
-		int h[4];
-		LCK(hipMemcpyAsync(h, info, sizeof(h), hipMemcpyDeviceToHost, stream));
-		LCK(hipStreamSynchronize(stream));
-		countsOut[0] = h[1], countsOut[1] = h[2], countsOut[2] = h[0];
-	}
-done:
-	if (f || kids || info)
-	{
-		const hipError_t se = hipStreamSynchronize(stream);
-		if (err == hipSuccess) err = se;
-	}
-	if (f) (void)hipFree(f);
-	if (kids) (void)hipFree(kids);
-	if (info) (void)hipFree(info);
-	return err;
+	return hipGetLastError();
+}
+
+hipError_t layout_counts(const void* ws, LayoutCounts& out, hipStream_t stream)
+{
+	const hipError_t e = hipMemcpyAsync(&out, ws, sizeof(out), hipMemcpyDeviceToHost, stream);
+	return e != hipSuccess ? e : hipStreamSynchronize(stream);
 }
 
 __global__ void k_gather_tris(const float4* __restrict__ v, const uint32_t* __restrict__ order, const uint8_t* __restrict__ last, int n, float4* __restrict__ tris)

@@ -208,6 +208,7 @@ void RenderCore::Shutdown()
 	(void)hipStreamSynchronize(stream);
 	(void)hipStreamSynchronize(stream2);
 	meshes.clear();
+	buildWs.release();
 	tlasNodes.release(), instRecs.release(), shadeInsts.release(), overflow.release(), counters.release();
 	overflow2.release(), sideCounters.release();
 	materials.release(), triLights.release(), pointLights.release(), spotLights.release(), dirLights.release();
@@ -344,15 +345,15 @@ void RenderCore::buildMesh(MeshData& m)
 {
 	const auto t0 = std::chrono::high_resolution_clock::now();
 	const int n = m.triCount;
-	DevBuf lo, hi;
-	lo.ensure(sizeof(float4) * n), hi.ensure(sizeof(float4) * n);
-	hipCheck(tri_bounds(m.verts.as<float4>(), n, lo.as<float4>(), hi.as<float4>(), stream), "tri_bounds");
+	const size_t boxes = sizeof(float4) * (size_t)n, ws = gpu_build_workspace_bytes(n);
+	buildWs.ensure(2 * boxes + ws);
+	float4 *lo = buildWs.as<float4>(), *hi = lo + n;
+	hipCheck(tri_bounds(m.verts.as<float4>(), n, lo, hi, stream), "tri_bounds");
 	DeviceBuild b;
-	hipCheck(gpu_build(lo.as<float4>(), hi.as<float4>(), n, 4, 255, b, stream), "gpu_build");
-	lo.release(), hi.release();
-	m.dBuildNodes.release(), m.dBuildPrims.release();
-	m.dBuildNodes.p = b.nodes, m.dBuildNodes.bytes = sizeof(BuildNode) * (size_t)(2 * n);
-	m.dBuildPrims.p = b.prims, m.dBuildPrims.bytes = sizeof(uint32_t) * (size_t)n;
+	m.buildNodeCount = 0;
+	m.dBuildNodes.ensure(sizeof(BuildNode) * 2 * (size_t)n), m.dBuildPrims.ensure(sizeof(uint32_t) * (size_t)n);
+	b.nodes = m.dBuildNodes.as<BuildNode>(), b.prims = m.dBuildPrims.as<uint32_t>();
+	hipCheck(gpu_build(lo, hi, n, 4, 255, b, (char*)buildWs.p + 2 * boxes, ws, stream), "gpu_build");
 	m.buildNodeCount = b.nodeCount;
 	m.levelStart = b.levelStart;
 	m.buildDepth = b.depth;
@@ -367,18 +368,19 @@ void RenderCore::buildMesh(MeshData& m)
 	L.f32 = m.nodesF32.as<NodeF32>(), L.f32Kids = m.dF32Kids.as<int32_t>();
 	L.q8 = m.nodesQ8.as<NodeQ8>(), L.q8Map = m.dQ8Map.as<int32_t>();
 	L.order = m.dOrder.as<uint32_t>(), L.last = m.dLast.as<uint8_t>();
-	int counts[3];
-	hipCheck(layout_device(m.dBuildNodes.as<BuildNode>(), m.dBuildPrims.as<uint32_t>(), b.nodeCount, b.levelStart, nullptr, L, counts, stream), "bvh layout");
+	buildWs.ensure(layout_workspace_bytes(b.nodeCount, true));   /* the boxes and the builder's lists are no longer needed */
+	hipCheck(layout_device(b.nodes, b.prims, b.nodeCount, b.levelStart, nullptr, L, buildWs.p, buildWs.bytes, stream), "bvh layout");
 	m.tris.ensure(sizeof(float4) * 3 * ((size_t)n + TRACE_TRI_PAD));
 	hipCheck(gather_tris(m.verts.as<float4>(), m.dOrder.as<uint32_t>(), m.dLast.as<uint8_t>(), n, m.tris.as<float4>(), stream), "gather_tris");
-	BuildNode root;
-	hipCheck(hipMemcpyAsync(&root, m.dBuildNodes.p, sizeof(BuildNode), hipMemcpyDeviceToHost, stream), "D2H root");
-	hipCheck(hipStreamSynchronize(stream), "sync");
+	LayoutCounts counts;
+	hipCheck(layout_counts(buildWs.p, counts, stream), "bvh counts");
+	trimBuildWorkspace();
+	const BuildNode root = counts.root;
 	const bool rootLeaf = root.count > 0;
-	m.nodeCountF32 = (size_t)counts[0], m.nodeCountQ8 = (size_t)counts[1];
+	m.nodeCountF32 = (size_t)counts.nF32, m.nodeCountQ8 = (size_t)counts.nQ8;
 	m.rootF32 = rootLeaf ? REF_LEAF : 0u, m.rootQ8 = rootLeaf ? REF_LEAF : 0u;
 	m.depthF32 = b.depth, m.stackF32 = b.depth + 1;
-	m.depthQ8 = counts[2], m.stackQ8 = 3 * counts[2] + 1;
+	m.depthQ8 = counts.depthQ8, m.stackQ8 = 3 * counts.depthQ8 + 1;
 	m.leafCount = (size_t)(b.nodeCount + 1) / 2;
 	for (int c = 0; c < 3; c++) m.lo[c] = root.lo[c], m.hi[c] = root.hi[c];
 	const auto t1 = std::chrono::high_resolution_clock::now();
@@ -386,8 +388,13 @@ void RenderCore::buildMesh(MeshData& m)
 	stats.bvhBuildTime = m.buildMs * 0.001f;
 }
 
+void RenderCore::trimBuildWorkspace()
+{	/* the stream has passed every use */
+	if (buildWs.bytes > BUILD_WS_KEEP) buildWs.release();
+}
+
 /* Refit keeps the build tree's topology and recomputes its boxes from the new
- * vertices on the device: one launch per tree level from the deepest up (a
+ * vertices on the device, level by level from the deepest up (a
  * leaf box is the min / max of its triangles' vertices, as tri_bounds computes
  * them, an interior box the union of its two children), then the f32 and q8
  * nodes are rewritten from the refitted boxes through the layout maps and the
@@ -395,9 +402,7 @@ void RenderCore::buildMesh(MeshData& m)
 void RenderCore::refitMesh(MeshData& m)
 {
 	const auto t0 = std::chrono::high_resolution_clock::now();
-	for (int d = (int)m.levelStart.size() - 2; d >= 0; d--)
-		hipCheck(refit_level(m.dBuildNodes.as<BuildNode>(), m.dBuildPrims.as<uint32_t>(), m.verts.as<float4>(),
-			m.levelStart[d], m.levelStart[d + 1] - m.levelStart[d], stream), "refit_level");
+	hipCheck(refit_levels(m.dBuildNodes.as<BuildNode>(), m.dBuildPrims.as<uint32_t>(), m.verts.as<float4>(), m.levelStart, stream), "refit_levels");
 	hipCheck(refit_layout(m.dBuildNodes.as<BuildNode>(), m.nodesF32.as<NodeF32>(), m.dF32Kids.as<int32_t>(), (int)m.nodeCountF32,
 		m.nodesQ8.as<NodeQ8>(), m.dQ8Map.as<int32_t>(), (int)m.nodeCountQ8, stream), "refit_layout");
 	hipCheck(gather_tris(m.verts.as<float4>(), m.dOrder.as<uint32_t>(), m.dLast.as<uint8_t>(), m.triCount, m.tris.as<float4>(), stream), "gather_tris");
@@ -566,21 +571,26 @@ void RenderCore::updateTopLevel()
 	else if (!live.empty())
 	{
 		const int n = (int)live.size();
-		DevBuf dlo, dhi;
-		dlo.upload(blo.data(), n * sizeof(float4), stream);
-		dhi.upload(bhi.data(), n * sizeof(float4), stream);
-		DevBuf liveMap;
-		liveMap.upload(live.data(), n * sizeof(int), stream);
+		/* boxes and the map of live instances go up together, into the workspace */
+		std::vector<char> up((size_t)n * (2 * sizeof(float4) + sizeof(int)));
+		memcpy(up.data(), blo.data(), n * sizeof(float4)), memcpy(up.data() + n * sizeof(float4), bhi.data(), n * sizeof(float4));
+		memcpy(up.data() + 2 * n * sizeof(float4), live.data(), n * sizeof(int));
+		const size_t head = (up.size() + 255) & ~(size_t)255, nodes = sizeof(BuildNode) * (size_t)(2 * n), prims = (sizeof(uint32_t) * n + 255) & ~(size_t)255;
+		const size_t buildBytes = gpu_build_workspace_bytes(n), layBytes = layout_workspace_bytes(2 * n, false);
+		buildWs.ensure(head + nodes + prims + std::max(buildBytes, layBytes));
+		char* const w = (char*)buildWs.p;
+		hipCheck(hipMemcpyAsync(w, up.data(), up.size(), hipMemcpyHostToDevice, stream), "H2D");
+		const float4* lo = (const float4*)w;
 		DeviceBuild b;
-		hipCheck(gpu_build(dlo.as<float4>(), dhi.as<float4>(), n, 1, 1, b, stream), "tlas build");
+		b.nodes = (BuildNode*)(w + head), b.prims = (uint32_t*)(w + head + nodes);
+		void* const ws = w + head + nodes + prims;
+		hipCheck(gpu_build(lo, lo + n, n, 1, 1, b, ws, buildBytes, stream), "tlas build");
 		/* one instance per leaf: leaf refs point straight at the instance id */
 		tlasNodes.ensure(sizeof(NodeF32) * std::max(1, (b.nodeCount - 1) / 2));
 		LayoutOut L;
 		L.f32 = tlasNodes.as<NodeF32>();
-		const hipError_t e = layout_device(b.nodes, b.prims, b.nodeCount, b.levelStart, liveMap.as<uint32_t>(), L, nullptr, stream);
+		hipCheck(layout_device(b.nodes, b.prims, b.nodeCount, b.levelStart, (const uint32_t*)(lo + 2 * n), L, ws, layBytes, stream), "tlas layout");
 		const int depth = b.depth;
-		free_build(b);
-		hipCheck(e, "tlas layout");
 		scene.twoLevel = 1;
 		scene.tlas = tlasNodes.as<NodeF32>();
 		scene.tlasRoot = n == 1 ? (REF_LEAF | (uint32_t)live[0]) : 0u;
@@ -588,6 +598,7 @@ void RenderCore::updateTopLevel()
 	}
 	if (scene.maxStack > TRACE_MAX_STACK) throw CoreError(LH2HIP_ERR_INVALID, "BVH too deep for the traversal stack");
 	hipCheck(hipStreamSynchronize(stream), "sync");
+	trimBuildWorkspace();
 	instancesDirty = false;
 }
 

@@ -227,6 +227,11 @@ private:
 	/* top level */
 	DevBuf tlasNodes, instRecs, shadeInsts;
 	TraceScene scene;
+	/* workspace of builds and layouts, kept between calls up to BUILD_WS_KEEP
+	 * bytes (a mesh of about 1.2 M triangles); used under the scene lock, on `stream` */
+	DevBuf buildWs;
+	static constexpr size_t BUILD_WS_KEEP = (size_t)256 << 20;
+	void trimBuildWorkspace();
 	/* trace scratch (overflow2 / sideCounters: the shadow-ray lane) */
 	DevBuf overflow, counters, overflow2, sideCounters;
 	hipStream_t stream2 = nullptr;
