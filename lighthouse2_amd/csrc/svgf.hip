@@ -5,9 +5,11 @@
  * sampling_shared.h:111-115,136-220, in the reference's operation order.
  * Two library calls are replaced by functions of our own so that the CPU
  * oracle reproduces every value bit for bit: powf(x, 128) is x squared seven
- * times, and __expf is cw_expf (lh_math.h). One pixel per thread, 8x8 blocks.
+ * times, and __expf is cw_expf (lh_math.h). One pixel per thread, 8x8 blocks
+ * (the a-trous passes: 16 x 16 lattices).
  */
 #include "svgf.h"
+#include <type_traits>
 #include "lh_math.h"
 #include "../../include/lh2hip.h"
 
@@ -75,26 +77,26 @@ __device__ __forceinline__ float clampf(float v, float a, float b) { return fmax
 /* ReadWorldPos (sampling_shared.h:111-115) */
 __device__ __forceinline__ float4 read_world_pos(const float4* buf, int x, int y, int w, int h)
 {
-	if (x >= 0 && y >= 0 && x < w && y < h) return buf[x + y * w];
-	return make_float4(1e20f, 1e20f, 1e20f, bitsf(0u));
+	/* loaded at a clamped address and replaced outside, so that a caller's loads are in flight together */
+	const float4 p = buf[min(max(x, 0), w - 1) + min(max(y, 0), h - 1) * w];
+	return x >= 0 && y >= 0 && x < w && y < h ? p : make_float4(1e20f, 1e20f, 1e20f, bitsf(0u));
 }
 
-__device__ float world_distance(int px, int py, float4 cur, const float4* prev, int w, int h)
+__device__ __forceinline__ float world_distance(float4 p, float4 cur)
 {
-	const float4 p = read_world_pos(prev, px, py, w, h);
 	const v3 ln = unpack_normal2(fbits(cur.w)), pn = unpack_normal2(fbits(p.w));
-	if ((fbits(p.w) & 3u) != 1u) return 1e21f;
-	if (dot(ln, pn) < 0.85f) return 1e21f;
-	return length(mk3(cur.x - p.x, cur.y - p.y, cur.z - p.z));
+	const float d = length(mk3(cur.x - p.x, cur.y - p.y, cur.z - p.z));
+	return (fbits(p.w) & 3u) != 1u || dot(ln, pn) < 0.85f ? 1e21f : d;
 }
 
-__device__ float fine_world_distance(f2 pixel, float4 cur, const float4* prev, int w, int h)
+__device__ __forceinline__ float fine_world_distance(f2 pixel, float4 cur, const float4* prev, int w, int h)
 {
 	const int p0x = f2i_sat(pixel.x), p0y = f2i_sat(pixel.y);
 	const float fx = pixel.x - floorf(pixel.x), fy = pixel.y - floorf(pixel.y);
 	const float w0 = (1 - fx) * (1 - fy), w1 = fx * (1 - fy), w2 = (1 - fx) * fy, w3 = fx * fy;
-	const float d0 = world_distance(p0x, p0y, cur, prev, w, h), d1 = world_distance(p0x + 1, p0y, cur, prev, w, h);
-	const float d2 = world_distance(p0x, p0y + 1, cur, prev, w, h), d3 = world_distance(p0x + 1, p0y + 1, cur, prev, w, h);
+	const float4 q0 = read_world_pos(prev, p0x, p0y, w, h), q1 = read_world_pos(prev, p0x + 1, p0y, w, h);
+	const float4 q2 = read_world_pos(prev, p0x, p0y + 1, w, h), q3 = read_world_pos(prev, p0x + 1, p0y + 1, w, h);
+	const float d0 = world_distance(q0, cur), d1 = world_distance(q1, cur), d2 = world_distance(q2, cur), d3 = world_distance(q3, cur);
 	float tw = 0, td = 0;
 	if (d0 < 1e20f) td += d0 * w0, tw += w0;
 	if (d1 < 1e20f) td += d1 * w1, tw += w1;
@@ -107,9 +109,13 @@ __device__ int refine_history_pos(f2& pos, f2 off, float4 cur, float& best, floa
 {
 	int tap = 0;
 	const f2 c[4] = { { pos.x - step, pos.y }, { pos.x + step, pos.y }, { pos.x, pos.y - step }, { pos.x, pos.y + step } };
+	float d4[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++) d4[i] = fine_world_distance(f2{ c[i].x + off.x, c[i].y + off.y }, cur, prev, w, h);
+#pragma unroll
 	for (int i = 0; i < 4; i++)
 	{
-		const float d = fine_world_distance(f2{ c[i].x + off.x, c[i].y + off.y }, cur, prev, w, h);
+		const float d = d4[i];
 		if (d < best) best = d, pos = c[i], tap = i + 1;
 	}
 	return tap;
@@ -246,92 +252,155 @@ __global__ void k_prepare(const float4* __restrict__ acc, const uint4* __restric
 	moments[p] = make_float4(lumD, lumD2, lumI, lumI2);
 }
 
-/* applyFilterKernel (finalize_shared.h:320-477) */
-__global__ void k_apply(const uint4* __restrict__ features, const float4* __restrict__ prevWorldPos, const float4* __restrict__ worldPos,
-	const float4* __restrict__ deltaDepth, const float2* __restrict__ motion, const float4* __restrict__ moments,
-	const float4* __restrict__ A, const float4* __restrict__ B, float4* __restrict__ C, int w, int h, int phase, int lastPass)
+/* n / d by the operations that the compiler emits for a correctly rounded
+ * division, without the scaling and the fix-up: the same bits for d in
+ * [1e-5, 1e30] except where n / d overflows (NaN here) or n is close to
+ * denormal (an ulp), and a tap's weight is the same 0, or unchanged, in both. */
+__device__ __forceinline__ float div_core(float n, float d)
 {
-	const int x = blockIdx.x * blockDim.x + threadIdx.x, y = blockIdx.y * blockDim.y + threadIdx.y;
+	const float r0 = __builtin_amdgcn_rcpf(d);
+	const float r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
+	const float q0 = n * r;
+	const float q1 = fmaf(fmaf(-d, q0, n), r, q0);
+	return fmaf(fmaf(-d, q1, n), r, q1);
+}
+
+/* cw_expf for x <= 0 or NaN (its scale by ldexp: the same rounding) */
+__device__ __forceinline__ float exp_neg(float x)
+{
+	const float k = floorf(fmaf(x, 1.44269504f, 0.5f));
+	const float r = fmaf(k, 2.12194440e-4f, fmaf(-k, 0.693359375f, x));
+	float p = fmaf(r, 1.9841270e-4f, 1.3888889e-3f);
+	p = fmaf(p, r, 8.3333333e-3f);
+	p = fmaf(p, r, 4.1666668e-2f);
+	p = fmaf(p, r, 0.16666667f);
+	p = fmaf(p, r, 0.5f);
+	p = fmaf(p, r, 1.0f);
+	p = fmaf(p, r, 1.0f);
+	return x < -87.0f ? 0.0f : ldexpf(p, (int)k);
+}
+
+/* applyFilterKernel (finalize_shared.h:320-477), pass with tap distance STEP.
+ *
+ * VALU-bound: 20 taps per pixel, each of which unpacked two colours, a normal and
+ * an albedo, two luminances, a division and two exponentials. A block stages
+ * the pixels it needs in LDS, decoded once (64 B: colours with their luminances,
+ * normal with depth, albedo with material), and a tap is four 16-byte LDS reads
+ * and about half the instructions. The taps of a pixel lie STEP apart, so a
+ * block owns a 16 x 16 lattice of that spacing (one of the STEP^2 of a 16 STEP
+ * square) and stages 20 x 20 pixels whatever the distance: 25.6 KB, where the
+ * square of the last pass would need 64 KB. Lattices that share cache lines (same
+ * rows) run one after the other on one XCD (blocks are dealt to the 8 XCDs round
+ * robin). A 1920 x 1080 pass takes 111 us (the first, with its history, 161), of
+ * which VALU issue is 95; it was 187 to 288 us with every tap read and decoded
+ * from memory. */
+template <int STEP, bool LAST>
+__global__ void __launch_bounds__(256) k_apply(const uint4* __restrict__ features, const float4* __restrict__ prevWorldPos, const float4* __restrict__ worldPos,
+	const float4* __restrict__ deltaDepth, const float2* __restrict__ motion, const float4* __restrict__ moments,
+	const float4* __restrict__ A, const float4* __restrict__ B, float4* __restrict__ C, int w, int h)
+{
+	constexpr int T = 16, TW = T + 4, PHASE = STEP == 1 ? 1 : STEP == 2 ? 2 : 3;
+	__shared__ float4 tile[4][TW * TW];
+	const int tilesX = (w + T * STEP - 1) / (T * STEP), tilesY = (h + T * STEP - 1) / (T * STEP);
+	const int b = blockIdx.x, k = b >> 3, m = (k / STEP) * 8 + (b & 7);
+	if (m >= tilesX * tilesY * STEP) return;
+	const int rx = k % STEP, ry = m % STEP, t = m / STEP;
+	const int x0 = (t % tilesX) * (T * STEP) + rx, y0 = (t / tilesX) * (T * STEP) + ry;
+	for (int i = threadIdx.x; i < TW * TW; i += 256)
+	{
+		const int px = min(max(x0 + (i % TW - 2) * STEP, 0), w - 1), py = min(max(y0 + (i / TW - 2) * STEP, 0), h - 1);   /* rows outside are not read */
+		const float4 c = A[px + py * w];
+		const uint4 f = features[px + py * w];
+		const v3 d = get_direct(c), in = get_indirect(c), n = unpack_normal2(f.y), a = rgb32_to_hdr(f.x);
+		tile[0][i] = make_float4(d.x, d.y, d.z, luminance(d));
+		tile[1][i] = make_float4(in.x, in.y, in.z, luminance(in));
+		tile[2][i] = make_float4(n.x, n.y, n.z, bitsf(f.z));
+		tile[3][i] = make_float4(a.x, a.y, a.z, bitsf(f.w));
+	}
+	__syncthreads();
+	const int lx = threadIdx.x % T, ly = threadIdx.x / T, x = x0 + lx * STEP, y = y0 + ly * STEP;
 	if (x >= w || y >= h) return;
-	const int p = x + y * w;
-	const uint4 lf = features[p];
-	const float4 lpos = worldPos[p];
-	const v3 ln = unpack_normal2(lf.y), lc = rgb32_to_hdr(lf.x);
-	const uint32_t lmat = lf.w >> 4;
+	const int p = x + y * w, me = (ly + 2) * TW + lx + 2;
+	const float4 c0 = tile[0][me], c1 = tile[1][me], c2 = tile[2][me], c3 = tile[3][me];
+	const v3 ln = xyz(c2), lc = xyz(c3);
+	const uint32_t lmat = fbits(c3.w) >> 4;
 	float dws = 1, iws = 1;
-	const float4 comb = A[p];
-	v3 dsum = get_direct(comb) * dws, isum = get_indirect(comb) * iws;
-	const float lD = luminance(get_direct(comb)), lI = luminance(get_indirect(comb));
-	const float ldepth = bitsf(lf.z), ddx = deltaDepth[p].z, ddy = deltaDepth[p].w;
-	const float sigma = 10.0f * bitsf((uint32_t)(127 - (phase - 1)) << 23);
-	const float factor = (lf.w & 15u) == 0 ? 400.0f : 1.0f;
-	const float4 m = moments[p];
-	const float varD = m.y - m.x * m.x, varI = m.w - m.z * m.z;
+	v3 dsum = xyz(c0) * dws, isum = xyz(c1) * iws;
+	const float lD = c0.w, lI = c1.w;
+	const float4 dd = deltaDepth[p];
+	const float ldepth = c2.w, ddx = dd.z, ddy = dd.w;
+	const float sigma = 10.0f * bitsf((uint32_t)(127 - (PHASE - 1)) << 23);
+	const float factor = (fbits(c3.w) & 15u) == 0 ? 400.0f : 1.0f;
+	const float4 mo = moments[p];
+	const float varD = mo.y - mo.x * mo.x, varI = mo.w - mo.z * mo.z;
 	const float rD = -1.0f / (sigma * factor * sqrtf(varD + 0.00001f) + 0.00001f);
 	const float rI = -1.0f / (sigma * factor * sqrtf(varI + 0.00001f) + 0.00001f);
-	const int step = 1 << (phase - 1);
-	for (int vv = -2; vv <= 2; vv++)
-	{
-		const int v = vv * step + y;
-		const int r = (vv == 2 || vv == -2) ? 1 : 2;
-		if (v < 0 || v >= h) continue;
-		for (int uu = -r; uu <= r; uu++)
+	const auto taps = [&](auto exact) {
+#pragma unroll
+		for (int vv = -2; vv <= 2; vv++)
 		{
-			if (uu == 0 && vv == 0) continue;
-			const int u = min(max(uu * step + x, 0), w - 1);
-			const int q = u + v * w;
-			const float4 c = A[q];
-			const uint4 nf = features[q];
-			const float wdist = (float)(uu * uu + vv * vv) * (-1.0f / 7.5f);
-			const v3 nd = get_direct(c), ni = get_indirect(c), nn = unpack_normal2(nf.y);
-			float wn = pow128(fmaxf(0.0f, fdot(nn, ln)));
-			const float expected = fmaf(ddy, (float)(vv * step), fmaf(ddx, (float)(uu * step), ldepth));
-			const float err = fabsf(expected - bitsf(nf.z));
-			const float expDiff = fabsf(expected - ldepth);
-			const float wdepth = err / fmaxf(0.00001f, (0.5f + (float)phase * 0.5f) * expDiff);
-			if ((nf.w >> 4) != lmat) wn = (float)((double)wn * 0.0001);
-			else wn = wn * fdot(lc, rgb32_to_hdr(nf.x));
-			float wd = wn * cw_expf(fmaf(fabsf(lD - luminance(nd)), rD, wdist) - wdepth);
-			float wi = wn * cw_expf(fmaf(fabsf(lI - luminance(ni)), rI, wdist) - wdepth);
-			if (!__builtin_isfinite(wd)) wd = 0;
-			if (!__builtin_isfinite(wi)) wi = 0;
-			dsum = mk3(fmaf(nd.x, wd, dsum.x), fmaf(nd.y, wd, dsum.y), fmaf(nd.z, wd, dsum.z)), dws += wd;
-			isum = mk3(fmaf(ni.x, wi, isum.x), fmaf(ni.y, wi, isum.y), fmaf(ni.z, wi, isum.z)), iws += wi;
+			const int v = vv * STEP + y, r = (vv == 2 || vv == -2) ? 1 : 2;
+			if (v < 0 || v >= h) continue;
+#pragma unroll
+			for (int uu = -2; uu <= 2; uu++)
+			{
+				if (uu < -r || uu > r || (uu == 0 && vv == 0)) continue;
+				const int q = me + vv * TW + uu;
+				const float4 q0 = tile[0][q], q1 = tile[1][q], q2 = tile[2][q], q3 = tile[3][q];
+				const float wdist = (float)(uu * uu + vv * vv) * (-1.0f / 7.5f);
+				float wn = pow128(fmaxf(0.0f, fdot(xyz(q2), ln)));
+				const float expected = fmaf(ddy, (float)(vv * STEP), fmaf(ddx, (float)(uu * STEP), ldepth));
+				const float err = fabsf(expected - q2.w);
+				const float expDiff = fabsf(expected - ldepth);
+				const float den = fmaxf(0.00001f, (0.5f + (float)PHASE * 0.5f) * expDiff);
+				const float wdepth = decltype(exact)::value ? err / den : div_core(err, den);
+				if ((fbits(q3.w) >> 4) != lmat) wn = (float)((double)wn * 0.0001);
+				else wn = wn * fdot(lc, xyz(q3));
+				float wd = wn * exp_neg(fmaf(fabsf(lD - q0.w), rD, wdist) - wdepth);
+				float wi = wn * exp_neg(fmaf(fabsf(lI - q1.w), rI, wdist) - wdepth);
+				if (!__builtin_isfinite(wd)) wd = 0;
+				if (!__builtin_isfinite(wi)) wi = 0;
+				dsum = mk3(fmaf(q0.x, wd, dsum.x), fmaf(q0.y, wd, dsum.y), fmaf(q0.z, wd, dsum.z)), dws += wd;
+				isum = mk3(fmaf(q1.x, wi, isum.x), fmaf(q1.y, wi, isum.y), fmaf(q1.z, wi, isum.z)), iws += wi;
+			}
 		}
-	}
+	};
+	/* a denominator is at most 4 STEP (|ddx| + |ddy|) and a rounding of the depth: beyond 1e30 the division as written */
+	const bool tame = (float)(8 * STEP) * (fabsf(ddx) + fabsf(ddy)) + fabsf(ldepth) * 1.0e-4f < 1.0e30f;
+	if (__all(tame)) taps(std::false_type());
+	else taps(std::true_type());
 	v3 df = dsum * (1.0f / fmaxf(0.0001f, dws));
 	v3 inf = isum * (1.0f / fmaxf(0.0001f, iws));
-	if (phase == 1)
+	if (STEP == 1)
 	{
 		const float2 mv = motion[p];
 		const int px = f2i_sat(mv.x), py = f2i_sat(mv.y);
 		if (px >= 0 && px < w && py >= 0 && py < h)
 		{
 			v3 pd, pi;
-			read_texel_consistent2(B, prevWorldPos, lpos, ln, mv.x, mv.y, w, h, pd, pi);
+			read_texel_consistent2(B, prevWorldPos, worldPos[p], ln, mv.x, mv.y, w, h, pd, pi);
 			if (pd.x != -1)
 			{
 				pd = rgb_to_ycocg(pd), pi = rgb_to_ycocg(pi);
 				v3 dAvg = rgb_to_ycocg(df), dVar = dAvg * dAvg;
 				v3 iAvg = rgb_to_ycocg(inf), iVar = iAvg * iAvg;
 				const auto add = [&](int q) {
-					const float4 c4 = A[q];
-					const v3 f = rgb_to_ycocg(get_direct(c4)), g = rgb_to_ycocg(get_indirect(c4));
+					const v3 f = rgb_to_ycocg(xyz(tile[0][q])), g = rgb_to_ycocg(xyz(tile[1][q]));
 					dAvg = dAvg + f, dVar = dVar + f * f, iAvg = iAvg + g, iVar = iVar + g * g;
 				};
 				if (x > 1)
 				{
-					if (y > 1) add(p - w - 1);
-					add(p - 1);
-					if (y < h - 1) add(p + w - 1);
+					if (y > 1) add(me - TW - 1);
+					add(me - 1);
+					if (y < h - 1) add(me + TW - 1);
 				}
-				if (y > 1) add(p - w);
-				if (y < h - 1) add(p + w);
+				if (y > 1) add(me - TW);
+				if (y < h - 1) add(me + TW);
 				if (x < w - 1)
 				{
-					if (y > 1) add(p + 1 - w);
-					add(p + 1);
-					if (y < h - 1) add(p + 1 + w);
+					if (y > 1) add(me + 1 - TW);
+					add(me + 1);
+					if (y < h - 1) add(me + 1 + TW);
 				}
 				dAvg = dAvg * (1.0f / 9.0f), dVar = dVar * (1.0f / 9.0f), iAvg = iAvg * (1.0f / 9.0f), iVar = iVar * (1.0f / 9.0f);
 				const v3 sd0 = dVar - dAvg * dAvg, si0 = iVar - iAvg * iAvg;
@@ -345,9 +414,9 @@ __global__ void k_apply(const uint4* __restrict__ features, const float4* __rest
 			}
 		}
 	}
-	if (lastPass)
+	if (LAST)
 	{
-		const v3 c = (df + inf) * rgb32_to_hdr(lf.x);
+		const v3 c = (df + inf) * lc;
 		C[p] = make_float4(sqrtf(c.x), sqrtf(c.y), sqrtf(c.z), 1);
 	}
 	else C[p] = combine(df, inf);
@@ -368,17 +437,28 @@ __device__ v3 read_texel_mitchell(const float4* buf, float u, float v, int w, in
 {
 	const int x1 = f2i_sat(u - 2.0f), y1 = f2i_sat(v - 2.0f);
 	float tw = 0;
-	float4 t = make_float4(0, 0, 0, 0);
-	for (int y = y1; y < y1 + 4; y++)
-		for (int x = x1; x < x1 + 4; x++)
-			if (x >= 0 && y > 0 && x < w && y < h)
-			{
-				const float dx = (float)x - u, dy = (float)y - v;
-				const float wt = mitchell_netravali(dx) * mitchell_netravali(dy);
-				const float4 b = buf[x + y * w];
-				t = make_float4(t.x + b.x * wt, t.y + b.y * wt, t.z + b.z * wt, t.w + b.w * wt);
-				tw += wt;
-			}
+	v3 t = mk3(0, 0, 0);
+	float wx[4];                     /* a column's factor, once for its four rows */
+#pragma unroll
+	for (int i = 0; i < 4; i++) wx[i] = mitchell_netravali((float)(x1 + i) - u);
+#pragma unroll
+	for (int j = 0; j < 4; j++)
+	{
+		const int y = y1 + j;
+		const float wy = mitchell_netravali((float)y - v);
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+		{
+			/* every tap's load is issued (at a clamped address) and the ones outside dropped afterwards: with a
+			 * branch around each, the 16 loads waited for one another */
+			const int x = x1 + i;
+			const bool in = x >= 0 && y > 0 && x < w && y < h;
+			const float wt = wx[i] * wy;
+			const float4 b = buf[min(max(x, 0), w - 1) + min(max(y, 0), h - 1) * w];
+			t = in ? mk3(t.x + b.x * wt, t.y + b.y * wt, t.z + b.z * wt) : t;
+			tw = in ? tw + wt : tw;
+		}
+	}
 	const float r = 1.0f / tw;
 	return mk3(t.x * r, t.y * r, t.z * r);
 }
@@ -402,24 +482,16 @@ __global__ void k_taa(const float4* __restrict__ px, const float4* __restrict__ 
 		const v3 np = rgb_to_ycocg(pixel);
 		v3 hist = rgb_to_ycocg(read_texel_mitchell(prevPixels, ux, uy, w, h));
 		v3 avg = np, var = np * np;
-		const auto add = [&](int q) {
-			const v3 f = rgb_to_ycocg(mk3(px[q].x, px[q].y, px[q].z));
-			avg = avg + f, var = var + f * f;
+		/* the neighbours, in the order left column, above, below, right column; loaded as above */
+		const auto add = [&](int dx, int dy, bool in) {
+			const float4 q = px[min(max(x + dx, 0), w - 1) + min(max(y + dy, 0), h - 1) * w];
+			const v3 f = rgb_to_ycocg(xyz(q));
+			avg = in ? avg + f : avg, var = in ? var + f * f : var;
 		};
-		if (x > 1)
-		{
-			if (y > 1) add(p - w - 1);
-			add(p - 1);
-			if (y < h - 1) add(p + w - 1);
-		}
-		if (y > 1) add(p - w);
-		if (y < h - 1) add(p + w);
-		if (x < w - 1)
-		{
-			if (y > 1) add(p + 1 - w);
-			add(p + 1);
-			if (y < h - 1) add(p + 1 + w);
-		}
+		const bool up = y > 1, down = y < h - 1, left = x > 1, right = x < w - 1;
+		add(-1, -1, left && up), add(-1, 0, left), add(-1, 1, left && down);
+		add(0, -1, up), add(0, 1, down);
+		add(1, -1, right && up), add(1, 0, right), add(1, 1, right && down);
 		avg = avg * (1.0f / 9.0f), var = var * (1.0f / 9.0f);
 		const v3 s0 = var - avg * avg;
 		const v3 sg = mk3(sqrtf(fmaxf(0.0f, s0.x)), sqrtf(fmaxf(0.0f, s0.y)), sqrtf(fmaxf(0.0f, s0.z)));
@@ -522,13 +594,15 @@ void Svgf::Frame(const float4* acc, const uint4* feat, const float4* wp, const f
 	k_prepare<<<g, b, 0, s>>>(acc, feat, features.as<uint4>(), wp, worldPos.as<float4>(), prevWorldPos.as<float4>(), shading.as<float4>(),
 		motion.as<float2>(), moments.as<float4>(), prevMoments.as<float4>(), cam, j0, j1, pj0, pj1, w, h, 1.0f / (float)samplesTaken, clampD,
 		clampI, stationary);
-	const auto apply = [&](int phase, DevBuf& A, const float4* B, DevBuf& C, int last) {
-		k_apply<<<g, b, 0, s>>>(features.as<uint4>(), prevWorldPos.as<float4>(), wp, dd, motion.as<float2>(),
-			moments.as<float4>(), A.as<float4>(), B, C.as<float4>(), w, h, phase, last);
+	const auto apply = [&](auto step, DevBuf& A, const float4* B, DevBuf& C) {
+		constexpr int STEP = decltype(step)::value;
+		const int lattices = ((w + 16 * STEP - 1) / (16 * STEP)) * ((h + 16 * STEP - 1) / (16 * STEP)) * STEP;   /* and STEP in x */
+		k_apply<STEP, STEP == 4><<<(lattices + 7) / 8 * 8 * STEP, 256, 0, s>>>(features.as<uint4>(), prevWorldPos.as<float4>(), wp, dd, motion.as<float2>(),
+			moments.as<float4>(), A.as<float4>(), B, C.as<float4>(), w, h);
 	};
-	apply(1, shading, filteredIn.as<float4>(), filteredOut, 0);
-	apply(2, filteredOut, nullptr, filteredIn, 0);
-	apply(3, filteredIn, nullptr, lastPass, 1);
+	apply(std::integral_constant<int, 1>(), shading, filteredIn.as<float4>(), filteredOut);
+	apply(std::integral_constant<int, 2>(), filteredOut, nullptr, filteredIn);
+	apply(std::integral_constant<int, 4>(), filteredIn, nullptr, lastPass);
 	if (taa)
 	{	/* TAApass + unsharpenTAA (rendercore.cpp:922-926); the TAA output is the next frame's history */
 		k_taa<<<g, b, 0, s>>>(lastPass.as<float4>(), prevPixels.as<float4>(), motion.as<float2>(), w, h, taaOut.as<float4>());
