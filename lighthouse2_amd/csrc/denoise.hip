@@ -27,22 +27,20 @@ typedef short s4v __attribute__((__vector_size__(4 * sizeof(short))));
 typedef float f4v __attribute__((__vector_size__(4 * sizeof(float))));
 
 __device__ __forceinline__ float bf2f(bf16_t b) { return __builtin_bit_cast(float, (uint32_t)b << 16); }
-/* round to nearest even; NaN stays a quiet NaN */
-__device__ __forceinline__ bf16_t f2bf(float f)
+/* round to nearest even, NaN stays a quiet NaN: v_cvt_pk_bf16_f32, whose result equals the
+ * integer formula's for all 2^32 inputs (six instructions per value before) */
+__device__ __forceinline__ bf16_t f2bf(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
+__device__ __forceinline__ uint32_t pack_bf(float lo, float hi)
 {
-	const uint32_t u = __builtin_bit_cast(uint32_t, f);
-	if ((u & 0x7fffffffu) > 0x7f800000u) return (bf16_t)((u >> 16) | 0x40u);
-	return (bf16_t)((u + 0x7fffu + ((u >> 16) & 1u)) >> 16);
+	typedef __bf16 bf2v __attribute__((ext_vector_type(2)));
+	const bf2v v = { (__bf16)lo, (__bf16)hi };
+	return __builtin_bit_cast(uint32_t, v);
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 static bool aligned16_3(const void* a, const void* b, const void* c) { return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15) == 0; }
 
 static const int DW_BLOCKS = 512;
-
-/* Rows per block of the forward / input-gradient convolution's tiles on
- * large images (a wave per row, 64 pixels wide). */
-static constexpr int TILE_ROWS = 8;
 
 /* ---- 3x3 convolution, forward and input gradient ------------------------ */
 template <int NB, bool RELU, bool F32OUT>
@@ -102,22 +100,6 @@ __global__ void __launch_bounds__(256) k_conv3x3(const bf16_t* __restrict__ x, i
 	}
 }
 
-/* Tiled variant for the network's shapes: a block of ROWS waves computes
- * ROWS rows x 16 MBW pixels (one row per wave; 8 x 64 on large images, 4 x 64
- * with 64 input channels, 4 x 16 on small ones). The (ROWS + 2) x (16 MBW + 2)
- * pixel input halo is staged once
- * in LDS with 16-byte loads, all of a thread's loads in flight together, CP
- * channels per pixel (8 of padding against bank conflicts). Each wave then
- * runs the 9 taps as v_mfma_f32_16x16x32_bf16 products with
- * A = 16 output channels x 32 input channels of the [tap][Cout][Cin] weights
- * (read from memory one tap ahead of their use) and B = 32 input channels x
- * 16 pixels from LDS (lane: pixel lane % 16, channels 8 (lane / 16) + 0..7);
- * D then gives each lane 4 consecutive output channels of one pixel; bf16
- * outputs pair channel blocks across lanes for 16-byte writes (below).
- * CIN = 16 is padded to K = 32 with zero channels. CAT: the input is the
- * 64-channel concatenation [nearest 2x upsample of coarse (32 channels),
- * x (32 channels)]; the coarse pixels under the tile (and their halo) are staged
- * separately and upsampled by the fragment addressing. */
 /* Decoders of the SVGF feature words (tools_shared.h:130-136,169-176):
  * albedo HDRtoRGB32 (10:11:11), normal PackNormal2, depth as float bits. */
 __device__ __forceinline__ float3 feat_albedo(uint32_t c)
@@ -168,11 +150,284 @@ __device__ __forceinline__ uint32_t relu_mask2(uint32_t act, uint32_t g)
 	return (bf2f((bf16_t)(act & 0xffffu)) > 0.0f ? g & 0xffffu : 0u) | (bf2f((bf16_t)(act >> 16)) > 0.0f ? g & 0xffff0000u : 0u);
 }
 
-template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL = false, int MBW = 4, int ROWS = 4, int IO = IO_NONE>
-__global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restrict__ x, const bf16_t* __restrict__ coarse,
+/* Tiled variants for the network's shapes (k_conv3x3_t for small images, k_conv_rows
+ * for large ones). A block's pixels and their halo are staged once in LDS with
+ * 16-byte loads, a thread's loads in flight together, CP channels per pixel (8 of
+ * padding against bank conflicts). The 9 taps run as v_mfma_f32_16x16x32_bf16
+ * products with A = 16 output channels x 32 input channels of the [tap][Cout][Cin]
+ * weights and B = 32 input channels x 16 pixels from LDS (lane: pixel lane % 16,
+ * channels 8 (lane / 16) + 0..7); D then gives each lane 4 consecutive output
+ * channels of one pixel; bf16 outputs pair channel blocks across lanes for 16-byte
+ * writes (below). CIN = 16 is padded to K = 32 with zero channels. CAT: the input is
+ * the 64-channel concatenation [nearest 2x upsample of coarse (32 channels),
+ * x (32 channels)]; the coarse pixels under the tile (and their halo) are staged
+ * separately and upsampled by the fragment addressing. */
+
+/* Large images: a wave computes 4 rows x 16 MBW pixels, a block's four waves a
+ * tile of 16 MBW x 16, staged as above (18 of 16 rows are read; 8 x 64 tiles, 10
+ * of 8). All nine taps' weight fragments sit in registers before the products
+ * start, and an input row's fragment, read from LDS once per horizontal shift,
+ * serves the up to three output rows it touches: 36 LDS reads for 144 products at
+ * 32 -> 32 channels. (With a wave per row 36 reads served 72 products, and every
+ * wave fetched every weight through L1 as it went, more bytes than the tile's own,
+ * waiting at each tap.) A row's sums run over the taps in the same order, so the
+ * results are those of the 16-pixel tiles bit for bit.
+ *   LOOP, for 64 channels: the weights are 147 KB a block and 144 registers a lane,
+ * so two blocks a CU stay and walk their XCD's tiles with them, one block's loads
+ * under the other's products (a block per tile: 121 us for the decoder's first
+ * convolution at 1920 x 1088, 100 -> 151 us for its gradient). With fewer weights
+ * three blocks a CU hide the loads better than a loop does.
+ *   Measured at 1920 x 1088 (a wave per row -> now; the bytes each must move at a
+ * copy's 5.06 TB/s): 16 -> 32 58 -> 42 us (40), 32 -> 32 76 -> 44 (53, partly from the
+ * cache), 32 -> 32 with pooling 117 -> 65 (59), 64 -> 32 175 -> 81 (59), 32 -> 16 float
+ * 49 -> 37 (53), display 71 -> 42; gradients 32 -> 32 110 -> 88 (79), 32 -> 64 187 -> 101
+ * (66). Memory bounds all but the 64-channel ones, which wait for it between their
+ * tiles' products as well. */
+template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL, int IO, int MBW>
+__global__ void __launch_bounds__(256, NB == 4 || CIN == 64 ? 2 : 3) k_conv_rows(const bf16_t* __restrict__ x, const bf16_t* __restrict__ coarse,
 	const bf16_t* __restrict__ w, const float* __restrict__ bias, void* __restrict__ y, int H, int W, bf16_t* __restrict__ ypool,
-	FrameIO io = FrameIO{}, const bf16_t* __restrict__ act = nullptr)
+	FrameIO io, const bf16_t* __restrict__ act, int across, int tiles)
 {
+	static_assert(IO != IO_SPLIT || (NB == 4 && !F32OUT && !RELU && !POOL), "the concatenation's gradient has 64 channels");
+	static_assert(IO != IO_DISPLAY || (NB == 1 && F32OUT && !RELU), "the display epilogue reads the first output channels");
+	constexpr int CX = CAT ? 32 : CIN, CKX = CX < 32 ? 32 : CX;   /* channels of x, padded to K */
+	constexpr int CP = CKX + 8, CH8 = CX / 8, CHP = CKX / 8, KS = CAT ? 2 : CKX / 32, WCIN = CAT ? 64 : CIN;
+	constexpr bool LOOP = CIN == 64 || NB == 4;
+	constexpr int TX = 16 * MBW, TY = 16, TW = TX + 2, TR = TY + 2;
+	constexpr int CPC = 40, TWC = TX / 2 + 2, TRC = TY / 2 + 2;   /* coarse tile */
+	constexpr int Cout = NB * 16;
+	__shared__ __attribute__((aligned(16))) bf16_t xs[TR * TW * CP];
+	__shared__ __attribute__((aligned(16))) float bs[Cout];
+	__shared__ __attribute__((aligned(16))) bf16_t cs[CAT ? TRC * TWC * CPC : IO == IO_SPLIT ? (TY / 2) * (TX / 2) * CPC : 8];   /* coarse pixels, or those of the coarse mask */
+	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ml = lane & 15, kg = lane >> 4;
+	bf8v wt[9][KS][NB];
+#pragma unroll
+	for (int tap = 0; tap < 9; tap++)
+#pragma unroll
+		for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+			for (int nb = 0; nb < NB; nb++)
+			{
+				const int k = ks * 32 + kg * 8;
+				wt[tap][ks][nb] = k < WCIN ? *(const bf8v*)(w + ((size_t)(tap * Cout + nb * 16 + ml) * WCIN + k)) : (bf8v){ 0, 0, 0, 0, 0, 0, 0, 0 };
+			}
+	if (tid < Cout) bs[tid] = bias ? bias[tid] : 0.0f;
+	const int wy = wave * 4;                                 /* the wave's first row in the tile */
+	const int fine = (wy * TW + ml) * CP + kg * 8;   /* the lane's place in the tile, and in the coarse one for the middle tap and the left (+ 1: the right) */
+	const int codd = ((wy >> 1) * TWC + (ml >> 1) + 1) * CPC + kg * 8, ceven = ((wy >> 1) * TWC + ((ml + 1) >> 1)) * CPC + kg * 8;
+	constexpr bool PAIRED = !F32OUT && (NB % 2) == 0, PAIRS = POOL || IO == IO_SPLIT;
+	constexpr int PNB = IO == IO_SPLIT ? 2 : NB;         /* channel blocks that are pooled */
+	/* XCD blockIdx % 8 gets an eighth of the tiles, in one piece: halos are read from its own L2 */
+	const int xcd = blockIdx.x & 7, end = (int)((long long)tiles * (xcd + 1) >> 3);
+	for (int tile = (int)((long long)tiles * xcd >> 3) + (blockIdx.x >> 3); tile < end; tile += gridDim.x >> 3)
+	{
+		const int x0 = (tile % across) * TX, r0 = (tile / across) * TY;
+		int lt = tid;
+		if (LOOP) asm volatile("" : "+v"(lt));            /* the staging's addresses are worked out per tile: kept over the loop they spill */
+		if (LOOP) __syncthreads();                       /* the waves have read the last tile */
+		{	/* the tile's loads in flight together */
+			constexpr int N = TR * TW * CHP, IT = (N + 255) / 256, BATCH = IT < 12 ? IT : (IT + 1) / 2;
+#pragma unroll
+			for (int it0 = 0; it0 < IT; it0 += BATCH)
+			{
+				uint4 v[BATCH];
+#pragma unroll
+				for (int j = 0; j < BATCH; j++)
+				{
+					const int i = lt + (it0 + j) * 256;
+					const int c8 = i % CHP, p = (i / CHP) % TW, gy = r0 - 1 + i / (CHP * TW), gx = x0 - 1 + p;
+					v[j] = it0 + j < IT && i < N && c8 < CH8 && gy >= 0 && gy < H && gx >= 0 && gx < W ?
+						*(const uint4*)(x + ((size_t)gy * W + gx) * CX + c8 * 8) : make_uint4(0, 0, 0, 0);
+				}
+#pragma unroll
+				for (int j = 0; j < BATCH; j++)
+				{
+					const int i = lt + (it0 + j) * 256;
+					if (it0 + j < IT && i < N) *(uint4*)(xs + (i / CHP) * CP + (i % CHP) * 8) = v[j];
+				}
+			}
+			if (IO == IO_SPLIT)
+			{
+				constexpr int NM = (TY / 2) * (TX / 2) * 4;
+				static_assert(IO != IO_SPLIT || NM == 256, "a load each");
+				const int cy = (r0 >> 1) + lt / (TX * 2), cx = (x0 >> 1) + (lt >> 2) % (TX / 2);
+				*(uint4*)(cs + (lt >> 2) * CPC + (lt & 3) * 8) = cy < (H >> 1) && cx < (W >> 1) ?
+					*(const uint4*)(act + ((size_t)cy * (W >> 1) + cx) * 32 + (lt & 3) * 8) : make_uint4(0, 0, 0, 0);
+			}
+			if (CAT)
+			{
+				constexpr int NC = TRC * TWC * 4, ITC = (NC + 255) / 256;
+				const int Hc = H >> 1, Wc = W >> 1;
+				uint4 v[ITC];
+#pragma unroll
+				for (int j = 0; j < ITC; j++)
+				{
+					const int i = lt + j * 256;
+					const int c8 = i % 4, p = (i / 4) % TWC, cy = (r0 >> 1) - 1 + i / (4 * TWC), cx = (x0 >> 1) - 1 + p;
+					v[j] = i < NC && cy >= 0 && cy < Hc && cx >= 0 && cx < Wc ? *(const uint4*)(coarse + ((size_t)cy * Wc + cx) * 32 + c8 * 8) : make_uint4(0, 0, 0, 0);
+				}
+#pragma unroll
+				for (int j = 0; j < ITC; j++)
+				{
+					const int i = lt + j * 256;
+					if (i < NC) *(uint4*)(cs + (i / 4) * CPC + (i % 4) * 8) = v[j];
+				}
+			}
+		}
+		f4v acc[4][MBW][NB];
+#pragma unroll
+		for (int o = 0; o < 4; o++)
+#pragma unroll
+			for (int mb = 0; mb < MBW; mb++)
+#pragma unroll
+				for (int nb = 0; nb < NB; nb++) acc[o][mb][nb] = (f4v){ 0.0f, 0.0f, 0.0f, 0.0f };
+		__syncthreads();
+#pragma unroll
+		for (int ir = 0; ir < 6; ir++)                      /* input row of the tile wy + ir */
+#pragma unroll
+			for (int dx = 0; dx < 3; dx++)
+#pragma unroll
+				for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+					for (int mb = 0; mb < MBW; mb++)
+					{
+						bf8v a;
+						if (CAT && ks == 0) a = *(const bf8v*)(cs + (((ir + 1) >> 1) * TWC + mb * 8 + (dx == 2)) * CPC + (dx == 1 ? codd : ceven));
+						else a = *(const bf8v*)(xs + (ir * TW + mb * 16 + dx) * CP + (CAT ? 0 : ks * 32) + fine);
+#pragma unroll
+						for (int o = 0; o < 4; o++)
+						{
+							const int dy = ir - o;
+							if (dy < 0 || dy > 2) continue;
+#pragma unroll
+							for (int nb = 0; nb < NB; nb++) acc[o][mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wt[dy * 3 + dx][ks][nb], a, acc[o][mb][nb], 0, 0, 0);
+						}
+					}
+#pragma unroll
+		for (int mb = 0; mb < MBW; mb++)
+		{
+			const int px = x0 + mb * 16 + ml;
+			if constexpr (IO == IO_DISPLAY)
+			{	/* channels 0..3 of the four rows are with lanes 0..15; swaps hand row kg to the lanes of kg, and each lane
+				 * writes one pixel of the frame */
+				float v[4];
+#pragma unroll
+				for (int i = 0; i < 4; i++)
+				{
+					auto u = [&](int o) { const float f = acc[o][mb][0][i]; return __builtin_bit_cast(uint32_t, f); };   /* (the cast of a vector's element takes element 0) */
+					const uint32_t r01 = __builtin_amdgcn_permlane16_swap(u(0), u(1), false, false)[0], r23 = __builtin_amdgcn_permlane16_swap(u(2), u(3), false, false)[0];
+					v[i] = __builtin_bit_cast(float, (uint32_t)__builtin_amdgcn_permlane32_swap(r01, r23, false, false)[0]) + bs[i];
+				}
+				const int py = r0 + wy + kg;
+				if (py < io.h && px < io.w)
+				{
+					const size_t q = (size_t)px + (size_t)py * io.w;
+					io.image[q] = frame_display(v[0], v[1], v[2], io.feat[q].x);
+				}
+				continue;
+			}
+			float above[PAIRS ? PNB : 1][4];                 /* sums of the pixel pairs of the row above */
+#pragma unroll
+			for (int o = 0; o < 4; o++)
+			{
+				const int ry = r0 + wy + o;
+				uint32_t pk[NB][2], pq[PAIRS ? PNB : 1][2];
+#pragma unroll
+				for (int nb = 0; nb < NB; nb++)
+				{
+					const f4v bv = *(const f4v*)(bs + nb * 16 + kg * 4);
+					float v[4];
+#pragma unroll
+					for (int i = 0; i < 4; i++)
+					{
+						v[i] = acc[o][mb][nb][i] + bv[i];
+						if (RELU) v[i] = v[i] > 0.0f ? v[i] : 0.0f;
+					}
+					if (F32OUT)
+					{
+						if (ry < H && px < W) *(float4*)((float*)y + ((size_t)ry * W + px) * Cout + nb * 16 + kg * 4) = make_float4(v[0], v[1], v[2], v[3]);
+					}
+					else
+					{
+						pk[nb][0] = pack_bf(v[0], v[1]), pk[nb][1] = pack_bf(v[2], v[3]);
+						if (!PAIRED && ry < H && px < W) *(uint2*)((bf16_t*)y + ((size_t)ry * W + px) * Cout + nb * 16 + kg * 4) = make_uint2(pk[nb][0], pk[nb][1]);
+					}
+					if (PAIRS && nb < PNB)
+					{	/* 2x2 sums of the stored (bf16) values: (left + right) of the top row + of the bottom row, as
+						 * dn_pool2 (times 1/4) and dn_upcat_bwd on the stored tensor */
+						float hs[4];
+#pragma unroll
+						for (int i = 0; i < 4; i++)
+						{
+							const float r = bf2f((bf16_t)(pk[nb][i >> 1] >> (16 * (i & 1))));
+							hs[i] = r + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, r), 0xb1, 0xf, 0xf, true));   /* lane ^ 1 */
+						}
+						const int pb = nb < PNB ? nb : 0;
+						if (o & 1)
+						{
+							float q[4];
+#pragma unroll
+							for (int i = 0; i < 4; i++) q[i] = (above[pb][i] + hs[i]) * (IO == IO_SPLIT ? 1.0f : 0.25f);
+							pq[pb][0] = pack_bf(q[0], q[1]), pq[pb][1] = pack_bf(q[2], q[3]);
+						}
+						else
+#pragma unroll
+							for (int i = 0; i < 4; i++) above[pb][i] = hs[i];
+					}
+				}
+				/* channel blocks in pairs: row swaps of 16 lanes leave each lane 8 consecutive channels of its pixel (kg even:
+				 * block nb, channels 4 kg .. + 7; kg odd: block nb + 1, channels 4 (kg - 1) .. + 7), so one 16-byte store
+				 * covers whole 64-byte pixels */
+				const int ch8 = (kg & 1) ? 16 + (kg - 1) * 4 : kg * 4;
+				auto octet = [](const uint32_t (&p)[2], const uint32_t (&q)[2])
+				{
+					const auto a = __builtin_amdgcn_permlane16_swap(p[0], q[0], false, false);
+					const auto b = __builtin_amdgcn_permlane16_swap(p[1], q[1], false, false);
+					return make_uint4(a[0], b[0], a[1], b[1]);
+				};
+				if (PAIRED)
+				{
+#pragma unroll
+					for (int nb = IO == IO_SPLIT ? 2 : 0; nb < NB; nb += 2)
+					{
+						uint4 q = octet(pk[nb], pk[nb + 1]);
+						constexpr int YC = IO == IO_SPLIT ? 32 : Cout;
+						const size_t at = ((size_t)ry * W + px) * YC + nb * 16 + ch8 - (Cout - YC);
+						if (ry < H && px < W)
+						{
+							if (IO == IO_MASK)
+							{
+								const uint4 m = *(const uint4*)(act + at);
+								q = make_uint4(relu_mask2(m.x, q.x), relu_mask2(m.y, q.y), relu_mask2(m.z, q.z), relu_mask2(m.w, q.w));
+							}
+							*(uint4*)((bf16_t*)y + at) = q;
+						}
+					}
+				}
+				if constexpr (PAIRS)
+					if (o & 1)
+					{
+						static_assert(PNB == 2, "one pair");
+						uint4 q = octet(pq[0], pq[1]);
+						if (IO == IO_SPLIT)
+						{
+							const uint4 m = *(const uint4*)(cs + (((wy + o) >> 1) * (TX / 2) + ((mb * 16 + ml) >> 1)) * CPC + ch8);
+							q = make_uint4(relu_mask2(m.x, q.x), relu_mask2(m.y, q.y), relu_mask2(m.z, q.z), relu_mask2(m.w, q.w));
+						}
+						if (!(ml & 1) && ry < H && px < W) *(uint4*)(ypool + ((size_t)(ry >> 1) * (W >> 1) + (px >> 1)) * 32 + ch8) = q;
+					}
+			}
+		}
+		if (!LOOP) break;
+	}
+}
+
+template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL, int IO>
+__global__ void __launch_bounds__(256) k_conv3x3_t(const bf16_t* __restrict__ x, const bf16_t* __restrict__ coarse,
+	const bf16_t* __restrict__ w, const float* __restrict__ bias, void* __restrict__ y, int H, int W, bf16_t* __restrict__ ypool,
+	FrameIO io, const bf16_t* __restrict__ act)
+{
+	constexpr int MBW = 1, ROWS = 4;
 	static_assert(IO != IO_SPLIT || (NB == 4 && !F32OUT && !RELU && !POOL), "the concatenation's gradient has 64 channels");
 	static_assert(IO != IO_DISPLAY || (NB == 1 && F32OUT && !RELU), "the display epilogue reads the first output channels");
 	constexpr int CX = CAT ? 32 : CIN;                  /* channels of x */
@@ -234,25 +489,17 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 		return k < WCIN ? *(const bf8v*)(w + ((size_t)(tap * Cout + nb * 16 + ml) * WCIN + k)) : (bf8v){ 0, 0, 0, 0, 0, 0, 0, 0 };
 	};
 	/* bias now, beside the tile's loads, so that the epilogue waits on nothing;
-	 * weight fragments two taps ahead of their products */
+	 * weight fragments a tap ahead of their products */
 	float bv[NB][4];
 #pragma unroll
 	for (int nb = 0; nb < NB; nb++)
 #pragma unroll
 		for (int i = 0; i < 4; i++) bv[nb][i] = bias ? bias[nb * 16 + kg * 4 + i] : 0.0f;
-	/* weight fragments PD taps ahead of their products: two where the third
-	 * set of registers costs no occupancy (64-pixel tiles, 32 input channels,
-	 * up to 32 outputs), else one with the tap loop kept rolled */
-	constexpr int PD = MBW > 1 && (CIN == 32 || CAT) && NB <= 2 ? 2 : 1;
-	bf8v wc[KS][NB], w1[KS][NB], w2[KS][NB];
+	bf8v wc[KS][NB], w1[KS][NB];
 #pragma unroll
 	for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-		for (int nb = 0; nb < NB; nb++)
-		{
-			wc[ks][nb] = wfrag(0, ks, nb);
-			if (PD == 2) w1[ks][nb] = wfrag(1, ks, nb);
-		}
+		for (int nb = 0; nb < NB; nb++) wc[ks][nb] = wfrag(0, ks, nb);
 	f4v acc[MBW][NB];
 #pragma unroll
 	for (int mb = 0; mb < MBW; mb++)
@@ -274,39 +521,19 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 				for (int nb = 0; nb < NB; nb++) acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wc[ks][nb], a, acc[mb][nb], 0, 0, 0);
 			}
 	};
-	if constexpr (PD == 2)
-	{
-#pragma unroll
-		for (int tap = 0; tap < 9; tap++)
-		{
-			if (tap < 7)
-#pragma unroll
-				for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-					for (int nb = 0; nb < NB; nb++) w2[ks][nb] = wfrag(tap + 2, ks, nb);
-			products(tap);
-#pragma unroll
-			for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-				for (int nb = 0; nb < NB; nb++) wc[ks][nb] = w1[ks][nb], w1[ks][nb] = w2[ks][nb];
-		}
-	}
-	else
-	{
 #pragma unroll 1
-		for (int tap = 0; tap < 9; tap++)
-		{
-			if (tap < 8)
-#pragma unroll
-				for (int ks = 0; ks < KS; ks++)
-#pragma unroll
-					for (int nb = 0; nb < NB; nb++) w1[ks][nb] = wfrag(tap + 1, ks, nb);
-			products(tap);
+	for (int tap = 0; tap < 9; tap++)
+	{
+		if (tap < 8)
 #pragma unroll
 			for (int ks = 0; ks < KS; ks++)
 #pragma unroll
-				for (int nb = 0; nb < NB; nb++) wc[ks][nb] = w1[ks][nb];
-		}
+				for (int nb = 0; nb < NB; nb++) w1[ks][nb] = wfrag(tap + 1, ks, nb);
+		products(tap);
+#pragma unroll
+		for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+			for (int nb = 0; nb < NB; nb++) wc[ks][nb] = w1[ks][nb];
 	}
 	const int ry = r0 + wave;
 	constexpr bool PAIRS = POOL || IO == IO_SPLIT;       /* 2 x 2 sums of the first PNB channel blocks */
@@ -336,7 +563,7 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 			}
 			const size_t o = ((size_t)ry * W + px) * Cout + ch;
 			if (PAIRED)
-				pk[mb][nb][0] = (uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16, pk[mb][nb][1] = (uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16;
+				pk[mb][nb][0] = pack_bf(v[0], v[1]), pk[mb][nb][1] = pack_bf(v[2], v[3]);
 			else if (IO == IO_DISPLAY)
 			{	/* lanes holding channels 0..3 write the display pixel of the frame */
 				if (kg == 0 && ry < io.h && px < io.w)
@@ -348,8 +575,8 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 			else if (ry < H && px < W)
 			{
 				if (F32OUT) *(float4*)((float*)y + o) = make_float4(v[0], v[1], v[2], v[3]);
-				else *(uint2*)((bf16_t*)y + o) = make_uint2((uint32_t)f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16,
-					(uint32_t)f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16);
+				else *(uint2*)((bf16_t*)y + o) = make_uint2(pack_bf(v[0], v[1]),
+					pack_bf(v[2], v[3]));
 			}
 			if (PAIRS && nb < PNB)                        /* the stored (bf16) values, left + right */
 #pragma unroll
@@ -430,54 +657,51 @@ __global__ void __launch_bounds__(64 * ROWS) k_conv3x3_t(const bf16_t* __restric
 	}
 }
 
-/* Images with fewer than SMALL_TILES 64-pixel-wide tiles of 4 rows (levels
- * 3 and 4 of the network at 1080p) run 4 x 16 tiles: four times the blocks,
- * so that a small layer spreads over more compute units instead of running
- * at the latency of a few blocks. (At level 2, 4 x 16 tiles were slower: a
- * block's nine dependent weight loads then outweigh its products.) */
-static const int SMALL_TILES = 256;
+/* Images with fewer than SMALL_TILES 64-pixel-wide tiles of 4 rows run 4 x 16
+ * tiles, a wave per row: four to eight times the blocks, so that a small layer
+ * spreads over more compute units instead of running at the latency of a few
+ * blocks (128 x 128, 64 such tiles: 4.6 against 6.3 us for 32 -> 32 with pooling, 6.7
+ * against 10.3 for the concatenation; 240 x 144, 144 tiles: 6.3 and 6.4, 14.7 and
+ * 11.1). */
+static const int SMALL_TILES = 128;
 static bool small_image(int H, int W) { return ((W + 63) / 64) * ((H + 3) / 4) < SMALL_TILES; }
 
 
-template <int CIN, int NB, bool CAT, int MBW, int ROWS>
-static void conv_t_w(const bf16_t* x, const bf16_t* coarse, const bf16_t* w, const float* bias, void* y, int H, int W, int flags, hipStream_t s)
+/* The tiled convolution with the tile that suits the image. Large ones: 32 x 16
+ * pixels, 16 x 16 where the sums of 64 outputs or the plain 64-channel tile would
+ * not leave two blocks a CU. */
+template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL, int IO>
+static hipError_t conv_tile(const bf16_t* x, const bf16_t* coarse, const bf16_t* w, const float* bias, void* y, int H, int W, bf16_t* ypool,
+	const FrameIO& io, const bf16_t* act, hipStream_t s)
 {
-	const dim3 grid((W + 16 * MBW - 1) / (16 * MBW), (H + ROWS - 1) / ROWS), block(64 * ROWS);
-	const bool relu = flags & DN_RELU, f32 = flags & DN_OUT_F32;
-	if (relu && f32) k_conv3x3_t<CIN, NB, true, true, CAT, false, MBW, ROWS><<<grid, block, 0, s>>>(x, coarse, w, bias, y, H, W, nullptr);
-	else if (relu) k_conv3x3_t<CIN, NB, true, false, CAT, false, MBW, ROWS><<<grid, block, 0, s>>>(x, coarse, w, bias, y, H, W, nullptr);
-	else if (f32) k_conv3x3_t<CIN, NB, false, true, CAT, false, MBW, ROWS><<<grid, block, 0, s>>>(x, coarse, w, bias, y, H, W, nullptr);
-	else k_conv3x3_t<CIN, NB, false, false, CAT, false, MBW, ROWS><<<grid, block, 0, s>>>(x, coarse, w, bias, y, H, W, nullptr);
+	constexpr int MBW = NB == 4 || (CIN == 64 && !CAT) ? 1 : 2, TX = 16 * MBW;
+	const int across = (W + TX - 1) / TX, tiles = across * ((H + 15) / 16);
+	const int blocks = (NB == 4 || CIN == 64) && tiles > 512 ? 512 : (tiles + 7) & ~7;   /* two a CU walk the tiles; or one a tile, a multiple of the XCDs */
+	if (small_image(H, W))
+		k_conv3x3_t<CIN, NB, RELU, F32OUT, CAT, POOL, IO><<<dim3((W + 15) / 16, (H + 3) / 4), 256, 0, s>>>(x, coarse, w, bias, y, H, W, ypool, io, act);
+	else
+		k_conv_rows<CIN, NB, RELU, F32OUT, CAT, POOL, IO, MBW><<<blocks, 256, 0, s>>>(x, coarse, w, bias, y, H, W,
+			ypool, io, act, across, tiles);
+	return hipGetLastError();
 }
 
 template <int CIN, int NB, bool CAT>
 static hipError_t conv_t(const bf16_t* x, const bf16_t* coarse, const bf16_t* w, const float* bias, void* y, int H, int W, int flags, hipStream_t s)
 {
-	/* 64 input channels without the concatenation keep 4-row tiles (an 8-row tile would not leave room for two blocks per CU) */
-	constexpr int ROWS = (CIN == 64 && !CAT) ? 4 : TILE_ROWS;
-	if (small_image(H, W)) conv_t_w<CIN, NB, CAT, 1, 4>(x, coarse, w, bias, y, H, W, flags, s);
-	else conv_t_w<CIN, NB, CAT, 4, ROWS>(x, coarse, w, bias, y, H, W, flags, s);
-	return hipGetLastError();
+	const bool relu = flags & DN_RELU, f32 = flags & DN_OUT_F32;
+	const FrameIO io{};
+	if (relu && f32) return conv_tile<CIN, NB, true, true, CAT, false, IO_NONE>(x, coarse, w, bias, y, H, W, nullptr, io, nullptr, s);
+	if (relu) return conv_tile<CIN, NB, true, false, CAT, false, IO_NONE>(x, coarse, w, bias, y, H, W, nullptr, io, nullptr, s);
+	if (f32) return conv_tile<CIN, NB, false, true, CAT, false, IO_NONE>(x, coarse, w, bias, y, H, W, nullptr, io, nullptr, s);
+	return conv_tile<CIN, NB, false, false, CAT, false, IO_NONE>(x, coarse, w, bias, y, H, W, nullptr, io, nullptr, s);
 }
 
 hipError_t dn_conv3x3_pool(const bf16_t* x, int Cin, const bf16_t* w, const float* bias, bf16_t* y, int Cout, int H, int W,
 	bf16_t* ypool, hipStream_t s)
 {
 	if (Cout != 32 || (Cin != 16 && Cin != 32) || H <= 0 || W <= 0 || H % 2 || W % 2) return hipErrorInvalidValue;
-	const dim3 block(256);
-	if (small_image(H, W))
-	{
-		const dim3 grid((W + 15) / 16, (H + 3) / 4);
-		if (Cin == 16) k_conv3x3_t<16, 2, true, false, false, true, 1><<<grid, block, 0, s>>>(x, nullptr, w, bias, y, H, W, ypool);
-		else k_conv3x3_t<32, 2, true, false, false, true, 1><<<grid, block, 0, s>>>(x, nullptr, w, bias, y, H, W, ypool);
-	}
-	else
-	{
-		const dim3 grid((W + 63) / 64, (H + TILE_ROWS - 1) / TILE_ROWS), blockL(64 * TILE_ROWS);
-		if (Cin == 16) k_conv3x3_t<16, 2, true, false, false, true, 4, TILE_ROWS><<<grid, blockL, 0, s>>>(x, nullptr, w, bias, y, H, W, ypool);
-		else k_conv3x3_t<32, 2, true, false, false, true, 4, TILE_ROWS><<<grid, blockL, 0, s>>>(x, nullptr, w, bias, y, H, W, ypool);
-	}
-	return hipGetLastError();
+	if (Cin == 16) return conv_tile<16, 2, true, false, false, true, IO_NONE>(x, nullptr, w, bias, y, H, W, ypool, FrameIO{}, nullptr, s);
+	return conv_tile<32, 2, true, false, false, true, IO_NONE>(x, nullptr, w, bias, y, H, W, ypool, FrameIO{}, nullptr, s);
 }
 
 hipError_t dn_conv3x3_cat(const bf16_t* coarse, const bf16_t* skip, const bf16_t* w, const float* bias, void* y, int Cout, int H, int W,
@@ -525,24 +749,12 @@ hipError_t dn_conv3x3(const bf16_t* x, int Cin, const bf16_t* w, const float* bi
  * dn_frame_output bit for bit, without the fp32 output tensor. (Reading the
  * frame into the first convolution's tile the same way was measured slower
  * than dn_frame_input + dn_conv3x3: 181 against 99 µs at 1080p.) */
-template <int CIN, int NB, bool RELU, bool F32OUT, int IO>
-static void conv_io(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int H, int W, const FrameIO& io, hipStream_t s)
-{
-	if (small_image(H, W))
-		k_conv3x3_t<CIN, NB, RELU, F32OUT, false, false, 1, 4, IO><<<dim3((W + 15) / 16, (H + 3) / 4), 256, 0, s>>>(x, nullptr, w, bias, y, H, W,
-			nullptr, io);
-	else
-		k_conv3x3_t<CIN, NB, RELU, F32OUT, false, false, 4, TILE_ROWS, IO><<<dim3((W + 63) / 64, (H + TILE_ROWS - 1) / TILE_ROWS), 64 * TILE_ROWS, 0,
-			s>>>(x, nullptr, w, bias, y, H, W, nullptr, io);
-}
-
 hipError_t dn_conv3x3_display(const bf16_t* x, const bf16_t* wts, const float* bias, const uint4* features, int w, int h, float4* image,
 	int Hp, int Wp, hipStream_t s)
 {
 	if (w <= 0 || h <= 0 || Hp < h || Wp < w) return hipErrorInvalidValue;
 	const FrameIO io{ features, w, h, image };
-	conv_io<32, 1, false, true, IO_DISPLAY>(x, wts, bias, nullptr, Hp, Wp, io, s);
-	return hipGetLastError();
+	return conv_tile<32, 1, false, true, false, false, IO_DISPLAY>(x, nullptr, wts, bias, nullptr, Hp, Wp, nullptr, io, nullptr, s);
 }
 
 /* Input gradients with what follows them in the backward pass done by the
@@ -550,30 +762,17 @@ hipError_t dn_conv3x3_display(const bf16_t* x, const bf16_t* wts, const float* b
  * the concatenation's (dn_conv3x3 to 64 channels + dn_upcat_bwd + dn_relu_bwd
  * of the coarse half), bit for bit. Level 0 at 1088 x 1920: the ReLU pass alone
  * moved 402 MB (66 us) per layer, the 64-channel tensor 268 MB out and back. */
-template <int CIN, int NB, int IO>
-static void conv_dx(const bf16_t* gy, const bf16_t* w, bf16_t* gx, bf16_t* gcoarse, const bf16_t* act, int H, int W, hipStream_t s)
-{
-	if (small_image(H, W))
-		k_conv3x3_t<CIN, NB, false, false, false, false, 1, 4, IO><<<dim3((W + 15) / 16, (H + 3) / 4), 256, 0, s>>>(gy, nullptr, w, nullptr, gx, H, W,
-			gcoarse, FrameIO{}, act);
-	else
-		k_conv3x3_t<CIN, NB, false, false, false, false, 4, TILE_ROWS, IO><<<dim3((W + 63) / 64, (H + TILE_ROWS - 1) / TILE_ROWS), 64 * TILE_ROWS, 0,
-			s>>>(gy, nullptr, w, nullptr, gx, H, W, gcoarse, FrameIO{}, act);
-}
-
 hipError_t dn_conv3x3_dx_relu(const bf16_t* gy, int Cin, const bf16_t* w, const bf16_t* act, bf16_t* gx, int Cout, int H, int W, hipStream_t s)
 {
 	if (Cout != 32 || (Cin != 16 && Cin != 32) || H <= 0 || W <= 0 || !aligned16_3(gy, act, gx)) return hipErrorInvalidValue;
-	if (Cin == 16) conv_dx<16, 2, IO_MASK>(gy, w, gx, nullptr, act, H, W, s);
-	else conv_dx<32, 2, IO_MASK>(gy, w, gx, nullptr, act, H, W, s);
-	return hipGetLastError();
+	if (Cin == 16) return conv_tile<16, 2, false, false, false, false, IO_MASK>(gy, nullptr, w, nullptr, gx, H, W, nullptr, FrameIO{}, act, s);
+	return conv_tile<32, 2, false, false, false, false, IO_MASK>(gy, nullptr, w, nullptr, gx, H, W, nullptr, FrameIO{}, act, s);
 }
 
 hipError_t dn_conv3x3_dx_cat(const bf16_t* gy, const bf16_t* w, const bf16_t* actCoarse, bf16_t* gcoarse, bf16_t* gskip, int H, int W, hipStream_t s)
 {
 	if (H <= 0 || W <= 0 || H % 2 || W % 2 || !aligned16_3(gy, actCoarse, gcoarse) || !aligned16(gskip)) return hipErrorInvalidValue;
-	conv_dx<32, 4, IO_SPLIT>(gy, w, gskip, gcoarse, actCoarse, H, W, s);
-	return hipGetLastError();
+	return conv_tile<32, 4, false, false, false, false, IO_SPLIT>(gy, nullptr, w, nullptr, gskip, H, W, gcoarse, FrameIO{}, actCoarse, s);
 }
 
 /* ---- weight gradient ---------------------------------------------------
@@ -1223,7 +1422,7 @@ __global__ void k_pack_input(const float4* __restrict__ rad, const float4* __res
 	{
 		const float4 r = rad[p], a = alb[p], n = nrm[p];
 		const float d = depth[p];
-		auto pk = [](float lo, float hi) { return (uint32_t)f2bf(lo) | (uint32_t)f2bf(hi) << 16; };
+		auto pk = [](float lo, float hi) { return pack_bf(lo, hi); };
 		uint4* o = (uint4*)(out + p * 16);
 		o[0] = make_uint4(pk(r.x, r.y), pk(r.z, a.x), pk(a.y, a.z), pk(n.x, n.y));
 		o[1] = make_uint4(pk(n.z, d), 0, 0, 0);
@@ -1261,7 +1460,7 @@ __global__ void k_frame_input(const float4* __restrict__ acc, const uint4* __res
 		float c[3];
 		for (int k = 0; k < 3; k++) c[k] = log1pf(fmaxf(r[k], 0.0f) / fmaxf(al[k], DN_ALBEDO_FLOOR));
 		const float dz = log1pf(depth) * 0.1f;
-		auto pk = [](float lo, float hi) { return (uint32_t)f2bf(lo) | (uint32_t)f2bf(hi) << 16; };
+		auto pk = [](float lo, float hi) { return pack_bf(lo, hi); };
 		o[0] = make_uint4(pk(c[0], c[1]), pk(c[2], a.x), pk(a.y, a.z), pk(n.x, n.y));
 		o[1] = make_uint4(pk(n.z, dz), 0, 0, 0);
 	}

@@ -1,7 +1,7 @@
 """The backward pass's fused and batched kernels against the separate calls they
 replace (bit for bit) and the weight gradient against FP64, at the edges of
-their tiles: 32-pixel segments and 8-row chunks of the weight gradient, 16- and
-64-pixel tiles of the convolutions, 256-element blocks of the Adam step."""
+their tiles: 32-pixel segments and 8-row chunks of the weight gradient, 16-
+and 32-pixel tiles of the convolutions, 256-element blocks of the Adam step."""
 import ctypes
 
 import numpy as np
@@ -79,7 +79,7 @@ def test_weight_gradient_batch_with_concatenation(torch_cuda):
 
 @pytest.mark.parametrize("H,W", [(2, 2), (6, 18), (22, 70), (202, 1930)])
 def test_input_gradients_equal_their_parts(torch_cuda, H, W):
-    """dx_relu, dx_cat and pool2_bwd_relu; 202 x 1930 runs the 8 x 64 tiles, ragged both ways."""
+    """dx_relu, dx_cat and pool2_bwd_relu; 202 x 1930 runs the large tiles, ragged both ways."""
     torch = torch_cuda
     L = lh.library()
     sh = torch.cuda.current_stream().cuda_stream
@@ -149,3 +149,43 @@ def test_adam_batch_and_vector_loss_equal_the_single_calls(torch_cuda):
 
 def test_batch_records_match_the_header():
     assert ctypes.sizeof(D._Layer) == 56 and ctypes.sizeof(D._Tensor) == 64
+
+
+@pytest.mark.parametrize("H,W", [(514, 62), (256, 128), (258, 130), (1038, 546)])
+def test_row_tiles_equal_small_tiles(torch_cuda, H, W):
+    """Large images (4 rows x 16 or 32 pixels a wave; with 64 channels, blocks that
+    walk several tiles at 1038 x 546), ragged or whole both ways, against crops of
+    the same input at even corners through the 4 x 16 tiles, whose sums run over
+    the taps and channels in the same order: bit for bit."""
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(H + W)
+    bf = lambda *s: R.bf16(rng.standard_normal(s))
+    x64, x32, coarse = bf(H, W, 64), bf(H, W, 32), bf(H // 2, W // 2, 32)
+    w64, w32, wg = dev(torch, bf(9, 32, 64) * 0.2), dev(torch, bf(9, 32, 32) * 0.2), dev(torch, bf(9, 64, 32) * 0.2)
+    b = torch.from_numpy(rng.standard_normal(32).astype(np.float32)).cuda()
+
+    def run(y0, y1, x0, x1):
+        h, w = y1 - y0, x1 - x0
+        cut = lambda t: dev(torch, np.ascontiguousarray(t[y0:y1, x0:x1]))
+        half = dev(torch, np.ascontiguousarray(coarse[y0 // 2:y1 // 2, x0 // 2:x1 // 2]))
+        a, s, out = cut(x64), cut(x32), [empty(torch, h * w * 32) for _ in range(4)]
+        small = [empty(torch, h * w * 8) for _ in range(2)]
+        assert L.lh2hip_dn_conv3x3(a.data_ptr(), 64, w64.data_ptr(), b.data_ptr(), out[0].data_ptr(), 32, h, w, 1, sh) == 0
+        assert L.lh2hip_dn_conv3x3_cat(half.data_ptr(), s.data_ptr(), w64.data_ptr(), b.data_ptr(), out[1].data_ptr(), 32, h, w, 1, sh) == 0
+        assert L.lh2hip_dn_conv3x3_pool(s.data_ptr(), 32, w32.data_ptr(), b.data_ptr(), out[2].data_ptr(), 32, h, w, small[0].data_ptr(), sh) == 0
+        assert L.lh2hip_dn_conv3x3_dx_cat(s.data_ptr(), wg.data_ptr(), half.data_ptr(), small[1].data_ptr(), out[3].data_ptr(), h, w, sh) == 0
+        torch.cuda.synchronize()
+        return [t.reshape(h, w, 32) for t in out] + [t.reshape(h // 2, w // 2, 32) for t in small]
+
+    full = run(0, H, 0, W)
+    for y0 in sorted({0, (H // 32) * 16 - 10, H - 28}):
+        for x0 in sorted({0, max((W // 64) * 32 - 10, 0), W - 28}):
+            y1, x1 = min(y0 + 28, H), min(x0 + 28, W)
+            part = run(y0, y1, x0, x1)
+            t, l = (2 if y0 else 0), (2 if x0 else 0)
+            e, r = y1 - y0 - (2 if y1 < H else 0), x1 - x0 - (2 if x1 < W else 0)
+            for k, (f, p) in enumerate(zip(full, part)):
+                q = 1 if k < 4 else 2
+                assert torch.equal(f[(y0 + t) // q:(y0 + e) // q, (x0 + l) // q:(x0 + r) // q], p[t // q:e // q, l // q:r // q]), (k, y0, x0)
