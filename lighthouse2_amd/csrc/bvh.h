@@ -109,6 +109,8 @@ hipError_t refit_layout(const BuildNode* dNodes, NodeF32* dF32, const int32_t* d
 
 /* Triangle soup (3 float4 per triangle) -> primitive boxes. */
 hipError_t tri_bounds(const float4* dVerts, int n, float4* dLo, float4* dHi, hipStream_t stream);
+/* *dMax = max(*dMax, records[i * stride]) over n records of `stride` words. */
+hipError_t max_word(const uint32_t* dRecords, int stride, int n, uint32_t* dMax, hipStream_t stream);
 
 /* Device layout of a build tree into the traversal formats (bvh_layout.hip).
  * Arrays are caller-owned device memory sized for the worst case: a build

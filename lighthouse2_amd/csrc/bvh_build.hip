@@ -108,6 +108,16 @@ __global__ void k_tri_bounds(const float4* __restrict__ v, int n, float4* __rest
 	hi[i] = make_float4(h.x, h.y, h.z, 0.0f);
 }
 
+/* One word of each record; bound by the 64-byte lines those words lie in. One
+ * atomic per wave, at most 1024 of them in a launch. */
+__global__ void k_max_word(const uint32_t* __restrict__ v, int stride, int n, uint32_t* __restrict__ out)
+{
+	uint32_t m = 0;
+	for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) m = max(m, v[(size_t)i * stride]);
+	m = (uint32_t)(wave_max((int)(m ^ 0x80000000u))) ^ 0x80000000u;
+	if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+}
+
 __global__ void k_build_init(BuildArgs A)
 {
 	if (threadIdx.x < 12) A.keys[threadIdx.x] = threadIdx.x % 6 < 3 ? KINF() : KNINF();
@@ -560,6 +570,13 @@ hipError_t tri_bounds(const float4* dVerts, int n, float4* dLo, float4* dHi, hip
 {
 	if (n <= 0) return hipSuccess;
 	k_tri_bounds<<<(n + 255) / 256, 256, 0, stream>>>(dVerts, n, dLo, dHi);
+	return hipGetLastError();
+}
+
+hipError_t max_word(const uint32_t* dRecords, int stride, int n, uint32_t* dMax, hipStream_t stream)
+{
+	if (n <= 0) return hipSuccess;
+	k_max_word<<<std::min((n + 255) / 256, 256), 256, 0, stream>>>(dRecords, stride, n, dMax);
 	return hipGetLastError();
 }
 

@@ -229,9 +229,10 @@ private:
 	TraceScene scene;
 	/* workspace of builds and layouts, kept between calls up to BUILD_WS_KEEP
 	 * bytes (a mesh of about 1.2 M triangles); used under the scene lock, on `stream` */
-	DevBuf buildWs;
+	DevBuf buildWs, maxMatB;           /* maxMatB: one word, largest material of a mesh being set */
 	static constexpr size_t BUILD_WS_KEEP = (size_t)256 << 20;
 	void trimBuildWorkspace();
+	hipError_t uploadCoreTris(MeshData& m, const lighthouse2::CoreTri* triangles, int count, uint32_t& maxMaterial);
 	/* trace scratch (overflow2 / sideCounters: the shadow-ray lane) */
 	DevBuf overflow, counters, overflow2, sideCounters;
 	hipStream_t stream2 = nullptr;
