@@ -51,15 +51,15 @@ static const uint32_t Q8_EMPTY = 0xffffffffu;
  * float whose exponent field is e (e = 0 gives 0, e = 255 infinity). */
 __host__ __device__ inline uint32_t q8_step_bits(uint32_t e) { return e << 23; }
 
-/* Per-instance record for the two-level traversal (64 bytes). */
+/* Per-instance record for the two-level traversal: as many bytes as a node, so
+ * that a lane entering an instance loads it where the others load their node. */
 struct InstanceRec
 {
 	float4 inv0, inv1, inv2;   /* rows of the inverse transform */
-	const void* nodes;         /* BLAS node array (NodeF32 or NodeQ8) */
-	const float4* tris;        /* BLAS leaf triangles */
-	uint32_t root;             /* BLAS root ref */
-	uint32_t flags;            /* bit 0: identity transform */
+	uint64_t nodes;            /* BLAS node array (NodeF32 or NodeQ8); bit 0: identity transform */
+	uint64_t tris;             /* BLAS leaf triangles; bit 0: the root is a leaf */
 };
+static_assert(sizeof(InstanceRec) == 64 && sizeof(NodeQ8) == 64 && sizeof(NodeF32) == 64, "one load path");
 
 /* A GPU build: the caller's device arrays (2 n nodes, n primitives) and what
  * the build found. */
@@ -129,12 +129,17 @@ struct LayoutOut
 };
 /* levelStart[d]..levelStart[d+1]: the build ids of depth d (gpu_build's breadth-first
  * order). leafRefMap non-null (top level, one primitive per leaf): leaf refs are
- * REF_LEAF | leafRefMap[primitive] and no triangle order is written.
+ * REF_LEAF | leafRefMap[primitive], the q8 nodes' refs all carry REF_TLAS, and no
+ * triangle order is written. f32 null: the 4-wide layout alone.
  * ws: device memory of layout_workspace_bytes(nodeCount, q8 wanted), needed
  * until layout_counts (or, without it, until the stream has passed the layout). */
 size_t layout_workspace_bytes(int nodeCount, bool q8);
 hipError_t layout_device(const BuildNode* dNodes, const uint32_t* dPrims, int nodeCount, const std::vector<int>& levelStart,
 	const uint32_t* leafRefMap, const LayoutOut& out, void* ws, size_t wsBytes, hipStream_t stream);
+/* 4-wide top level over a build tree with one primitive per leaf, in one launch:
+ * node x of the build tree heads the wide node in slot x (out holds nodeCount of
+ * them; those of adopted nodes are never referred to), refs as layout_device's. */
+hipError_t layout_top(const BuildNode* dNodes, const uint32_t* dPrims, int nodeCount, const uint32_t* leafRefMap, NodeQ8* out, hipStream_t stream);
 /* What the layout found, read back from its workspace (waits for the stream). */
 struct LayoutCounts { int nF32, nQ8, depthQ8, pad; BuildNode root; };
 hipError_t layout_counts(const void* ws, LayoutCounts& out, hipStream_t stream);

@@ -17,7 +17,7 @@ struct TraceScene
 	const float4* tris = nullptr;
 	uint32_t root = 0;
 	/* two level */
-	const NodeF32* tlas = nullptr;
+	const void* tlas = nullptr;   /* NodeF32 or NodeQ8, as format */
 	uint32_t tlasRoot = 0;
 	const InstanceRec* inst = nullptr;
 	int maxStack = 0;

@@ -127,12 +127,16 @@ __device__ __forceinline__ bool is_top(uint32_t r) { return (r & REF_TLAS) && r 
 /* One 4-wide quantised node. Child planes are origin + q * 2^e per axis; per
  * node and axis b = (origin - O) / D and d = 2^e / D, so a plane lies at
  * t = q * d + b. Near and far planes are picked by the sign of D, and
- * e = 2^-20 (|b| + 255 |d|), an upper bound of the rounding of this form, is
- * subtracted from near and added to far planes: every box that the exact
- * interval [tmin, tbest] reaches is kept. Sets ref to the nearest hit child
- * (the others pushed far to near) or pops. */
+ * e = w (|b| + 255 |d|) is subtracted from near and added to far planes. With
+ * w = 2^-20 (Q8_WIDEN) that is an upper bound of the rounding of this form: every
+ * box that the exact interval [tmin, tbest] reaches is kept. The top level takes
+ * w = 2^-16 (TOP_WIDEN), for the instance transforms' rounding, as slab does.
+ * Sets ref to the nearest hit child (the others pushed far to near) or pops. */
+static constexpr float Q8_WIDEN = 9.5367431640625e-7f, TOP_WIDEN = 1.52587890625e-5f;
+__device__ __forceinline__ float widening(float d, float b, float w) { return fmaf(fabsf(d), 255.0f, fabsf(b)) * w; }
+
 template <int BLOCK>
-__device__ __forceinline__ void visit_q8(const NodeQ8& n, const Lane& L, Stack<BLOCK>& st, uint32_t& ref)
+__device__ __forceinline__ void visit_q8(const NodeQ8& n, float w, const Lane& L, Stack<BLOCK>& st, uint32_t& ref)
 {
 	const float dx = bitsf(n.qb.z) * L.inv.x;
 	const float dy = bitsf(n.qb.w) * L.inv.y;
@@ -140,9 +144,7 @@ __device__ __forceinline__ void visit_q8(const NodeQ8& n, const Lane& L, Stack<B
 	const float bx = (n.origin.x - L.O.x) * L.inv.x;
 	const float by = (n.origin.y - L.O.y) * L.inv.y;
 	const float bz = (n.origin.z - L.O.z) * L.inv.z;
-	const float ex = fmaf(fabsf(dx), 2.43186950683593750e-4f, fabsf(bx) * 9.5367431640625e-7f);   /* 255 * 2^-20, 2^-20 */
-	const float ey = fmaf(fabsf(dy), 2.43186950683593750e-4f, fabsf(by) * 9.5367431640625e-7f);
-	const float ez = fmaf(fabsf(dz), 2.43186950683593750e-4f, fabsf(bz) * 9.5367431640625e-7f);
+	const float ex = widening(dx, bx, w), ey = widening(dy, by, w), ez = widening(dz, bz, w);
 	const float bnx = bx - ex, bfx = bx + ex, bny = by - ey, bfy = by + ey, bnz = bz - ez, bfz = bz + ez;
 	const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
 	const uint32_t qnx = px ? n.qa.x : n.qa.w, qfx = px ? n.qa.w : n.qa.x;
@@ -185,37 +187,39 @@ __device__ __forceinline__ void visit_f32(const NodeF32& n, const Lane& L, Stack
 }
 
 /* Object-space ray and BLAS root of an instance. */
-__device__ __forceinline__ void enter_instance(const TraceScene& sc, int id, Lane& L, uint32_t& ref)
+__device__ __forceinline__ void enter_instance(const InstanceRec& I, int id, Lane& L, uint32_t& ref)
 {
-	const InstanceRec& I = sc.inst[id];
-	if (!(I.flags & 1u))
-	{
-		const float4 a = I.inv0, b = I.inv1, c = I.inv2;
-		const v3 wO = L.wO, wD = L.wD;
-		L.O = mk3(a.x * wO.x + a.y * wO.y + a.z * wO.z + a.w, b.x * wO.x + b.y * wO.y + b.z * wO.z + b.w, c.x * wO.x + c.y * wO.y + c.z * wO.z + c.w);
-		L.D = mk3(a.x * wD.x + a.y * wD.y + a.z * wD.z, b.x * wD.x + b.y * wD.y + b.z * wD.z, c.x * wD.x + c.y * wD.y + c.z * wD.z);
-		L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
-	}
+	const float4 a = I.inv0, b = I.inv1, c = I.inv2;
+	const v3 wO = L.wO, wD = L.wD;
+	L.O = mk3(a.x * wO.x + a.y * wO.y + a.z * wO.z + a.w, b.x * wO.x + b.y * wO.y + b.z * wO.z + b.w, c.x * wO.x + c.y * wO.y + c.z * wO.z + c.w);
+	L.D = mk3(a.x * wD.x + a.y * wD.y + a.z * wD.z, b.x * wD.x + b.y * wD.y + b.z * wD.z, c.x * wD.x + c.y * wD.y + c.z * wD.z);
+	if (I.nodes & 1u) L.O = wO, L.D = wD;
+	L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
 	L.rp = ray_setup(L.D);
 	L.inst = id;
-	L.nodes = I.nodes, L.tris = I.tris;
-	ref = I.root;
+	L.nodes = (const void*)(I.nodes & ~(uint64_t)1), L.tris = (const float4*)(I.tris & ~(uint64_t)1);
+	ref = (I.tris & 1u) ? REF_LEAF : 0u;
 }
 
-/* A top-level entry: restore the world ray if a BLAS was being walked, then
- * either enter an instance (object-space ray, BLAS root) or walk a TLAS node. */
-template <int BLOCK>
+/* Back to the world ray, for a top-level node after an instance. */
+__device__ __forceinline__ void leave_instance(Lane& L)
+{
+	if (L.inst < 0) return;
+	L.O = L.wO, L.D = L.wD;
+	L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
+	L.inst = -1;
+}
+
+/* A top-level entry: enter an instance (object-space ray, BLAS root) or walk a
+ * TLAS node with the world ray. */
+template <int FMT, int BLOCK>
 __device__ __forceinline__ void visit_top(const TraceScene& sc, Lane& L, Stack<BLOCK>& st, uint32_t& ref)
 {
-	if (L.inst >= 0)
-	{
-		L.O = L.wO, L.D = L.wD;
-		L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
-		L.inst = -1;
-	}
-	const uint32_t r = ref & ~REF_TLAS;
-	if (r & REF_LEAF) enter_instance(sc, (int)(r & REF_MASK), L, ref);
-	else visit_f32(sc.tlas[r], L, st, ref, REF_TLAS);
+	const uint32_t r = ref & REF_MASK;
+	if (ref & REF_LEAF) return enter_instance(sc.inst[r], (int)r, L, ref);
+	leave_instance(L);
+	if (FMT == FMT_Q8) visit_q8(((const NodeQ8*)sc.tlas)[r], TOP_WIDEN, L, st, ref);
+	else visit_f32(((const NodeF32*)sc.tlas)[r], L, st, ref, REF_TLAS);
 }
 
 /* Watertight test of one leaf triangle; true when an any-hit query is done. */
@@ -342,7 +346,7 @@ __device__ __forceinline__ void start_ray(const TraceScene& sc, const float4* ra
  * them. No ray feed: quad i traces ray i, so the launch needs no counters cleared.
  * Each lane keeps the best hit of its own triangles under the shared distance;
  * the quad's best is picked by (t, instance, primitive) at the end, so hits equal
- * the other loops' bit for bit. 4,096 rays: 183 -> 76 us over 20k triangles, 222 -> 99
+ * the other loops' bit for bit. 4,096 rays: 183 -> 76 us over 20k triangles, 157 -> 92
  * over 1,000 instances; a 256 x 256 wave of the Cornell box 151 -> 49 us. */
 static const int QUAD_BLOCK = 64;
 static const int QUAD_LDS_STACK = 32;
@@ -382,7 +386,7 @@ struct QuadStack
 
 /* visit_q8 with a child per lane: the same planes, widening and tests. */
 template <typename STACK>
-__device__ __forceinline__ void visit_quad(const NodeQ8* node, int c, int lane, const Lane& L, STACK& st, uint32_t& ref)
+__device__ __forceinline__ void visit_quad(const NodeQ8* node, float w, int c, int lane, const Lane& L, STACK& st, uint32_t& ref)
 {
 	const float4 mine = ((const float4*)node)[c];
 	const uint32_t child = ((const uint32_t*)&node->refs)[c];
@@ -392,9 +396,7 @@ __device__ __forceinline__ void visit_quad(const NodeQ8* node, int c, int lane, 
 	const float stepx = quad_f<QUAD_2>(mine.z), stepy = quad_f<QUAD_2>(mine.w);
 	const float dx = stepx * L.inv.x, dy = stepy * L.inv.y, dz = stepz * L.inv.z;
 	const float bx = (ox - L.O.x) * L.inv.x, by = (oy - L.O.y) * L.inv.y, bz = (oz - L.O.z) * L.inv.z;
-	const float ex = fmaf(fabsf(dx), 2.43186950683593750e-4f, fabsf(bx) * 9.5367431640625e-7f);   /* 255 * 2^-20, 2^-20 */
-	const float ey = fmaf(fabsf(dy), 2.43186950683593750e-4f, fabsf(by) * 9.5367431640625e-7f);
-	const float ez = fmaf(fabsf(dz), 2.43186950683593750e-4f, fabsf(bz) * 9.5367431640625e-7f);
+	const float ex = widening(dx, bx, w), ey = widening(dy, by, w), ez = widening(dz, bz, w);
 	const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
 	const int sh = 8 * c;
 	const auto plane = [&](uint32_t w) { return (float)((w >> sh) & 255u); };
@@ -462,31 +464,11 @@ __device__ __forceinline__ void quad_walk(const TraceScene& sc, Lane& L, STACK& 
 		if (doNode)
 		{
 			if (++steps > TRACE_MAX_STEPS) ref = REF_DONE, st.sp = 0;
-			else if (!top) visit_quad((const NodeQ8*)L.nodes + ref, c, lane, L, st, ref);
+			else if (top && (ref & REF_LEAF)) enter_instance(sc.inst[ref & REF_MASK], (int)(ref & REF_MASK), L, ref);   /* the four lanes do the same */
 			else
-			{	/* top level: the four lanes do the same */
-				if (L.inst >= 0)
-				{
-					L.O = L.wO, L.D = L.wD;
-					L.inv = mk3(safe_rcp(L.D.x), safe_rcp(L.D.y), safe_rcp(L.D.z));
-					L.inst = -1;
-				}
-				const uint32_t r = ref & ~REF_TLAS;
-				if (r & REF_LEAF) enter_instance(sc, (int)(r & REF_MASK), L, ref);
-				else
-				{
-					const NodeF32 nd = sc.tlas[r];
-					float tl, tr;
-					const bool hl = slab(nd.lxy.x, nd.lxy.y, nd.lxy.z, nd.lxy.w, nd.lrz.x, nd.lrz.y, L.O, L.inv, L.tmin, L.tbest, tl);
-					const bool hr = slab(nd.rxy.x, nd.rxy.y, nd.rxy.z, nd.rxy.w, nd.lrz.z, nd.lrz.w, L.O, L.inv, L.tmin, L.tbest, tr);
-					const uint32_t rl = nd.refs.x | REF_TLAS, rr = nd.refs.y | REF_TLAS;
-					if (hl && hr)
-					{
-						st.put(st.sp, tr < tl ? rl : rr), st.sp++;
-						ref = tr < tl ? rr : rl;
-					}
-					else ref = hl ? rl : hr ? rr : st.sp ? st.pop() : REF_DONE;
-				}
+			{
+				if (top) leave_instance(L);
+				visit_quad((const NodeQ8*)(top ? sc.tlas : L.nodes) + (ref & REF_MASK), top ? TOP_WIDEN : Q8_WIDEN, c, lane, L, st, ref);
 			}
 		}
 		if (pend == REF_DONE && is_blas_leaf(ref)) pend = ref & REF_MASK, ref = st.sp ? st.pop() : REF_DONE;
@@ -509,8 +491,9 @@ __device__ __forceinline__ void quad_walk(const TraceScene& sc, Lane& L, STACK& 
 }
 
 /* Merged loop (default): every iteration each lane tests one pending leaf
- * triangle and visits one node, both predicated, with both loads issued at
- * the top of the iteration. Lanes never wait for one another between a node
+ * triangle and visits one node of either level (or enters an instance, whose
+ * record is a node's size), both predicated, with both loads issued at the top
+ * of the iteration. Lanes never wait for one another between a node
  * phase and a leaf phase; finished lanes are refilled while rays remain. */
 template <int FMT, int MODE, bool TWO, bool COUNT>
 __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const TraceScene sc, const float4* __restrict__ rays, void* __restrict__ out,
@@ -568,13 +551,15 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 			/* issue the triangle and node loads together */
 			float4 ta, tb, tc;
 			if (doTri) ta = L.tris[3 * pend], tb = L.tris[3 * pend + 1], tc = L.tris[3 * pend + 2];
-			const bool bl = doNode && !(TWO && is_top(ref));
+			/* a node of either level, or the record of the instance being entered */
+			const bool top = TWO && is_top(ref), enter = top && (ref & REF_LEAF);
 			NodeQ8 nq;
 			NodeF32 nf;
-			if (bl)
+			if (doNode)
 			{
-				if (FMT == FMT_Q8) nq = ((const NodeQ8*)L.nodes)[ref];
-				else nf = ((const NodeF32*)L.nodes)[ref];
+				const char* const at = (const char*)(enter ? sc.inst : top ? sc.tlas : L.nodes) + (size_t)(TWO ? ref & REF_MASK : ref) * sizeof(NodeQ8);
+				if (FMT == FMT_Q8) nq = *(const NodeQ8*)at;
+				else nf = *(const NodeF32*)at;
 			}
 			if (doTri)
 			{
@@ -586,12 +571,17 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 			if (doNode)
 			{
 				if (++steps > TRACE_MAX_STEPS) { ref = REF_DONE, st.sp = 0; }
-				else if (!bl) visit_top(sc, L, st, ref);
+				else if (enter)
+				{
+					const InstanceRec I = FMT == FMT_Q8 ? __builtin_bit_cast(InstanceRec, nq) : __builtin_bit_cast(InstanceRec, nf);
+					enter_instance(I, (int)(ref & REF_MASK), L, ref);
+				}
 				else
 				{
-					if (COUNT) cn++;
-					if (FMT == FMT_Q8) visit_q8(nq, L, st, ref);
-					else visit_f32(nf, L, st, ref, 0u);
+					if (COUNT && !top) cn++;
+					if (TWO && top) leave_instance(L);
+					if (FMT == FMT_Q8) visit_q8(nq, top ? TOP_WIDEN : Q8_WIDEN, L, st, ref);
+					else visit_f32(nf, L, st, ref, top ? REF_TLAS : 0u);
 				}
 			}
 			if (pend == REF_DONE && is_blas_leaf(ref)) pend = ref & REF_MASK, ref = st.sp ? st.pop() : REF_DONE;
@@ -605,7 +595,7 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 	{	/* The wave's last rays (at most 16), four lanes each: quad q takes the q-th lane that still holds one. With
 		 * the feed dry a launch lasts until its longest rays end, and a step costs a wave the same for one ray as
 		 * for 64; the quads' steps have half the instructions. 1 M rays towards area lights over 1,000 instances
-		 * 764 -> 689 us, 2 M incoherent rays over 4 M triangles 1,100 -> 1,068 us (12 rays instead of 16: the
+		 * (under a binary top level) 764 -> 689 us, 2 M incoherent rays over 4 M triangles 1,100 -> 1,068 us (12 rays instead of 16: the
 		 * same within 2%; the ray's state moves by lane shuffles and the LDS stack stays where it is, so the
 		 * main loop keeps its registers). */
 		uint64_t m = __ballot(active);
@@ -623,7 +613,7 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const
 		if (!mine) return;
 		uint32_t root;
 		start_ray<TWO>(sc, rays, (uint32_t)rayIdx, L, root);
-		if (TWO && inst >= 0) enter_instance(sc, inst, L, root);
+		if (TWO && inst >= 0) enter_instance(sc.inst[inst], inst, L, root);
 		L.tbest = tbest, L.bU = U, L.bV = V, L.bdet = det, L.binst = binst, L.bprim = bprim;
 		quad_walk<MODE, TWO>(sc, L, qs, ref, pend, steps, c, lane, tbest);
 		if (c == 0) write_result<MODE>(L, out, rayIdx);
@@ -710,11 +700,11 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 6 : 8) k_trace_greedy(const
 				if (wantNode)
 				{
 					if (++steps > TRACE_MAX_STEPS) { ref = REF_DONE, st.sp = 0; }
-					else if (TWO && is_top(ref)) visit_top(sc, L, st, ref);
+					else if (TWO && is_top(ref)) visit_top<FMT>(sc, L, st, ref);
 					else
 					{
 						if (COUNT) cn++;
-						if (FMT == FMT_Q8) visit_q8(((const NodeQ8*)L.nodes)[ref], L, st, ref);
+						if (FMT == FMT_Q8) visit_q8(((const NodeQ8*)L.nodes)[ref], Q8_WIDEN, L, st, ref);
 						else visit_f32(((const NodeF32*)L.nodes)[ref], L, st, ref, 0u);
 					}
 				}
@@ -792,11 +782,11 @@ __global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 6 : 8) k_trace_ww(const Tra
 				if (!(is_inner(ref) || (top && leaf == REF_DONE))) break;
 				COUNT_WAVE(true, wn, wl);
 				if (++steps > TRACE_MAX_STEPS) { ref = REF_DONE, leaf = REF_DONE, st.sp = 0; break; }
-				if (top) visit_top(sc, L, st, ref);
+				if (top) visit_top<FMT>(sc, L, st, ref);
 				else
 				{
 					if (COUNT) cn++;
-					if (FMT == FMT_Q8) visit_q8(((const NodeQ8*)L.nodes)[ref], L, st, ref);
+					if (FMT == FMT_Q8) visit_q8(((const NodeQ8*)L.nodes)[ref], Q8_WIDEN, L, st, ref);
 					else visit_f32(((const NodeF32*)L.nodes)[ref], L, st, ref, 0u);
 				}
 				if (leaf == REF_DONE && is_blas_leaf(ref)) leaf = ref, ref = st.sp ? st.pop() : REF_DONE;
@@ -936,11 +926,11 @@ static void launch1(const TraceScene& s, int mode, const float4* rays, void* out
 /* Launches of at most this many rays take four lanes per ray. Incoherent
  * closest hits, us, a lane per ray / four lanes:
  *   rays      20k triangles   1M triangles   1,000 instances
- *   1,024        172 / 72        208 / 104       202 / 79
- *   16,384       212 / 106       259 / 161       245 / 130
- *   131,072      260 / 188       301 / 238       328 / 255
- *   262,144      278 / 266       340 / 355       323 / 400
- *   524,288      301 / 452       413 / 608       465 / 699 */
+ *   1,024        172 / 72        208 / 104       151 / 71
+ *   16,384       212 / 106       259 / 161       163 / 92
+ *   131,072      260 / 188       301 / 238       232 / 207
+ *   262,144      278 / 266       340 / 355       228 / 315
+ *   524,288      301 / 452       413 / 608       287 / 544 */
 static const int QUAD_MAX_RAYS = 1 << 17;
 
 template <int MODE>
