@@ -474,6 +474,29 @@ __device__ __forceinline__ void acc_add(float4* a, v3 c)
 	*a = v;
 }
 
+/* Queue position -> path of a primary wave: bands of 4 image rows in tiles of
+ * 8 x 4 pixels (the last tile of a band as wide as is left; the paths past the
+ * last whole band in order), so that the 32 rays a wave takes at a time, and their
+ * bounces after them, share nodes, triangles and texels: k_shadeF at 1080p 229 -> 202
+ * us, a session's frame 2.78 -> 2.72 ms, 12 jobs of 512 x 384 10.36 -> 10.14 ms (the
+ * traversal itself takes the same). Small frames keep image order: at 256 x 256 the
+ * divisions cost more than they bring (16 Cornell frames 5.97 -> 5.99 ms). */
+__device__ __forceinline__ uint32_t tile_order(uint32_t j, uint32_t n, uint32_t w)
+{
+	if (n <= 131072u) return j;
+	const uint32_t band = 4 * w, b = j / band;
+	if ((b + 1) * band > n) return j;
+	const uint32_t k = j - b * band, whole = w >> 3;
+	uint32_t x, y;
+	if (k < whole * 32) x = (k >> 5) * 8 + (k & 7), y = (k >> 3) & 3;
+	else
+	{
+		const uint32_t r = w & 7, q = k - whole * 32;
+		y = q / r, x = whole * 8 + (q - y * r);
+	}
+	return b * band + y * w + x;
+}
+
 __global__ void k_generate(CamParams c, uint32_t R0, uint32_t jobBase, int n, float eps, float4* __restrict__ rays,
 	float4* __restrict__ state, uint32_t* __restrict__ pathId, float4* __restrict__ pathAcc, uint32_t* __restrict__ counters,
 	uint32_t slotBase, uint32_t total, int storeSlot)
@@ -481,14 +504,14 @@ __global__ void k_generate(CamParams c, uint32_t R0, uint32_t jobBase, int n, fl
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
 	if (j == 0 && slotBase == 0) counters[0] = total, counters[2] = 0, counters[3] = 0;
 	if (j >= n) return;
-	const uint32_t job = jobBase + (uint32_t)j;
+	const uint32_t path = tile_order((uint32_t)j, (uint32_t)n, (uint32_t)c.w), job = jobBase + path;
 	const uint32_t o = slotBase + (uint32_t)j;
 	v3 O, D;
 	eye_ray(c, (int)job, R0, O, D);
 	rays[2 * o] = make_float4(O.x, O.y, O.z, eps);
 	rays[2 * o + 1] = make_float4(D.x, D.y, D.z, 1e34f);
 	state[o] = make_float4(1.0f, 1.0f, 1.0f, bitsf(S_SPECULAR));
-	pathId[o] = storeSlot ? o : job;
+	pathId[o] = storeSlot ? slotBase + path : job;
 	pathAcc[o] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
@@ -860,7 +883,7 @@ __global__ void k_generate7(CamParams c, ShadeParams P, uint32_t jobBase, int n,
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
 	if (j == 0 && slotBase == 0) counters[0] = total, counters[2] = 0, counters[3] = 0;
 	if (j >= n) return;
-	const uint32_t pathIdx = jobBase + (uint32_t)j;
+	const uint32_t path = tile_order((uint32_t)j, (uint32_t)n, (uint32_t)c.w), pathIdx = jobBase + path;
 	const uint32_t o = slotBase + (uint32_t)j;
 	const uint32_t wh = (uint32_t)(c.w * c.h);
 	const uint32_t pixelIdx = pathIdx % wh, sampleIdx = pathIdx / wh + (uint32_t)P.pass;
@@ -899,7 +922,7 @@ __global__ void k_generate7(CamParams c, ShadeParams P, uint32_t jobBase, int n,
 	rays[2 * o + 1] = make_float4(D.x, D.y, D.z, 1e34f);
 	state[o] = make_float4(1.0f, 1.0f, 1.0f, bitsf(S7_SPECULAR));
 	aux[o] = make_float2(1.0f, bitsf(0u));
-	pathId[o] = storeSlot ? o : pathIdx;
+	pathId[o] = storeSlot ? slotBase + path : pathIdx;
 	pathAcc[o] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
@@ -1131,7 +1154,7 @@ __global__ void k_generateF(CamParams c, ShadeParams P, uint32_t jobBase, int n,
 	const int j = blockIdx.x * blockDim.x + threadIdx.x;
 	if (j == 0 && slotBase == 0) counters[0] = total, counters[2] = 0, counters[3] = 0;
 	if (j >= n) return;
-	const uint32_t pathIdx = jobBase + (uint32_t)j;
+	const uint32_t path = tile_order((uint32_t)j, (uint32_t)n, (uint32_t)c.w), pathIdx = jobBase + path;
 	const uint32_t o = slotBase + (uint32_t)j;
 	const uint32_t wh = (uint32_t)(c.w * c.h);
 	const uint32_t pixelIdx = pathIdx % wh, sampleIdx = pathIdx / wh + (uint32_t)P.pass;
@@ -1159,7 +1182,7 @@ __global__ void k_generateF(CamParams c, ShadeParams P, uint32_t jobBase, int n,
 	rays[2 * o + 1] = make_float4(D.x, D.y, D.z, 1e34f);
 	state[o] = make_float4(1.0f, 1.0f, 1.0f, bitsf(SF_SPECULAR));
 	aux[o] = make_float2(1.0f, bitsf(0u));
-	pathId[o] = storeSlot ? o : pathIdx;
+	pathId[o] = storeSlot ? slotBase + path : pathIdx;
 	pathAcc[o] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	pathAcc[o + total] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }

@@ -81,3 +81,25 @@ def test_bounce_block_edges(torch_cuda, n):
     assert np.array_equal(p2.cpu().numpy()[:m][order].astype(np.uint32), np.sort(want_id))
     assert np.array_equal(r2.cpu().numpy()[:m][order].view(np.uint32), want[np.argsort(want_id)].view(np.uint32))
     core.Shutdown()
+
+
+@pytest.mark.parametrize("w,h,spp", [(362, 363, 1), (5, 26300, 1), (131100, 1, 1), (181, 363, 2)])
+@pytest.mark.parametrize("estimator", [0, 1])
+def test_tile_order_covers_every_path(torch_cuda, w, h, spp, estimator):
+    """Frames of more than 131,072 paths start in tiles of 8 x 4 pixels: ragged widths and last bands, an image narrower
+    than a tile, a band longer than the image, bands across two samples."""
+    s = scenes.cornell_box(sphere_tris=400)
+    view = scenes.cornell_view(w, h)
+    core = lh.RenderCore()
+    lh.load_scene(core, s)
+    core.SetTarget(w, h, spp)
+    for k, v in (("estimator", estimator), ("epsilon", 1e-3), ("maxDepth", 3)):
+        core.Setting(k, v)
+    core.Render(view, lh.LH2_RESTART)
+    acc = core.read_accumulator_f64()
+    core.Shutdown()
+    if estimator == 0:
+        ref = orc.render(s, view, w, h, spp, 1, 3, 1e-3, modes=[orc.RESTART])[1]
+    else:
+        ref = orc.render7(s, view, w, h, spp, 1, threads=16, modes=[orc.RESTART])[1]
+    assert np.array_equal(acc, ref)
