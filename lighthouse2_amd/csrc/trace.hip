@@ -144,8 +144,8 @@ __device__ __forceinline__ void visit_q8(const NodeQ8& n, float w, const Lane& L
 	const float bx = (n.origin.x - L.O.x) * L.inv.x;
 	const float by = (n.origin.y - L.O.y) * L.inv.y;
 	const float bz = (n.origin.z - L.O.z) * L.inv.z;
-	const float ex = widening(dx, bx, w), ey = widening(dy, by, w), ez = widening(dz, bz, w);
-	const float bnx = bx - ex, bfx = bx + ex, bny = by - ey, bfy = by + ey, bnz = bz - ez, bfz = bz + ez;
+	const float sx = fmaf(fabsf(dx), 255.0f, fabsf(bx)), sy = fmaf(fabsf(dy), 255.0f, fabsf(by)), sz = fmaf(fabsf(dz), 255.0f, fabsf(bz));
+	const float bnx = fmaf(-w, sx, bx), bfx = fmaf(w, sx, bx), bny = fmaf(-w, sy, by), bfy = fmaf(w, sy, by), bnz = fmaf(-w, sz, bz), bfz = fmaf(w, sz, bz);
 	const bool px = L.inv.x >= 0.0f, py = L.inv.y >= 0.0f, pz = L.inv.z >= 0.0f;
 	const uint32_t qnx = px ? n.qa.x : n.qa.w, qfx = px ? n.qa.w : n.qa.x;
 	const uint32_t qny = py ? n.qa.y : n.qb.x, qfy = py ? n.qb.x : n.qa.y;
@@ -157,7 +157,7 @@ __device__ __forceinline__ void visit_q8(const NodeQ8& n, float w, const Lane& L
 	{
 		const float tn = fmaxf(fmaxf(fmaf(ubyte(qnx, c), dx, bnx), fmaf(ubyte(qny, c), dy, bny)), fmaxf(fmaf(ubyte(qnz, c), dz, bnz), L.tmin));
 		const float tf = fminf(fminf(fmaf(ubyte(qfx, c), dx, bfx), fmaf(ubyte(qfy, c), dy, bfy)), fminf(fmaf(ubyte(qfz, c), dz, bfz), L.tbest));
-		tk[c] = (rk[c] != Q8_EMPTY && tn <= tf) ? tn : __builtin_huge_valf();
+		tk[c] = ((c < 2 || rk[c] != Q8_EMPTY) && tn <= tf) ? tn : __builtin_huge_valf();
 	}
 	cswap(tk[0], tk[1], rk[0], rk[1]);
 	cswap(tk[2], tk[3], rk[2], rk[3]);
@@ -494,9 +494,13 @@ __device__ __forceinline__ void quad_walk(const TraceScene& sc, Lane& L, STACK& 
  * triangle and visits one node of either level (or enters an instance, whose
  * record is a node's size), both predicated, with both loads issued at the top
  * of the iteration. Lanes never wait for one another between a node
- * phase and a leaf phase; finished lanes are refilled while rays remain. */
+ * phase and a leaf phase; finished lanes are refilled while rays remain.
+ *   Bound by VALU issue (85% of it at 2.1 M primary rays over 1,000 instances).
+ * Five waves per SIMD: single-level closest hits take 81 registers (2 M incoherent
+ * rays over 4 M triangles 1,005 us, 1,068 with six waves and a spill in the loop),
+ * two-level ones 95 (2 M: 741 us, six waves 1,056, four 779). */
 template <int FMT, int MODE, bool TWO, bool COUNT>
-__global__ void __launch_bounds__(TRACE_BLOCK, TWO ? 5 : 6) k_trace_merged(const TraceScene sc, const float4* __restrict__ rays, void* __restrict__ out,
+__global__ void __launch_bounds__(TRACE_BLOCK, 5) k_trace_merged(const TraceScene sc, const float4* __restrict__ rays, void* __restrict__ out,
 	int maxCount, const uint32_t* __restrict__ countDev, uint32_t* __restrict__ queue, uint32_t* __restrict__ overflow, TraceStats* __restrict__ stats)
 {
 	__shared__ uint32_t sstack[TRACE_LDS_STACK * TRACE_BLOCK];
