@@ -180,7 +180,7 @@ __device__ __forceinline__ uint32_t relu_mask2(uint32_t act, uint32_t g)
  *   Measured at 1920 x 1088 (a wave per row -> now; the bytes each must move at a
  * copy's 5.06 TB/s): 16 -> 32 58 -> 42 us (40), 32 -> 32 76 -> 44 (53, partly from the
  * cache), 32 -> 32 with pooling 117 -> 65 (59), 64 -> 32 175 -> 81 (59), 32 -> 16 float
- * 49 -> 37 (53), display 71 -> 42; gradients 32 -> 32 110 -> 88 (79), 32 -> 64 187 -> 101
+ * 49 -> 37 (53), display 71 -> 51; gradients 32 -> 32 110 -> 88 (79), 32 -> 64 187 -> 101
  * (66). Memory bounds all but the 64-channel ones, which wait for it between their
  * tiles' products as well. */
 template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL, int IO, int MBW>
