@@ -457,9 +457,9 @@ void RenderCore::SetGeometry(const int meshIdx, const lighthouse2::float4* verte
 	/* The records go up on the second stream, by a thread of their own beside the build when they are many: the build
 	 * needs the vertices alone, and a pageable copy keeps a host thread busy (500k triangles: the copy takes 3.5 ms and
 	 * the build 2.2 ms, 7.3 -> 4.0 ms for the call). 4 MB take 0.15 ms, several times a thread's start. */
-	Joined copier;
 	uint32_t maxMaterial = 0;
 	hipError_t copied = hipSuccess;
+	Joined copier;                                                /* last: joined before what its thread writes goes */
 	const size_t recordBytes = triangles ? sizeof(CoreTri) * (size_t)triangleCount : 0;
 	if (recordBytes)
 	{
@@ -570,7 +570,9 @@ void RenderCore::FinalizeInstances()
  * 1080p session's frame 3.45 -> 2.80 ms).
  * fp32 nodes serve both levels where quantised boxes will not do: a transform
  * without a usable inverse (singular: the object-space ray is the world ray and
- * the exact box alone keeps it out), or wide nodes too deep for the stack. */
+ * the exact box alone keeps it out), or wide nodes too deep for the stack
+ * (1,000,001 closest hits over 1,000 instances: q8 465 us, fp32 628, q8 under a
+ * binary top level 737). */
 void RenderCore::updateTopLevel()
 {
 	if (!instancesDirty) return;
