@@ -117,7 +117,13 @@ LH2HIP_API int lh2hip_get_stats(lh2hip_core* core, CoreStats* out);
 LH2HIP_API int lh2hip_plugin_read_image(void* core, lh2_float4* hostOut);
 LH2HIP_API int lh2hip_plugin_read_accumulator_f64(void* core, double* hostOut);
 
-/* ---- traversal queries (OptiX Prime rtpQueryExecute replacement) ---------- */
+/* ---- traversal queries (OptiX Prime rtpQueryExecute replacement) ----------
+ * Asynchronous on `stream`. The queries of a core run one after the other,
+ * whatever their streams (they share the ray feed and the stacks' overflow
+ * area), and beside no frame of lh2hip_render; a scene update called after a
+ * query takes effect once the query is done. A query captured into a graph is
+ * outside this order: its replays must not run beside other queries or frames of
+ * the core, and every later scene update waits for the whole device. */
 
 /* Closest hit, RTP_QUERY_TYPE_CLOSEST (lib/RenderCore_PrimeRef/rendercore.cpp:559-573;
  * rendercore_optix7/optix/.optix.cu:125-140,174-184). rays/hits are device

@@ -199,6 +199,8 @@ void RenderCore::Init()
 	hipCheck(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking), "hipStreamCreate");
 	for (int i = 0; i < 2 + 2 * SIDE_TIMED; i++)
 		hipCheck(i < 2 ? hipEventCreateWithFlags(&sideEv[i], hipEventDisableTiming) : hipEventCreate(&sideEv[i]), "hipEventCreate");
+	hipCheck(hipEventCreateWithFlags(&queryEv, hipEventDisableTiming), "hipEventCreate");
+	hipCheck(hipEventCreateWithFlags(&frameEv, hipEventDisableTiming), "hipEventCreate");
 	sideCounters.ensure((4 + TRACE_QUEUE_WORDS) * sizeof(uint32_t));
 	overflow2.ensure(trace_overflow_bytes(persistentBlocks));
 }
@@ -218,6 +220,8 @@ void RenderCore::Shutdown()
 	svgf.reset();
 	for (int i = 0; i < 8; i++) (void)hipEventDestroy(ev[i]);
 	for (int i = 0; i < 2 + 2 * SIDE_TIMED; i++) (void)hipEventDestroy(sideEv[i]);
+	(void)hipEventDestroy(queryEv), (void)hipEventDestroy(frameEv);
+	queryPending = bouncePending = capturedQueries = framePending = false;
 	(void)hipStreamDestroy(stream2);
 	(void)hipStreamDestroy(stream);
 	stream = stream2 = nullptr;
@@ -371,6 +375,7 @@ void RenderCore::buildMesh(MeshData& m)
 	L.q8 = m.nodesQ8.as<NodeQ8>(), L.q8Map = m.dQ8Map.as<int32_t>();
 	L.order = m.dOrder.as<uint32_t>(), L.last = m.dLast.as<uint8_t>();
 	buildWs.ensure(layout_workspace_bytes(b.nodeCount, true));   /* the boxes and the builder's lists are no longer needed */
+	waitQueries();                     /* they may still walk the nodes and triangles that the layout rewrites */
 	hipCheck(layout_device(b.nodes, b.prims, b.nodeCount, b.levelStart, nullptr, L, buildWs.p, buildWs.bytes, stream), "bvh layout");
 	m.tris.ensure(sizeof(float4) * 3 * ((size_t)n + TRACE_TRI_PAD));
 	hipCheck(gather_tris(m.verts.as<float4>(), m.dOrder.as<uint32_t>(), m.dLast.as<uint8_t>(), n, m.tris.as<float4>(), stream), "gather_tris");
@@ -405,6 +410,7 @@ void RenderCore::refitMesh(MeshData& m)
 {
 	const auto t0 = std::chrono::high_resolution_clock::now();
 	hipCheck(refit_levels(m.dBuildNodes.as<BuildNode>(), m.dBuildPrims.as<uint32_t>(), m.verts.as<float4>(), m.levelStart, stream), "refit_levels");
+	waitQueries();                     /* as in buildMesh: up to here only what no query reads was written */
 	hipCheck(refit_layout(m.dBuildNodes.as<BuildNode>(), m.nodesF32.as<NodeF32>(), m.dF32Kids.as<int32_t>(), (int)m.nodeCountF32,
 		m.nodesQ8.as<NodeQ8>(), m.dQ8Map.as<int32_t>(), (int)m.nodeCountQ8, stream), "refit_layout");
 	hipCheck(gather_tris(m.verts.as<float4>(), m.dOrder.as<uint32_t>(), m.dLast.as<uint8_t>(), m.triCount, m.tris.as<float4>(), stream), "gather_tris");
@@ -482,6 +488,7 @@ void RenderCore::SetGeometry(const int meshIdx, const lighthouse2::float4* verte
 		if (!copier.t.joinable()) copied = uploadCoreTris(m, triangles, triangleCount, maxMaterial);
 	}
 	else if (!triangles) m.coreTris.release();
+	if (bouncePending) waitQueries();                             /* bounces read the vertices */
 	m.verts.upload(vertexData, sizeof(float4) * 3 * (size_t)triangleCount, stream);
 	if (refit) refitMesh(m);
 	else if (triangleCount > 0) buildMesh(m);
@@ -619,6 +626,7 @@ void RenderCore::updateTopLevel()
 		blo.push_back(make_float4(lo[0], lo[1], lo[2], 0)), bhi.push_back(make_float4(hi[0], hi[1], hi[2], 0));
 		live.push_back(i);
 	}
+	waitQueries();                     /* they read both tables and the top level's nodes */
 	shadeInsts.upload(sh.data(), sh.size() * sizeof(ShadeInst), stream);
 	int recFormat;
 	const auto uploadRecs = [&]() {
@@ -717,17 +725,44 @@ const TraceScene& RenderCore::Scene()
 	return scene;
 }
 
+/* Before a query on s: after the queries before it (they share the ray feed
+ * and the overflow area) and the frame that may still run. Waits for work of the
+ * same stream cost nothing on the device. */
+hipEvent_t RenderCore::beginQuery(hipStream_t s)
+{
+	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+	if (s && hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
+	{	/* events from outside the graph have no place in it */
+		capturedQueries = true;
+		return nullptr;
+	}
+	hipCheck(hipStreamWaitEvent(s, queryEv, 0), "wait");
+	if (framePending) hipCheck(hipStreamWaitEvent(s, frameEv, 0), "wait");
+	return queryEv;
+}
+
+void RenderCore::waitQueries()
+{
+	if (capturedQueries) hipCheck(hipDeviceSynchronize(), "sync");
+	else if (queryPending) hipCheck(hipStreamWaitEvent(stream, queryEv, 0), "wait");
+	queryPending = bouncePending = false;
+}
+
 void RenderCore::TraceClosest(const void* rays, void* hits, int count, hipStream_t s)
 {
 	if (count < 0 || (count > 0 && (!rays || !hits))) throw CoreError(LH2HIP_ERR_INVALID, "trace: bad arguments");
 	const TraceScene& sc = Scene();
-	hipCheck(launch_trace_dev(sc, MODE_CLOSEST, (const float4*)rays, hits, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s ? s : 0), "trace");
+	const hipEvent_t done = beginQuery(s);
+	hipCheck(launch_trace_dev(sc, MODE_CLOSEST, (const float4*)rays, hits, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s,
+		nullptr, done), "trace");
+	queryPending |= done && count > 0;
 }
 
 void RenderCore::TraceClosestCounted(const void* rays, void* hits, int count, hipStream_t s, uint64_t* out2)
 {
 	if (count < 0 || (count > 0 && (!rays || !hits))) throw CoreError(LH2HIP_ERR_INVALID, "trace: bad arguments");
 	const TraceScene& sc = Scene();
+	beginQuery(s);                     /* and waited for below */
 	DevBuf st;
 	st.ensure(sizeof(TraceStats));
 	hipCheck(hipMemsetAsync(st.p, 0, sizeof(TraceStats), s), "memset");
@@ -748,16 +783,21 @@ void RenderCore::TraceAny(const void* rays, uint32_t* mask, int count, hipStream
 {
 	if (count < 0 || (count > 0 && (!rays || !mask))) throw CoreError(LH2HIP_ERR_INVALID, "trace: bad arguments");
 	const TraceScene& sc = Scene();
+	const hipEvent_t done = beginQuery(s);
 	hipCheck(hipMemsetAsync(mask, 0, sizeof(uint32_t) * ((count + 31) / 32), s), "memset");
-	hipCheck(launch_trace_dev(sc, MODE_ANY_MASK, (const float4*)rays, mask, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s ? s : 0), "trace");
+	hipCheck(launch_trace_dev(sc, MODE_ANY_MASK, (const float4*)rays, mask, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s,
+		nullptr, done), "trace");
+	queryPending |= done && count > 0;
 }
 
 void RenderCore::Bounce(const void* raysIn, const void* hits, const uint32_t* pathIn, int count, uint32_t R0, float tmin,
 	void* raysOut, uint32_t* pathOut, uint32_t* countOut, hipStream_t s)
 {
 	Scene();
+	const hipEvent_t done = beginQuery(s);
 	hipCheck(launch_bounce(shadeInsts.as<ShadeInst>(), (const float4*)raysIn, (const float4*)hits, pathIn, count, R0, tmin,
-		(float4*)raysOut, pathOut, countOut, s), "bounce");
+		(float4*)raysOut, pathOut, countOut, s, done), "bounce");
+	if (done && count > 0) queryPending = bouncePending = true;
 }
 
 void RenderCore::BvhInfo(int mesh, int64_t* o) const
@@ -1239,6 +1279,7 @@ void RenderCore::Render(const ViewPyramid& view, const Convergence converge, boo
 	updateTopLevel();
 	if (!sceneReady) return; /* no geometry yet: nothing to render (rendercore_optix7/rendercore.cpp:821) */
 	checkRenderable();
+	waitQueries();                     /* the frame's traversals use the same overflow area */
 	const auto t0 = std::chrono::high_resolution_clock::now();
 	bool fresh = false;   /* the frame's first pass writes the accumulators (no clear needed) */
 	if (converge == Restart || firstConvergingFrame)
@@ -1292,7 +1333,9 @@ void RenderCore::Render(const ViewPyramid& view, const Convergence converge, boo
 		hipCheck(launch_finalize(wf.acc32(), pixels, 1.0f / (float)samplesTaken, wf.image(), stream), "finalize");
 	}
 	prevView = view;
-	if (!async)
+	framePending = async;
+	if (async) hipCheck(hipEventRecord(frameEv, stream), "event");
+	else
 	{
 		hipCheck(hipStreamSynchronize(stream), "sync");
 		int probe[3];
@@ -1318,7 +1361,7 @@ void RenderCore::Render(const ViewPyramid& view, const Convergence converge, boo
 
 void RenderCore::WaitForRender()
 {
-	if (stream) hipCheck(hipStreamSynchronize(stream), "sync");
+	if (stream) hipCheck(hipStreamSynchronize(stream), "sync"), framePending = false;
 }
 
 void RenderCore::ReadImage(void* hostOut)

@@ -241,6 +241,17 @@ private:
 	int persistentBlocks = 0;
 	float minRaysPerLane = 0.0f;       /* 0: always launch persistentBlocks */
 	int blocksFor(int count) const;
+	/* Order between the core's streams and the caller's. Queries run on the
+	 * caller's stream and read the trees and instance tables (Bounce also the
+	 * vertices), which scene updates rewrite in place on `stream`, and they
+	 * share the ray feed and the stacks' overflow area with each other and
+	 * (the overflow area) with frames. queryEv follows the last query, frameEv
+	 * the last frame that was not waited for. A query captured into a graph
+	 * may be replayed at any time: updates then wait for the whole device. */
+	hipEvent_t queryEv = nullptr, frameEv = nullptr;
+	bool queryPending = false, bouncePending = false, capturedQueries = false, framePending = false;
+	hipEvent_t beginQuery(hipStream_t s);   /* the event to record at the query's end; null: s is being captured */
+	void waitQueries();                /* `stream` goes on once the queries launched so far are done */
 	/* settings (RenderCore_PrimeRef rendercore.cpp:484-502 + extensions) */
 	float geometryEpsilon = 1.0e-3f, clampValue = 10.0f;
 	int maxDepth = 64, nodeFormat = FMT_Q8, traceLoop = LOOP_MERGED, triBias = 16, refillLanes = 16, chunk = 32;

@@ -43,9 +43,11 @@ struct TraceStats
 hipError_t launch_trace(const TraceScene& s, int mode, const float4* rays, void* out, int count,
 	uint32_t* queue, uint32_t* overflow, int persistentBlocks, hipStream_t stream, TraceStats* statsDev = nullptr);
 /* As launch_trace, with the ray count read by the kernel from countDev
- * (device memory) and maxCount an upper bound: no host round trip. */
+ * (device memory) and maxCount an upper bound: no host round trip. done (if
+ * given): an event recorded as the traversal's end. */
 hipError_t launch_trace_dev(const TraceScene& s, int mode, const float4* rays, void* out, int maxCount, const uint32_t* countDev,
-	uint32_t* queue, uint32_t* overflow, int persistentBlocks, hipStream_t stream, TraceStats* statsDev = nullptr);
+	uint32_t* queue, uint32_t* overflow, int persistentBlocks, hipStream_t stream, TraceStats* statsDev = nullptr,
+	hipEvent_t done = nullptr);
 size_t trace_overflow_bytes(int persistentBlocks);
 
 static const int TRACE_TRI_PAD = 3;                 /* records that may be read (and are ignored) past a mesh's last leaf triangle */

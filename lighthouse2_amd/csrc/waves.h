@@ -24,7 +24,8 @@ struct ShadeInst
 };
 
 hipError_t launch_primary(const CamParams& c, uint32_t R0, float tmin, float4* rays, uint32_t* pathId, hipStream_t s);
+/* done (if given): an event recorded as the kernel's end. */
 hipError_t launch_bounce(const ShadeInst* inst, const float4* raysIn, const float4* hits, const uint32_t* pathIn, int n,
-	uint32_t R0, float tmin, float4* raysOut, uint32_t* pathOut, uint32_t* counter, hipStream_t s);
+	uint32_t R0, float tmin, float4* raysOut, uint32_t* pathOut, uint32_t* counter, hipStream_t s, hipEvent_t done = nullptr);
 
 } // namespace lh
