@@ -49,6 +49,11 @@ def layer_specs():
     return spec
 
 
+_SPECS = layer_specs()
+_INPUT = {"e1": "in", "e2": "a", "d1": "b", "d2": "c"}      # a layer's input and output activation at its level
+_OUTPUT = {"e1": "a", "e2": "b", "d1": "c", "d2": "d"}
+
+
 def init_params(seed=0):
     """He-normal weights [9][Cout][Cin] and zero biases (float32, numpy)."""
     rng = np.random.default_rng(seed)
@@ -87,7 +92,6 @@ class UNetDenoiser:
             d["wf"] = torch.zeros(9 * co * ci, **bf)
             d["wb"] = torch.zeros(9 * co * ci, **bf)
             self.p[name] = d
-        self._tensors = self._tensor_table(grads=True)
         self._cast()
         # activations per level (kept for the backward pass) and the gradients of
         # what each layer adds up before its ReLU (kept for the weight gradients)
@@ -105,37 +109,32 @@ class UNetDenoiser:
         self.out = torch.zeros(H * W * COUT, **f32)
         self.dout = torch.zeros(H * W * COUT, **bf)
         self.loss = torch.zeros(1, **f32)
-        self._layers = self._layer_table()
-        need = int(library().lh2hip_dn_dw_batch_workspace_bytes(self._layers, len(self._layers)))
+        need = int(library().lh2hip_dn_dw_batch_workspace_bytes(*self._layer_table()))
         self.ws = torch.zeros(need // 4, **f32)    # empty (and the backward pass refused) beyond the weight gradient's sizes
 
     # ---- helpers --------------------------------------------------------
+    # Both tables are made for each call: a program may have put other tensors into p, a or g since the last one.
     def _tensor_table(self, grads):
-        """Every weight and bias for one Adam launch; without gradients: the weights' bf16 copies only."""
+        """Every weight and bias for one Adam launch, and their number; without gradients: the weights' bf16 copies only."""
         rows = []
         for d in self.p.values():
-            for k in ("w", "b") if grads else ("w",):
-                rows.append(_Tensor(d[k].data_ptr(), d["m" + k].data_ptr(), d["v" + k].data_ptr(), d["g" + k].data_ptr() if grads else None,
-                                    d["wf"].data_ptr() if k == "w" else None, d["wb"].data_ptr() if k == "w" else None, d[k].numel(),
-                                    d["co"], d["ci"]))
-        return (_Tensor * len(rows))(*rows)
+            w = d["w"]
+            rows.append((w.data_ptr(), d["mw"].data_ptr(), d["vw"].data_ptr(), d["gw"].data_ptr() if grads else None, d["wf"].data_ptr(),
+                         d["wb"].data_ptr(), w.numel(), d["co"], d["ci"]))
+            if grads:
+                b = d["b"]
+                rows.append((b.data_ptr(), d["mb"].data_ptr(), d["vb"].data_ptr(), d["gb"].data_ptr(), None, None, b.numel(), 0, 0))
+        return (_Tensor * len(rows))(*rows), len(rows)
 
     def _layer_table(self):
-        """Inputs and output gradients of the 19 convolutions, for one weight-gradient launch."""
-        rows = []
-        for name, ci, co in layer_specs():
-            lvl = 0 if name == "out" else int(name[-1])
-            coarse = None
-            if name == "out":
-                x, gy = self.a["d_0"], self.dout
-            else:
-                x = self.a[{"e1": "in", "e2": "a", "d1": "b", "d2": "c"}[name[:2]] + f"_{lvl}"]
-                gy = self.g[{"e1": "a", "e2": "b", "d1": "c", "d2": "d"}[name[:2]] + f"_{lvl}"]
-                if name[:2] == "d1":
-                    coarse = self._below(lvl).data_ptr()
-            d = self.p[name]
-            rows.append(_Layer(x.data_ptr(), coarse, gy.data_ptr(), d["gw"].data_ptr(), d["gb"].data_ptr(), ci, co, self.H >> lvl, self.W >> lvl))
-        return (_Layer * len(rows))(*rows)
+        """Inputs and output gradients of the 19 convolutions for one weight-gradient launch, and their number."""
+        a, g, rows = self.a, self.g, []
+        for name, ci, co in _SPECS:
+            d, kind, lvl = self.p[name], name[:2], 0 if name == "out" else int(name[-1])
+            x, gy = (a["d_0"], self.dout) if name == "out" else (a[_INPUT[kind] + name[2:]], g[_OUTPUT[kind] + name[2:]])
+            rows.append((x.data_ptr(), self._below(lvl).data_ptr() if kind == "d1" else None, gy.data_ptr(), d["gw"].data_ptr(), d["gb"].data_ptr(),
+                         ci, co, self.H >> lvl, self.W >> lvl))
+        return (_Layer * len(rows))(*rows), len(rows)
 
     def _below(self, lvl, grad=False):
         """The tensor a decoder level upsamples (or its gradient)."""
@@ -143,8 +142,7 @@ class UNetDenoiser:
         return t[f"d_{lvl + 1}"] if lvl + 1 < LEVELS - 1 else t[f"b_{LEVELS - 1}"]
 
     def _cast(self):
-        t = self._tensor_table(grads=False)
-        _check(library().lh2hip_dn_adam_batch(t, len(t), 0.0, 0.9, 0.999, 1e-8, 1, self.sh))
+        _check(library().lh2hip_dn_adam_batch(*self._tensor_table(grads=False), 0.0, 0.9, 0.999, 1e-8, 1, self.sh))
 
     def _conv(self, x, name, y, h, w, flags):
         d = self.p[name]
@@ -219,13 +217,13 @@ class UNetDenoiser:
             if lvl > 0:
                 d = self.p[f"e1_{lvl}"]
                 _check(L.lh2hip_dn_conv3x3(g[f"a_{lvl}"].data_ptr(), CH, d["wb"].data_ptr(), None, g[f"in_{lvl}"].data_ptr(), CH, h, w, 0, self.sh))
-        _check(L.lh2hip_dn_conv3x3_dw_batch(self._layers, len(self._layers), self.ws.data_ptr(), self.ws.numel() * 4, self.sh))
+        _check(L.lh2hip_dn_conv3x3_dw_batch(*self._layer_table(), self.ws.data_ptr(), self.ws.numel() * 4, self.sh))
         return self.loss
 
     def step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         """One Adam step on every parameter (also refreshes the bf16 copies)."""
         self.t += 1
-        _check(library().lh2hip_dn_adam_batch(self._tensors, len(self._tensors), lr, b1, b2, eps, self.t, self.sh))
+        _check(library().lh2hip_dn_adam_batch(*self._tensor_table(grads=True), lr, b1, b2, eps, self.t, self.sh))
 
     def weights_blob(self):
         """The network's inference weights as one blob (the job server's

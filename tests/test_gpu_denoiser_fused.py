@@ -189,3 +189,45 @@ def test_row_tiles_equal_small_tiles(torch_cuda, H, W):
             for k, (f, p) in enumerate(zip(full, part)):
                 q = 1 if k < 4 else 2
                 assert torch.equal(f[(y0 + t) // q:(y0 + e) // q, (x0 + l) // q:(x0 + r) // q], p[t // q:e // q, l // q:r // q]), (k, y0, x0)
+
+
+def test_replaced_tensors_are_the_ones_used(torch_cuda):
+    """Entries of the network's dictionaries replaced by other tensors: a step does what it does after copying into the old ones."""
+    torch = torch_cuda
+    H, W = 32, 48
+    rng = np.random.default_rng(12)
+    f = lambda *s: torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda()
+    inputs, target = (f(H, W, 4).abs(), f(H, W, 4).abs(), f(H, W, 4), f(H, W).abs()), f(H, W, 4)
+    nets = [D.UNetDenoiser(H, W, seed=5) for _ in range(2)]
+    old = []
+
+    def put(net, at, key, value):
+        if net is nets[0]:
+            at[key].copy_(value.view(at[key].shape))
+        else:
+            old.append((at[key], at[key].clone()))
+            at[key] = value.clone().view(at[key].shape)
+
+    new = {}
+    for name, ci, co in D.layer_specs():
+        for k, shape in (("w", (9, co, ci)), ("b", (co,))):
+            new[name, k] = f(*shape) * 0.1
+            new[name, "m" + k], new[name, "v" + k], new[name, "g" + k] = f(*shape) * 0.01, f(*shape).abs() * 0.01, f(*shape)
+    for net in nets:
+        for (name, k), t in new.items():
+            put(net, net.p[name], k, t)
+        net._cast()
+        for d in (net.a, net.g):
+            for k in list(d):
+                put(net, d, k, torch.zeros_like(d[k]))
+        put(net, vars(net), "dout", torch.zeros_like(net.dout))
+        net.set_input(*inputs)
+        net.forward()
+        net.loss_backward(target)
+        net.step(lr=1e-2)
+    torch.cuda.synchronize()
+    for name, ci, co in D.layer_specs():
+        for k in nets[0].p[name]:
+            a, b = nets[0].p[name][k], nets[1].p[name][k]
+            assert a == b if isinstance(a, int) else torch.equal(a, b), (name, k)
+    assert all(torch.equal(t, was) for t, was in old)
