@@ -1203,24 +1203,28 @@ __global__ void k_pool2_bwd8(const bf16_t* __restrict__ dy, int gs, int W, bf16_
 }
 
 /* the gradient of an encoder level's second activation: the skip connection's gradient plus a
- * quarter of the pooled tensor's (k_pool2_bwd8, accumulating), then the ReLU gradient, in one pass */
-__global__ void k_pool2_bwd_relu8(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ skip, const bf16_t* __restrict__ act, int gs, int W,
+ * quarter of the pooled tensor's (k_pool2_bwd8, accumulating), then the ReLU gradient, in one pass
+ * (images of more rows than a grid has: a block takes several) */
+__global__ void k_pool2_bwd_relu8(const bf16_t* __restrict__ dy, const bf16_t* __restrict__ skip, const bf16_t* __restrict__ act, int gs, int H, int W,
 	bf16_t* __restrict__ out)
 {
-	const int j = blockIdx.x * blockDim.x + threadIdx.x, G = 1 << gs, py = blockIdx.y;
+	const int j = blockIdx.x * blockDim.x + threadIdx.x, G = 1 << gs;
 	if (j >= W * G) return;
 	const int px = j >> gs, c8 = j & (G - 1);
-	const size_t at = ((size_t)py * W + px) * (8 * G) + 8 * c8;
-	const u16x8 d = ld8(dy + ((size_t)(py >> 1) * (W >> 1) + (px >> 1)) * (8 * G) + 8 * c8), prev = ld8(skip + at), a = ld8(act + at);
-	u16x8 r;
-#pragma unroll
-	for (int k = 0; k < 8; k++)
+	for (int py = blockIdx.y; py < H; py += gridDim.y)
 	{
-		float v = bf2f(d[k]) * 0.25f;
-		v += bf2f(prev[k]);
-		r[k] = bf2f(a[k]) > 0.0f ? f2bf(v) : (unsigned short)0;
+		const size_t at = ((size_t)py * W + px) * (8 * G) + 8 * c8;
+		const u16x8 d = ld8(dy + ((size_t)(py >> 1) * (W >> 1) + (px >> 1)) * (8 * G) + 8 * c8), prev = ld8(skip + at), a = ld8(act + at);
+		u16x8 r;
+#pragma unroll
+		for (int k = 0; k < 8; k++)
+		{
+			float v = bf2f(d[k]) * 0.25f;
+			v += bf2f(prev[k]);
+			r[k] = bf2f(a[k]) > 0.0f ? f2bf(v) : (unsigned short)0;
+		}
+		st8(out + at, r);
 	}
-	st8(out + at, r);
 }
 
 __global__ void k_pool2_8(const bf16_t* __restrict__ x, int gs, int W, bf16_t* __restrict__ y)
@@ -1383,10 +1387,10 @@ hipError_t dn_pool2_bwd(const bf16_t* dy, int C, int H, int W, bf16_t* dx, int a
 
 hipError_t dn_pool2_bwd_relu(const bf16_t* dy, const bf16_t* skip, const bf16_t* act, int C, int H, int W, bf16_t* out, hipStream_t s)
 {
-	if (H % 2 || W % 2 || H <= 0 || W <= 0 || H > 65535) return hipErrorInvalidValue;
+	if (H % 2 || W % 2 || H <= 0 || W <= 0) return hipErrorInvalidValue;
 	const int gs = C <= 0 || C % 8 ? -1 : log2_exact(C / 8);
 	if (gs < 0 || !aligned16_3(dy, skip, act) || !aligned16(out)) return hipErrorInvalidValue;
-	k_pool2_bwd_relu8<<<row_grid(W << gs, H), 256, 0, s>>>(dy, skip, act, gs, W, out);
+	k_pool2_bwd_relu8<<<row_grid(W << gs, H < 65535 ? H : 65535), 256, 0, s>>>(dy, skip, act, gs, H, W, out);
 	return hipGetLastError();
 }
 

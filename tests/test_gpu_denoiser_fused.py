@@ -231,3 +231,27 @@ def test_replaced_tensors_are_the_ones_used(torch_cuda):
             a, b = nets[0].p[name][k], nets[1].p[name][k]
             assert a == b if isinstance(a, int) else torch.equal(a, b), (name, k)
     assert all(torch.equal(t, was) for t, was in old)
+
+
+def test_images_taller_than_a_grid(torch_cuda):
+    """65,552 rows: pool2_bwd_relu equals its parts, and a training step runs."""
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    H, W = 65552, 16
+    rng = np.random.default_rng(2)
+    rnd = lambda n: dev(torch, R.bf16(rng.standard_normal(n)))
+    for C, w in ((8, 2), (32, W)):
+        dy, skip, act, out = rnd(H * w * C // 4), rnd(H * w * C), rnd(H * w * C), empty(torch, H * w * C)
+        assert L.lh2hip_dn_pool2_bwd_relu(dy.data_ptr(), skip.data_ptr(), act.data_ptr(), C, H, w, out.data_ptr(), sh) == 0
+        assert L.lh2hip_dn_pool2_bwd(dy.data_ptr(), C, H, w, skip.data_ptr(), 1, sh) == 0
+        assert L.lh2hip_dn_relu_bwd(act.data_ptr(), skip.data_ptr(), skip.data_ptr(), H * w * C, sh) == 0
+        assert torch.equal(out, skip), C
+    net = D.UNetDenoiser(H, W, seed=1)
+    f = lambda *s: torch.rand(s, device="cuda", generator=torch.Generator("cuda").manual_seed(3))
+    before = net.p["e1_0"]["w"].clone()
+    net.set_input(f(H, W, 4), f(H, W, 4), f(H, W, 4), f(H, W))
+    net.forward()
+    loss = net.loss_backward(f(H, W, 4))
+    net.step()
+    assert torch.isfinite(loss).all() and not torch.equal(net.p["e1_0"]["w"], before) and torch.isfinite(net.p["e1_0"]["w"]).all()
