@@ -221,7 +221,7 @@ void RenderCore::Shutdown()
 	for (int i = 0; i < 8; i++) (void)hipEventDestroy(ev[i]);
 	for (int i = 0; i < 2 + 2 * SIDE_TIMED; i++) (void)hipEventDestroy(sideEv[i]);
 	(void)hipEventDestroy(queryEv), (void)hipEventDestroy(frameEv);
-	queryPending = bouncePending = capturedQueries = framePending = false;
+	queryPending = queryRecorded = bouncePending = capturedQueries = framePending = false;
 	(void)hipStreamDestroy(stream2);
 	(void)hipStreamDestroy(stream);
 	stream = stream2 = nullptr;
@@ -736,7 +736,7 @@ hipEvent_t RenderCore::beginQuery(hipStream_t s)
 		capturedQueries = true;
 		return nullptr;
 	}
-	hipCheck(hipStreamWaitEvent(s, queryEv, 0), "wait");
+	if (queryRecorded) hipCheck(hipStreamWaitEvent(s, queryEv, 0), "wait");
 	if (framePending) hipCheck(hipStreamWaitEvent(s, frameEv, 0), "wait");
 	return queryEv;
 }
@@ -755,7 +755,7 @@ void RenderCore::TraceClosest(const void* rays, void* hits, int count, hipStream
 	const hipEvent_t done = beginQuery(s);
 	hipCheck(launch_trace_dev(sc, MODE_CLOSEST, (const float4*)rays, hits, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s,
 		nullptr, done), "trace");
-	queryPending |= done && count > 0;
+	if (done && count > 0) queryPending = queryRecorded = true;
 }
 
 void RenderCore::TraceClosestCounted(const void* rays, void* hits, int count, hipStream_t s, uint64_t* out2)
@@ -787,7 +787,7 @@ void RenderCore::TraceAny(const void* rays, uint32_t* mask, int count, hipStream
 	hipCheck(hipMemsetAsync(mask, 0, sizeof(uint32_t) * ((count + 31) / 32), s), "memset");
 	hipCheck(launch_trace_dev(sc, MODE_ANY_MASK, (const float4*)rays, mask, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s,
 		nullptr, done), "trace");
-	queryPending |= done && count > 0;
+	if (done && count > 0) queryPending = queryRecorded = true;
 }
 
 void RenderCore::Bounce(const void* raysIn, const void* hits, const uint32_t* pathIn, int count, uint32_t R0, float tmin,
@@ -797,7 +797,7 @@ void RenderCore::Bounce(const void* raysIn, const void* hits, const uint32_t* pa
 	const hipEvent_t done = beginQuery(s);
 	hipCheck(launch_bounce(shadeInsts.as<ShadeInst>(), (const float4*)raysIn, (const float4*)hits, pathIn, count, R0, tmin,
 		(float4*)raysOut, pathOut, countOut, s, done), "bounce");
-	if (done && count > 0) queryPending = bouncePending = true;
+	if (done && count > 0) queryPending = queryRecorded = bouncePending = true;
 }
 
 void RenderCore::BvhInfo(int mesh, int64_t* o) const

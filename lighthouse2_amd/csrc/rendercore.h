@@ -249,7 +249,7 @@ private:
 	 * the last frame that was not waited for. A query captured into a graph
 	 * may be replayed at any time: updates then wait for the whole device. */
 	hipEvent_t queryEv = nullptr, frameEv = nullptr;
-	bool queryPending = false, bouncePending = false, capturedQueries = false, framePending = false;
+	bool queryPending = false, queryRecorded = false, bouncePending = false, capturedQueries = false, framePending = false;
 	hipEvent_t beginQuery(hipStream_t s);   /* the event to record at the query's end; null: s is being captured */
 	void waitQueries();                /* `stream` goes on once the queries launched so far are done */
 	/* settings (RenderCore_PrimeRef rendercore.cpp:484-502 + extensions) */
