@@ -19,6 +19,7 @@
  * scan bit for bit.
  */
 #include "trace.h"
+#include "trace_stack.h"
 #include <hip/hip_ext.h>
 #include <algorithm>
 #include <map>
@@ -55,54 +56,6 @@ __device__ __forceinline__ bool slab(float lx, float hx, float ly, float hy, flo
 	tnear = tn;
 	return tn <= tf;
 }
-
-/* An LDS pointer typed as such, so that loads through it stay LDS loads. */
-typedef __attribute__((address_space(3))) uint32_t lds_u32;
-
-template <int BLOCK>
-struct Stack
-{
-	lds_u32* lds;       /* TRACE_LDS_STACK x BLOCK */
-	uint32_t* ovf;      /* this thread's overflow area */
-	int tid, sp;
-	/* The host checks that the tree depth fits TRACE_MAX_STACK; a push beyond
-	 * it is dropped (never written out of bounds). */
-	__device__ __forceinline__ void push(uint32_t v)
-	{
-		if (sp < TRACE_LDS_STACK) lds[sp * BLOCK + tid] = v, sp++;
-		else if (sp < TRACE_MAX_STACK) ovf[sp - TRACE_LDS_STACK] = v, sp++;
-	}
-	/* Pushes c (bottom) if hc, then b if hb, then a (top) if ha. With room
-	 * for three entries in LDS, every lane writes all three slots and only
-	 * moves its stack pointer for the pushed ones: no divergent branch. */
-	__device__ __forceinline__ void push3(uint32_t c, bool hc, uint32_t b, bool hb, uint32_t a, bool ha)
-	{
-		if (sp + 3 <= TRACE_LDS_STACK)
-		{
-			lds[sp * BLOCK + tid] = c;
-			sp += hc ? 1 : 0;
-			lds[sp * BLOCK + tid] = b;
-			sp += hb ? 1 : 0;
-			lds[sp * BLOCK + tid] = a;
-			sp += ha ? 1 : 0;
-		}
-		else
-		{
-			if (hc) push(c);
-			if (hb) push(b);
-			if (ha) push(a);
-		}
-	}
-	/* LDS read for every lane (the row clamped into the LDS part), the
-	 * overflow area read only by lanes below it. */
-	__device__ __forceinline__ uint32_t pop()
-	{
-		sp--;
-		uint32_t v = lds[min(sp, TRACE_LDS_STACK - 1) * BLOCK + tid];
-		if (sp >= TRACE_LDS_STACK) v = ovf[sp - TRACE_LDS_STACK];
-		return v;
-	}
-};
 
 /* Sort up to 4 (tnear, ref) pairs ascending (misses carry +inf). */
 __device__ __forceinline__ void cswap(float& a, float& b, uint32_t& ra, uint32_t& rb)
@@ -363,28 +316,6 @@ __device__ __forceinline__ uint32_t quad_bits(uint64_t m, int lane)
 	return ((lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32)) >> (lane & 28)) & 15u;
 }
 
-/* One stack per ray, entries written by the quad's lanes: DEPTH in LDS
- * (interleaved over STRIDE rays), the others in the ray's overflow area. */
-template <int DEPTH, int STRIDE>
-struct QuadStack
-{
-	lds_u32* lds;
-	uint32_t* ovf;
-	int col, sp;
-	__device__ __forceinline__ void put(int at, uint32_t v)
-	{
-		if (at < DEPTH) lds[at * STRIDE + col] = v;
-		else if (at < TRACE_MAX_STACK) ovf[at - DEPTH] = v;
-	}
-	__device__ __forceinline__ uint32_t pop()
-	{
-		sp--;
-		uint32_t v = lds[min(sp, DEPTH - 1) * STRIDE + col];
-		if (sp >= DEPTH) v = ovf[sp - DEPTH];
-		return v;
-	}
-};
-
 /* visit_q8 with a child per lane: the same planes, widening and tests. */
 template <typename STACK>
 __device__ __forceinline__ void visit_quad(const NodeQ8* node, float w, int c, int lane, const Lane& L, STACK& st, uint32_t& ref)
@@ -418,7 +349,7 @@ __device__ __forceinline__ void visit_quad(const NodeQ8* node, float w, int c, i
 	const uint32_t first = min(min(key, k1), min(k2, k3)) & 3u, far = first ^ (uint32_t)c;
 	const uint32_t r1 = quad_u<QUAD_X1>(child), r2 = quad_u<QUAD_X2>(child), r3 = quad_u<QUAD_X3>(child);
 	if (hit && rank > 0) st.put(st.sp + n - rank, child);
-	st.sp += n;
+	st.grow(n);
 	__builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* another lane of the quad may pop it */
 	ref = far < 2 ? (far == 0 ? child : r1) : (far == 2 ? r2 : r3);
 }
