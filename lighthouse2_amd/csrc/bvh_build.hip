@@ -382,8 +382,8 @@ __global__ void __launch_bounds__(256) k_big_decide(BuildArgs A, int d)
 	}
 }
 
-/* Partition of the level's big nodes into the other buffer, a block per chunk:
- * one atomic per chunk and side reserves its places. Children that are big get
+/* Partition of the level's big nodes into the other buffer (a leaf's primitives
+ * to the output), a block per chunk: one atomic per chunk and side reserves its places. Children that are big get
  * their centroid bounds here. */
 __global__ void __launch_bounds__(256) k_big_part(BuildArgs A, int d)
 {
@@ -463,6 +463,7 @@ __global__ void __launch_bounds__(256) k_big_part(BuildArgs A, int d)
 			const uint64_t bmL = __ballot(left), bmR = __ballot(in && !left), mine = left ? bmL : bmR;
 			const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mine >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mine, 0u));
 			if (in && mode >= 0) A.buf[par ^ 1][(mode == 3 ? p : (left ? atL : atR) + rank)] = prim[k];
+			else if (in) A.out[p] = prim[k];
 			atL += __popcll(bmL), atR += __popcll(bmR);
 		}
 		__syncthreads();

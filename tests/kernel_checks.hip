@@ -1,6 +1,9 @@
 /* kernel_checks.hip - entry points for tests of what the C ABI does not reach:
- * the traversal's stacks (run on the host). Built beside the library into tests/bin/libkernel_checks.so. */
+ * the traversal's stacks (run on the host) and the builder with leaves of any size.
+ * Built beside the library into tests/bin/libkernel_checks.so. */
 #include "../lighthouse2_amd/csrc/trace_stack.h"
+#include "../lighthouse2_amd/csrc/bvh.h"
+#include <cstring>
 #include <vector>
 
 using namespace lh;
@@ -68,4 +71,18 @@ CHECK_API int check_stack(int which, uint32_t seed, int grow)
 	return run_stack(st, TRACE_LDS_STACK * TRACE_BLOCK, TRACE_OVF_STACK, seed, grow, [](Stack<TRACE_BLOCK>& s, const uint32_t* e, int n) {
 		s.push3(e[0], true, n > 1 ? e[1] : 0, n > 1, n > 2 ? e[2] : 0, n > 2);
 	});
+}
+
+/* ---- builder ------------------------------------------------------------------
+ * gpu_build over n device boxes; nodes (2 n) and prims (n) are device memory,
+ * wsBytes of them at ws (0: how many it needs, returned). Returns the node count,
+ * or minus the error. */
+CHECK_API int64_t check_build(const float4* lo, const float4* hi, int n, int maxLeaf, int maxDegenerateLeaf, BuildNode* nodes, uint32_t* prims, void* ws,
+	uint64_t wsBytes)
+{
+	if (wsBytes == 0) return (int64_t)gpu_build_workspace_bytes(n);
+	DeviceBuild b;
+	b.nodes = nodes, b.prims = prims;
+	const hipError_t e = gpu_build(lo, hi, n, maxLeaf, maxDegenerateLeaf, b, ws, (size_t)wsBytes, nullptr);
+	return e == hipSuccess ? b.nodeCount : -(int64_t)e;
 }
