@@ -460,32 +460,36 @@ void RenderCore::SetGeometry(const int meshIdx, const lighthouse2::float4* verte
 	const bool refit = refitSetting && triangleCount > 0 && m.triCount == triangleCount && m.buildNodeCount > 0;
 	m.triCount = triangleCount;
 	m.maxMaterial = -1;
-	/* The records go up on the second stream, by a thread of their own beside the build when they are many: the build
-	 * needs the vertices alone, and a pageable copy keeps a host thread busy (500k triangles: the copy takes 3.5 ms and
-	 * the build 2.2 ms, 7.3 -> 4.0 ms for the call). 4 MB take 0.15 ms, several times a thread's start. */
+	/* Many records (4 MB and more) go up on the second stream, by a thread of their own beside the build: the build needs
+	 * the vertices alone, and a pageable copy keeps a host thread busy (500k triangles: the copy takes 3.5 ms and the build
+	 * 2.2 ms, 7.3 -> 4.0 ms for the call). 4 MB take 0.15 ms, several times a thread's start. Fewer follow on the same
+	 * stream, their largest material found on the host while they travel: a kernel, its read-back and their wait cost a
+	 * small refit more than that (1,000 triangles 130 -> 78 us, 5,000 180 -> 144). */
 	uint32_t maxMaterial = 0;
 	hipError_t copied = hipSuccess;
 	Joined copier;                                                /* last: joined before what its thread writes goes */
 	const size_t recordBytes = triangles ? sizeof(CoreTri) * (size_t)triangleCount : 0;
-	if (recordBytes)
+	if (recordBytes >= ((size_t)4 << 20))
 	{
 		m.coreTris.ensure(recordBytes), maxMatB.ensure(sizeof(uint32_t));
 		hipCheck(hipEventRecord(sideEv[0], stream), "event");      /* frames still reading the old records */
 		hipCheck(hipStreamWaitEvent(stream2, sideEv[0], 0), "event");
-		if (recordBytes >= ((size_t)4 << 20))
+		int dev = 0;
+		hipCheck(hipGetDevice(&dev), "hipGetDevice");
+		try
 		{
-			int dev = 0;
-			hipCheck(hipGetDevice(&dev), "hipGetDevice");
-			try
-			{
-				copier.t = std::thread([&, dev] {
-					copied = hipSetDevice(dev);
-					if (copied == hipSuccess) copied = uploadCoreTris(m, triangles, triangleCount, maxMaterial);
-				});
-			}
-			catch (const std::system_error&) {}                   /* no thread to be had */
+			copier.t = std::thread([&, dev] {
+				copied = hipSetDevice(dev);
+				if (copied == hipSuccess) copied = uploadCoreTris(m, triangles, triangleCount, maxMaterial);
+			});
 		}
+		catch (const std::system_error&) {}                       /* no thread to be had */
 		if (!copier.t.joinable()) copied = uploadCoreTris(m, triangles, triangleCount, maxMaterial);
+	}
+	else if (recordBytes)
+	{
+		m.coreTris.upload(triangles, recordBytes, stream);
+		for (int i = 0; i < triangleCount; i++) maxMaterial = std::max(maxMaterial, (uint32_t)triangles[i].material);
 	}
 	else if (!triangles) m.coreTris.release();
 	if (bouncePending) waitQueries();                             /* bounces read the vertices */
