@@ -1031,9 +1031,14 @@ __global__ void __launch_bounds__(256) k_dw_reduce(const DwBatch B, const float*
 
 /* Jobs of a list of layers: chunk heights (the same for all layers: enough
  * chunks for 8,192 waves, each at least 8 rows: fewer waves leave compute units
- * idle at the end, shorter chunks re-read two rows of their neighbours' input),
- * block and workspace ranges; taller chunks where the partial sums would exceed
- * maxFloats. false: a shape that is not supported. */
+ * idle at the end, shorter chunks re-read two rows of their neighbours' input;
+ * lists of few segment rows, a single layer of a small image among them, take 2 or
+ * 4, as a block's walk is then the whole time), block and workspace ranges; taller
+ * chunks where the partial sums would exceed maxFloats. One layer 32 -> 32, us with
+ * chunks of 8 / 4 / 2 rows: 64 x 64 (128 segment rows) 19.5 / 14.9 / 13.0, 128 x 192
+ * (768) 19.7 / 15.5 / 14.8, 160 x 256 (1,280) 20.0 / 16.4 / 16.4, 256 x 256 (2,048) 20.4 /
+ * 17.8 / 18.9, 272 x 480 (4,080) 22.9 / 22.1 / 25.7, 544 x 960 (16,320) 34.4 / 53.6. (Before
+ * all layers shared a launch: 12.9, 15.8, 18.1, 22.6, 42.6 and 73.9.) false: a shape that is not supported. */
 static bool dw_plan(const DwLayer* L, int layers, size_t maxFloats, DwBatch& B, size_t& floats, int& blocks, int& outs)
 {
 	B.n = 0;
@@ -1063,7 +1068,8 @@ static bool dw_plan(const DwLayer* L, int layers, size_t maxFloats, DwBatch& B, 
 			tallest = tallest > l.H ? tallest : l.H;
 		}
 	}
-	int rows = (int)(steps / 8192 < 8 ? 8 : steps / 8192 < tallest ? steps / 8192 : tallest);
+	const int least = steps <= 1280 ? 2 : steps < 4096 ? 4 : 8;
+	int rows = (int)(steps / 8192 < least ? least : steps / 8192 < tallest ? steps / 8192 : tallest);
 	while (true)
 	{
 		blocks = outs = 0, floats = 0;

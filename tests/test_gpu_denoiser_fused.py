@@ -255,3 +255,20 @@ def test_images_taller_than_a_grid(torch_cuda):
     loss = net.loss_backward(f(H, W, 4))
     net.step()
     assert torch.isfinite(loss).all() and not torch.equal(net.p["e1_0"]["w"], before) and torch.isfinite(net.p["e1_0"]["w"]).all()
+
+
+@pytest.mark.parametrize("H,W", [(161, 250), (163, 250), (521, 250), (527, 258)])
+def test_weight_gradient_chunk_heights(torch_cuda, H, W):
+    """Sizes whose chunks are 4 and 8 rows high (2 in the tests above), with a short last chunk."""
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(H)
+    for cin, cout in ((32, 32), (64, 32), (16, 16)):
+        x, gy = R.bf16(rng.standard_normal((H, W, cin))), R.bf16(rng.standard_normal((H, W, cout)))
+        dx, dgy = dev(torch, x), dev(torch, gy)
+        ws = torch.zeros(int(L.lh2hip_dn_dw_workspace_bytes(cin, cout)) // 4, device="cuda")
+        gw, gb = torch.full((9 * cout * cin,), 7.0, device="cuda"), torch.full((cout,), 7.0, device="cuda")
+        assert L.lh2hip_dn_conv3x3_dw(dx.data_ptr(), cin, dgy.data_ptr(), cout, H, W, gw.data_ptr(), gb.data_ptr(), ws.data_ptr(), sh) == 0
+        torch.cuda.synchronize()
+        check_dw(torch, x, gy, gw, gb, (cin, cout, H, W))
