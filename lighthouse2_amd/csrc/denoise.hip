@@ -657,14 +657,15 @@ __global__ void __launch_bounds__(256) k_conv3x3_t(const bf16_t* __restrict__ x,
 	}
 }
 
-/* Images with fewer than SMALL_TILES 64-pixel-wide tiles of 4 rows run 4 x 16
- * tiles, a wave per row: four to eight times the blocks, so that a small layer
- * spreads over more compute units instead of running at the latency of a few
- * blocks (128 x 128, 64 such tiles: 4.6 against 6.3 us for 32 -> 32 with pooling, 6.7
- * against 10.3 for the concatenation; 240 x 144, 144 tiles: 6.3 and 6.4, 14.7 and
- * 11.1). */
-static const int SMALL_TILES = 128;
-static bool small_image(int H, int W) { return ((W + 63) / 64) * ((H + 3) / 4) < SMALL_TILES; }
+/* Images with few 64-pixel-wide tiles of 4 rows run 4 x 16 tiles, a wave per row:
+ * four to eight times the blocks, so that a small layer spreads over more compute
+ * units instead of running at the latency of a few blocks. The line is 128 such
+ * tiles (128 x 128, 64 tiles: 4.6 against 6.3 us for 32 -> 32 with pooling, 6.7 against
+ * 10.3 for the concatenation; 240 x 144, 144 tiles: 6.3 and 6.4, 14.7 and 11.1), and
+ * 256 for layers of at most half of 32 -> 32's weights, which wait less for them at
+ * each tap (16 -> 32 at 144, 192, 252 and 260 tiles: 4.5 against 5.5, 4.8 and 5.8, 5.4 and 5.9,
+ * 5.4 and 5.9; 32 -> 16 3.9 and 4.6, 3.9 and 4.7, 4.6 and 4.7, 4.7 and 4.8). */
+static bool small_image(int H, int W, int weights) { return ((W + 63) / 64) * ((H + 3) / 4) < (weights <= 512 ? 256 : 128); }
 
 
 /* The tiled convolution with the tile that suits the image. Large ones: 32 x 16
@@ -677,7 +678,7 @@ static hipError_t conv_tile(const bf16_t* x, const bf16_t* coarse, const bf16_t*
 	constexpr int MBW = NB == 4 || (CIN == 64 && !CAT) ? 1 : 2, TX = 16 * MBW;
 	const int across = (W + TX - 1) / TX, tiles = across * ((H + 15) / 16);
 	const int blocks = (NB == 4 || CIN == 64) && tiles > 512 ? 512 : (tiles + 7) & ~7;   /* two a CU walk the tiles; or one a tile, a multiple of the XCDs */
-	if (small_image(H, W))
+	if (small_image(H, W, CIN * NB * 16))
 		k_conv3x3_t<CIN, NB, RELU, F32OUT, CAT, POOL, IO><<<dim3((W + 15) / 16, (H + 3) / 4), 256, 0, s>>>(x, coarse, w, bias, y, H, W, ypool, io, act);
 	else
 		k_conv_rows<CIN, NB, RELU, F32OUT, CAT, POOL, IO, MBW><<<blocks, 256, 0, s>>>(x, coarse, w, bias, y, H, W,

@@ -272,3 +272,31 @@ def test_weight_gradient_chunk_heights(torch_cuda, H, W):
         assert L.lh2hip_dn_conv3x3_dw(dx.data_ptr(), cin, dgy.data_ptr(), cout, H, W, gw.data_ptr(), gb.data_ptr(), ws.data_ptr(), sh) == 0
         torch.cuda.synchronize()
         check_dw(torch, x, gy, gw, gb, (cin, cout, H, W))
+
+
+@pytest.mark.parametrize("H,W", [(126, 254), (250, 254), (254, 256)])
+def test_light_layers_on_both_sides_of_their_line(torch_cuda, H, W):
+    """16 -> 32 and 32 -> 16 take small tiles up to 255 tiles of 64 x 4 (here 128, 252 and 256): equal to crops of 28 x 28, bit for bit."""
+    torch = torch_cuda
+    L = lh.library()
+    sh = torch.cuda.current_stream().cuda_stream
+    rng = np.random.default_rng(H + W)
+    x = R.bf16(rng.standard_normal((H, W, 32)))
+    w = dev(torch, R.bf16(rng.standard_normal((9, 32, 16)) * 0.2))
+    b = torch.from_numpy(rng.standard_normal(32).astype(np.float32)).cuda()
+
+    def run(y0, x0, h, w_):
+        cut = x[y0:y0 + h, x0:x0 + w_]
+        a16, a32 = dev(torch, np.ascontiguousarray(cut[..., :16])), dev(torch, np.ascontiguousarray(cut))
+        o = empty(torch, h * w_ * 32), torch.full((h * w_ * 16,), 7.0, device="cuda")
+        assert L.lh2hip_dn_conv3x3(a16.data_ptr(), 16, w.data_ptr(), b.data_ptr(), o[0].data_ptr(), 32, h, w_, 1, sh) == 0
+        assert L.lh2hip_dn_conv3x3(a32.data_ptr(), 32, w.data_ptr(), b.data_ptr(), o[1].data_ptr(), 16, h, w_, 2, sh) == 0
+        torch.cuda.synchronize()
+        return o[0].view(h, w_, 32), o[1].view(h, w_, 16)
+
+    full = run(0, 0, H, W)
+    for y0 in (0, H // 2 - 11, H - 28):
+        for x0 in (0, W // 2 - 13, W - 28):
+            t, l, e, r = (1 if y0 else 0), (1 if x0 else 0), 28 - (y0 + 28 < H), 28 - (x0 + 28 < W)
+            for f, p in zip(full, run(y0, x0, 28, 28)):
+                assert torch.equal(f[y0 + t:y0 + e, x0 + l:x0 + r], p[t:e, l:r]), (y0, x0)
