@@ -242,23 +242,6 @@ __device__ __forceinline__ ConstF4 as_const(const float4* p) { return (ConstF4)p
 
 /* dot product with its two adds fused into the products */
 __device__ __forceinline__ float fdot3(v3 a, v3 b) { return fmaf(a.z, b.z, fmaf(a.y, b.y, a.x * b.x)); }
-/* 1 / x and sqrt(x), correctly rounded, for x in [2^-100, 2^100): there the
- * compiler's sequences need neither scaling nor fix-up, and one step from the
- * hardware's estimate is enough (every float of that range compared: the same
- * bits; 3 and 6 instructions instead of 11 and 18). With 64 lights the potentials
- * are most of a path's shading: k_shadeF at 1080p 202 -> 184 us. */
-__device__ __forceinline__ float rcp_tame(float x)
-{
-	const float r = __builtin_amdgcn_rcpf(x);
-	return fmaf(fmaf(-x, r, 1.0f), r, r);
-}
-__device__ __forceinline__ float sqrt_tame(float x)
-{
-	const float y = __builtin_amdgcn_rsqf(x), s = x * y;
-	return fmaf(fmaf(-s, s, x), 0.5f * y, s);
-}
-static constexpr float TAME_MAX = 1.2676506e30f;   /* 2^100 */
-
 /* A triangle light's potential seen along Lv (light point - shading point):
  * energy max(0, -LN.L) max(0, N.L) / |Lv|^2 with L = Lv / |Lv|, its dot
  * products fused. TAME: as the tame functions; span keeps the largest |Lv|^2 and

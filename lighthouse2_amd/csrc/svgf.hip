@@ -252,34 +252,6 @@ __global__ void k_prepare(const float4* __restrict__ acc, const uint4* __restric
 	moments[p] = make_float4(lumD, lumD2, lumI, lumI2);
 }
 
-/* n / d by the operations that the compiler emits for a correctly rounded
- * division, without the scaling and the fix-up: the same bits for d in
- * [1e-5, 1e30] except where n / d overflows (NaN here) or n is close to
- * denormal (an ulp), and a tap's weight is the same 0, or unchanged, in both. */
-__device__ __forceinline__ float div_core(float n, float d)
-{
-	const float r0 = __builtin_amdgcn_rcpf(d);
-	const float r = fmaf(fmaf(-d, r0, 1.0f), r0, r0);
-	const float q0 = n * r;
-	const float q1 = fmaf(fmaf(-d, q0, n), r, q0);
-	return fmaf(fmaf(-d, q1, n), r, q1);
-}
-
-/* cw_expf for x <= 0 or NaN (its scale by ldexp: the same rounding) */
-__device__ __forceinline__ float exp_neg(float x)
-{
-	const float k = floorf(fmaf(x, 1.44269504f, 0.5f));
-	const float r = fmaf(k, 2.12194440e-4f, fmaf(-k, 0.693359375f, x));
-	float p = fmaf(r, 1.9841270e-4f, 1.3888889e-3f);
-	p = fmaf(p, r, 8.3333333e-3f);
-	p = fmaf(p, r, 4.1666668e-2f);
-	p = fmaf(p, r, 0.16666667f);
-	p = fmaf(p, r, 0.5f);
-	p = fmaf(p, r, 1.0f);
-	p = fmaf(p, r, 1.0f);
-	return x < -87.0f ? 0.0f : ldexpf(p, (int)k);
-}
-
 /* applyFilterKernel (finalize_shared.h:320-477), pass with tap distance STEP.
  *
  * VALU-bound: 20 taps per pixel, each of which unpacked two colours, a normal and

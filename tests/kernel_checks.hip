@@ -1,9 +1,10 @@
 /* kernel_checks.hip - entry points for tests of what the C ABI does not reach:
- * the traversal's stacks (run on the host) and the builder with leaves of any size.
+ * the traversal's stacks (run on the host), the builder with leaves of any size and
+ * the short forms of the math functions.
  * Built beside the library into tests/bin/libkernel_checks.so. */
 #include "../lighthouse2_amd/csrc/trace_stack.h"
 #include "../lighthouse2_amd/csrc/bvh.h"
-#include <cstring>
+#include "../lighthouse2_amd/csrc/lh_math.h"
 #include <vector>
 
 using namespace lh;
@@ -85,4 +86,19 @@ CHECK_API int64_t check_build(const float4* lo, const float4* hi, int n, int max
 	b.nodes = nodes, b.prims = prims;
 	const hipError_t e = gpu_build(lo, hi, n, maxLeaf, maxDegenerateLeaf, b, ws, (size_t)wsBytes, nullptr);
 	return e == hipSuccess ? b.nodeCount : -(int64_t)e;
+}
+
+/* ---- short math ---------------------------------------------------------------
+ * out[i] of n device floats: 0 rcp_tame(a), 1 sqrt_tame(a), 2 div_core(a, b), 3 exp_neg(a), 4 cw_expf(a). */
+__global__ void k_short(int which, const float* a, const float* b, float* out, int n)
+{
+	for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+		out[i] = which == 0 ? rcp_tame(a[i]) : which == 1 ? sqrt_tame(a[i]) : which == 2 ? div_core(a[i], b[i]) : which == 3 ? exp_neg(a[i]) : cw_expf(a[i]);
+}
+
+CHECK_API int check_short(int which, const float* a, const float* b, float* out, int n)
+{
+	if (n <= 0 || which < 0 || which > 4 || !a || !out || (which == 2 && !b)) return (int)hipErrorInvalidValue;
+	k_short<<<4096, 256>>>(which, a, b, out, n);
+	return (int)hipGetLastError();
 }
