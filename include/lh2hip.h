@@ -121,7 +121,8 @@ LH2HIP_API int lh2hip_plugin_read_accumulator_f64(void* core, double* hostOut);
  * Asynchronous on `stream`. The queries of a core run one after the other,
  * whatever their streams (they share the ray feed and the stacks' overflow
  * area), and beside no frame of lh2hip_render; a scene update called after a
- * query takes effect once the query is done. A query captured into a graph is
+ * query takes effect once the query is done (on the null stream: once that stream
+ * has done what it holds). A query captured into a graph is
  * outside this order: its replays must not run beside other queries or frames of
  * the core, and every later scene update waits for the whole device. */
 

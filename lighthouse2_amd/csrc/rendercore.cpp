@@ -202,6 +202,7 @@ void RenderCore::Init()
 	hipCheck(hipEventCreateWithFlags(&queryEv, hipEventDisableTiming), "hipEventCreate");
 	hipCheck(hipEventCreateWithFlags(&frameEv, hipEventDisableTiming), "hipEventCreate");
 	sideCounters.ensure((4 + TRACE_QUEUE_WORDS) * sizeof(uint32_t));
+	hipCheck(hipMemsetAsync(sideCounters.p, 0, sideCounters.bytes, stream), "memset");
 	overflow2.ensure(trace_overflow_bytes(persistentBlocks));
 }
 
@@ -221,7 +222,7 @@ void RenderCore::Shutdown()
 	for (int i = 0; i < 8; i++) (void)hipEventDestroy(ev[i]);
 	for (int i = 0; i < 2 + 2 * SIDE_TIMED; i++) (void)hipEventDestroy(sideEv[i]);
 	(void)hipEventDestroy(queryEv), (void)hipEventDestroy(frameEv);
-	queryPending = queryRecorded = bouncePending = capturedQueries = framePending = false;
+	queryPending = queryOnNull = queryRecorded = bouncePending = capturedQueries = framePending = false;
 	(void)hipStreamDestroy(stream2);
 	(void)hipStreamDestroy(stream);
 	stream = stream2 = nullptr;
@@ -730,25 +731,42 @@ const TraceScene& RenderCore::Scene()
 }
 
 /* Before a query on s: after the queries before it (they share the ray feed
- * and the overflow area) and the frame that may still run. Waits for work of the
- * same stream cost nothing on the device. */
-hipEvent_t RenderCore::beginQuery(hipStream_t s)
+ * and the overflow area) and the frame that may still run. */
+RenderCore::QueryMark RenderCore::beginQuery(hipStream_t s)
 {
 	hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
 	if (s && hipStreamIsCapturing(s, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone)
 	{	/* events from outside the graph have no place in it */
 		capturedQueries = true;
-		return nullptr;
+		return QueryMark();
 	}
+	if (s && queryOnNull) markNullQuery();
 	if (queryRecorded) hipCheck(hipStreamWaitEvent(s, queryEv, 0), "wait");
 	if (framePending) hipCheck(hipStreamWaitEvent(s, frameEv, 0), "wait");
-	return queryEv;
+	return QueryMark{ s ? queryEv : nullptr, true };
+}
+
+void RenderCore::endQuery(hipStream_t s, const QueryMark& mark, bool bounce)
+{
+	if (!mark.ordered) return;
+	queryPending = true, bouncePending |= bounce;
+	queryOnNull = !s, queryRecorded = s != nullptr;
+}
+
+void RenderCore::markNullQuery()
+{
+	hipCheck(hipEventRecord(queryEv, nullptr), "event");
+	queryOnNull = false, queryRecorded = true;
 }
 
 void RenderCore::waitQueries()
 {
 	if (capturedQueries) hipCheck(hipDeviceSynchronize(), "sync");
-	else if (queryPending) hipCheck(hipStreamWaitEvent(stream, queryEv, 0), "wait");
+	else if (queryPending)
+	{
+		if (queryOnNull) markNullQuery();
+		hipCheck(hipStreamWaitEvent(stream, queryEv, 0), "wait");
+	}
 	queryPending = bouncePending = false;
 }
 
@@ -756,10 +774,10 @@ void RenderCore::TraceClosest(const void* rays, void* hits, int count, hipStream
 {
 	if (count < 0 || (count > 0 && (!rays || !hits))) throw CoreError(LH2HIP_ERR_INVALID, "trace: bad arguments");
 	const TraceScene& sc = Scene();
-	const hipEvent_t done = beginQuery(s);
+	const QueryMark mark = beginQuery(s);
 	hipCheck(launch_trace_dev(sc, MODE_CLOSEST, (const float4*)rays, hits, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s,
-		nullptr, done), "trace");
-	if (done && count > 0) queryPending = queryRecorded = true;
+		nullptr, mark.done), "trace");
+	if (count > 0) endQuery(s, mark);
 }
 
 void RenderCore::TraceClosestCounted(const void* rays, void* hits, int count, hipStream_t s, uint64_t* out2)
@@ -787,21 +805,21 @@ void RenderCore::TraceAny(const void* rays, uint32_t* mask, int count, hipStream
 {
 	if (count < 0 || (count > 0 && (!rays || !mask))) throw CoreError(LH2HIP_ERR_INVALID, "trace: bad arguments");
 	const TraceScene& sc = Scene();
-	const hipEvent_t done = beginQuery(s);
-	hipCheck(hipMemsetAsync(mask, 0, sizeof(uint32_t) * ((count + 31) / 32), s), "memset");
+	const QueryMark mark = beginQuery(s);
+	hipCheck(clear_words(mask, (int)(((int64_t)count + 31) / 32), s, mark.done), "clear");
 	hipCheck(launch_trace_dev(sc, MODE_ANY_MASK, (const float4*)rays, mask, count, nullptr, counters.as<uint32_t>(), overflow.as<uint32_t>(), blocksFor(count), s,
-		nullptr, done), "trace");
-	if (done && count > 0) queryPending = queryRecorded = true;
+		nullptr, mark.done), "trace");
+	if (count > 0) endQuery(s, mark);
 }
 
 void RenderCore::Bounce(const void* raysIn, const void* hits, const uint32_t* pathIn, int count, uint32_t R0, float tmin,
 	void* raysOut, uint32_t* pathOut, uint32_t* countOut, hipStream_t s)
 {
 	Scene();
-	const hipEvent_t done = beginQuery(s);
+	const QueryMark mark = beginQuery(s);
 	hipCheck(launch_bounce(shadeInsts.as<ShadeInst>(), (const float4*)raysIn, (const float4*)hits, pathIn, count, R0, tmin,
-		(float4*)raysOut, pathOut, countOut, s, done), "bounce");
-	if (done && count > 0) queryPending = queryRecorded = bouncePending = true;
+		(float4*)raysOut, pathOut, countOut, s, mark.done), "bounce");
+	if (count > 0) endQuery(s, mark, true);
 }
 
 void RenderCore::BvhInfo(int mesh, int64_t* o) const

@@ -49,11 +49,13 @@ RenderServer::RenderServer(RenderCore& c, uint64_t budgetBytes, size_t pp) : cor
 	check(hipGetDevice(&device), "hipGetDevice");
 	check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
 	queue.ensure(TRACE_QUEUE_WORDS * sizeof(uint32_t));
+	check(hipMemsetAsync(queue.p, 0, queue.bytes, stream), "memset");
 	ovf.ensure(trace_overflow_bytes(core.traceBlocks()));
 	check(hipStreamCreateWithFlags(&stream2, hipStreamNonBlocking), "hipStreamCreate");
 	for (int i = 0; i < 2; i++) check(hipEventCreateWithFlags(&laneEv[i], hipEventDisableTiming), "hipEventCreate");
 	for (int i = 0; i < 4; i++) check(hipEventCreate(&passEv[i]), "hipEventCreate");
 	laneScratch.ensure((4 + TRACE_QUEUE_WORDS) * sizeof(uint32_t));
+	check(hipMemsetAsync(laneScratch.p, 0, laneScratch.bytes, stream), "memset");
 	laneOvf.ensure(trace_overflow_bytes(core.traceBlocks()));
 	segs.ensure(sizeof(JobSeg) * JOB_SEGS_MAX);
 	check(hipHostMalloc((void**)&segsHost, sizeof(JobSeg) * JOB_SEGS_MAX, hipHostMallocDefault), "hipHostMalloc");

@@ -39,7 +39,8 @@ struct TraceStats
 /* rays: Ray4 {O.xyz, tmin; D.xyz, tmax}. out: MODE_CLOSEST -> float4 hit records;
  * MODE_ANY_MASK -> uint32 bitmask (must be zeroed); MODE_ANY_FLAG -> uint32 per ray.
  * overflow: device overflow stack (see trace_overflow_bytes), queue:
- * TRACE_QUEUE_WORDS uint32 ray-feed counters (cleared by the call). */
+ * TRACE_QUEUE_WORDS uint32 ray-feed counters, zero between launches (a launch
+ * clears them behind itself). */
 hipError_t launch_trace(const TraceScene& s, int mode, const float4* rays, void* out, int count,
 	uint32_t* queue, uint32_t* overflow, int persistentBlocks, hipStream_t stream, TraceStats* statsDev = nullptr);
 /* As launch_trace, with the ray count read by the kernel from countDev
@@ -49,6 +50,9 @@ hipError_t launch_trace_dev(const TraceScene& s, int mode, const float4* rays, v
 	uint32_t* queue, uint32_t* overflow, int persistentBlocks, hipStream_t stream, TraceStats* statsDev = nullptr,
 	hipEvent_t done = nullptr);
 size_t trace_overflow_bytes(int persistentBlocks);
+/* p[0] .. p[n - 1] = 0 by a kernel (a memset recorded into a graph may not clear
+ * on every replay); done as above. */
+hipError_t clear_words(uint32_t* p, int n, hipStream_t stream, hipEvent_t done = nullptr);
 
 static const int TRACE_TRI_PAD = 3;                 /* records that may be read (and are ignored) past a mesh's last leaf triangle */
 static const int TRACE_BLOCK = 256;
@@ -58,8 +62,7 @@ static const int TRACE_MAX_STACK = TRACE_LDS_STACK + TRACE_OVF_STACK;
 static const uint32_t TRACE_MAX_STEPS = 1u << 26;   /* node visits per ray (safety bound) */
 /* Ray feed: the rays of a launch are split into TRACE_QUEUES contiguous
  * ranges, each handed out by its own counter (TRACE_QSTRIDE words apart, so
- * the counters sit on separate cache lines). A launch needs a zeroed area of
- * TRACE_QUEUE_WORDS words; launch_trace clears it on the stream. */
+ * the counters sit on separate cache lines). */
 static const int TRACE_QUEUES = 8;
 static const int TRACE_QSTRIDE = 64;
 static const int TRACE_QUEUE_WORDS = TRACE_QUEUES * TRACE_QSTRIDE;

@@ -789,9 +789,29 @@ size_t trace_overflow_bytes(int persistentBlocks)
 	return (size_t)persistentBlocks * TRACE_BLOCK * TRACE_OVF_STACK * sizeof(uint32_t);
 }
 
-__global__ void k_reset_queue(uint32_t* q)
+/* A launch, with an event that stands for the kernel's own end if one is given: a
+ * record behind the kernel costs the stream 3-5 us (4,096 rays over 20k triangles
+ * 85.5 -> 90.9 us a query). A kernel's own completion signal costs nothing measurable
+ * where every kernel of the stream has one, 4 us on a long kernel behind one without,
+ * 1.4 on a short one behind a long one: so all kernels of a small query carry the
+ * event, and a large one's is on the clearing of its feed. */
+template <typename K, typename... Args>
+static void launch_with(K kernel, int blocks, int threads, hipStream_t stream, hipEvent_t done, Args... args)
 {
-	for (int i = threadIdx.x; i < TRACE_QUEUE_WORDS; i += blockDim.x) q[i] = 0u;
+	if (done) hipExtLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, stream, nullptr, done, 0, args...);
+	else kernel<<<blocks, threads, 0, stream>>>(args...);
+}
+
+__global__ void __launch_bounds__(256) k_clear_words(uint32_t* __restrict__ p, int n)
+{
+	for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) p[i] = 0u;
+}
+
+hipError_t clear_words(uint32_t* p, int n, hipStream_t stream, hipEvent_t done)
+{
+	if (n <= 0) return hipSuccess;
+	launch_with(k_clear_words, std::min((n + 255) / 256, 1024), 256, stream, done, p, n);
+	return hipGetLastError();
 }
 
 /* Blocks of a kernel that stay resident on the whole device: a persistent
@@ -813,60 +833,50 @@ static int resident_blocks(const void* fn)
 	return n;
 }
 
-/* A launch, with an event that stands for the kernel's own end if one is given: a
- * record behind the kernel costs the stream 3-5 us (4,096 rays over 20k triangles
- * 85.5 -> 90.9 us a query), the kernel's own completion signal nothing measurable. */
-template <typename K, typename... Args>
-static void launch_with(K kernel, int blocks, int threads, hipStream_t stream, hipEvent_t done, Args... args)
-{
-	if (done) hipExtLaunchKernelGGL(kernel, dim3(blocks), dim3(threads), 0, stream, nullptr, done, 0, args...);
-	else kernel<<<blocks, threads, 0, stream>>>(args...);
-}
-
 template <typename K>
 static void go(K kernel, const TraceScene& s, const float4* rays, void* out, int count, const uint32_t* countDev, uint32_t* queue, uint32_t* overflow,
-	int blocks, hipStream_t stream, TraceStats* stats, hipEvent_t done)
+	int blocks, hipStream_t stream, TraceStats* stats)
 {
 	blocks = std::max(1, std::min(blocks, resident_blocks((const void*)kernel)));
-	launch_with(kernel, blocks, TRACE_BLOCK, stream, done, s, rays, out, count, countDev, queue, overflow, stats);
+	kernel<<<blocks, TRACE_BLOCK, 0, stream>>>(s, rays, out, count, countDev, queue, overflow, stats);
 }
 
 template <int FMT, int MODE, bool TWO>
 static void launch3(const TraceScene& s, const float4* rays, void* out, int count, const uint32_t* countDev, uint32_t* queue, uint32_t* overflow,
-	int blocks, hipStream_t stream, TraceStats* stats, hipEvent_t done)
+	int blocks, hipStream_t stream, TraceStats* stats)
 {
 	if (s.loop == LOOP_GREEDY)
 	{
-		if (stats) go(k_trace_greedy<FMT, MODE, TWO, true>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
-		else go(k_trace_greedy<FMT, MODE, TWO, false>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
+		if (stats) go(k_trace_greedy<FMT, MODE, TWO, true>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
+		else go(k_trace_greedy<FMT, MODE, TWO, false>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
 	}
 	else if (s.loop == LOOP_WHILE_WHILE)
 	{
-		if (stats) go(k_trace_ww<FMT, MODE, TWO, true>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
-		else go(k_trace_ww<FMT, MODE, TWO, false>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
+		if (stats) go(k_trace_ww<FMT, MODE, TWO, true>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
+		else go(k_trace_ww<FMT, MODE, TWO, false>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
 	}
 	else
 	{
-		if (stats) go(k_trace_merged<FMT, MODE, TWO, true>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
-		else go(k_trace_merged<FMT, MODE, TWO, false>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
+		if (stats) go(k_trace_merged<FMT, MODE, TWO, true>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
+		else go(k_trace_merged<FMT, MODE, TWO, false>, s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
 	}
 }
 
 template <int FMT, int MODE>
 static void launch2(const TraceScene& s, const float4* rays, void* out, int count, const uint32_t* countDev, uint32_t* queue, uint32_t* overflow,
-	int blocks, hipStream_t stream, TraceStats* stats, hipEvent_t done)
+	int blocks, hipStream_t stream, TraceStats* stats)
 {
-	if (s.twoLevel) launch3<FMT, MODE, true>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
-	else launch3<FMT, MODE, false>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
+	if (s.twoLevel) launch3<FMT, MODE, true>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
+	else launch3<FMT, MODE, false>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
 }
 
 template <int FMT>
 static void launch1(const TraceScene& s, int mode, const float4* rays, void* out, int count, const uint32_t* countDev, uint32_t* queue, uint32_t* overflow,
-	int blocks, hipStream_t stream, TraceStats* stats, hipEvent_t done)
+	int blocks, hipStream_t stream, TraceStats* stats)
 {
-	if (mode == MODE_CLOSEST) launch2<FMT, MODE_CLOSEST>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
-	else if (mode == MODE_ANY_MASK) launch2<FMT, MODE_ANY_MASK>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
-	else launch2<FMT, MODE_ANY_FLAG>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats, done);
+	if (mode == MODE_CLOSEST) launch2<FMT, MODE_CLOSEST>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
+	else if (mode == MODE_ANY_MASK) launch2<FMT, MODE_ANY_MASK>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
+	else launch2<FMT, MODE_ANY_FLAG>(s, rays, out, count, countDev, queue, overflow, blocks, stream, stats);
 }
 
 /* Launches of at most this many rays take four lanes per ray. Incoherent
@@ -902,10 +912,9 @@ hipError_t launch_trace_dev(const TraceScene& s, int mode, const float4* rays, v
 		else launch_quad<MODE_ANY_FLAG>(s, rays, out, maxCount, countDev, overflow, stream, done);
 		return hipGetLastError();
 	}
-	k_reset_queue<<<1, 256, 0, stream>>>(queue);
-	if (s.format == FMT_Q8) launch1<FMT_Q8>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats, done);
-	else launch1<FMT_F32>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats, done);
-	return hipGetLastError();
+	if (s.format == FMT_Q8) launch1<FMT_Q8>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats);
+	else launch1<FMT_F32>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats);
+	return clear_words(queue, TRACE_QUEUE_WORDS, stream, done);
 }
 
 hipError_t launch_trace(const TraceScene& s, int mode, const float4* rays, void* out, int count,

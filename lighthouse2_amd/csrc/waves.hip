@@ -9,6 +9,7 @@
  * survivors are compacted through an atomic counter.
  */
 #include "waves.h"
+#include "trace.h"
 #include <hip/hip_ext.h>
 #include "sample.h"
 
@@ -81,7 +82,7 @@ hipError_t launch_primary(const CamParams& c, uint32_t R0, float tmin, float4* r
 hipError_t launch_bounce(const ShadeInst* inst, const float4* raysIn, const float4* hits, const uint32_t* pathIn, int n,
 	uint32_t R0, float tmin, float4* raysOut, uint32_t* pathOut, uint32_t* counter, hipStream_t s, hipEvent_t done)
 {
-	hipError_t e = hipMemsetAsync(counter, 0, sizeof(uint32_t), s);
+	const hipError_t e = clear_words(counter, 1, s, done);
 	if (e != hipSuccess || n <= 0) return e;
 	const int blocks = (n + BOUNCE_BLOCK - 1) / BOUNCE_BLOCK;
 	if (done) hipExtLaunchKernelGGL(k_bounce, dim3(blocks), dim3(BOUNCE_BLOCK), 0, s, nullptr, done, 0, inst, raysIn, hits, pathIn, n, R0, tmin, raysOut, pathOut, counter);

@@ -52,12 +52,14 @@ def launch(torch, core, stream, kind, rays):
 @pytest.mark.parametrize("n", [3000, MANY])
 @pytest.mark.parametrize("two_level", [False, True])
 @pytest.mark.parametrize("update", ["rebuild", "refit", "move"])
-def test_update_after_query(torch_cuda, update, two_level, n, kind):
+@pytest.mark.parametrize("own", [True, False], ids=["own stream", "null stream"])
+def test_update_after_query(torch_cuda, own, update, two_level, n, kind):
     torch = torch_cuda
     v = meshes()
     core = make(torch, two_level, int(update == "refit"), v[0])
     rays = torch.from_numpy(_random_rays(np.random.default_rng(n), n, -2, 2)).cuda()
-    stream = torch.cuda.Stream()
+    stream = torch.cuda.Stream() if own else torch.cuda.default_stream()
+    assert own == (stream.cuda_stream != 0)
     want = launch(torch, core, torch.cuda.current_stream(), kind, rays)
     torch.cuda.synchronize()
     want = want.cpu()
@@ -75,14 +77,15 @@ def test_update_after_query(torch_cuda, update, two_level, n, kind):
     core.Shutdown()
 
 
-def test_update_after_bounce(torch_cuda):
+@pytest.mark.parametrize("own", [True, False], ids=["own stream", "null stream"])
+def test_update_after_bounce(torch_cuda, own):
     torch = torch_cuda
     v = meshes()
     core = make(torch, False, 0, v[0])
     rays = torch.from_numpy(_random_rays(np.random.default_rng(1), 5000)).cuda()
     hits = launch(torch, core, torch.cuda.current_stream(), "closest", rays).view(torch.float32)
     ids = torch.arange(len(rays), dtype=torch.int32, device="cuda")
-    stream = torch.cuda.Stream()
+    stream = torch.cuda.Stream() if own else torch.cuda.default_stream()
 
     def bounce():
         out, path, cnt = torch.zeros_like(rays), torch.zeros_like(ids), torch.zeros(1, dtype=torch.int32, device="cuda")
@@ -108,8 +111,9 @@ def test_update_after_bounce(torch_cuda):
     core.Shutdown()
 
 
-def test_queries_on_several_streams(torch_cuda):
-    """They share the ray feed and the stacks' overflow area."""
+@pytest.mark.parametrize("late", [0, 1, 2])
+def test_queries_on_several_streams(torch_cuda, late):
+    """They share the ray feed and the stacks' overflow area; one of the streams is the null stream."""
     torch = torch_cuda
     core = make(torch, True, 0, meshes()[0])
     rays = [torch.from_numpy(_random_rays(np.random.default_rng(k), MANY, -2, 2)).cuda() for k in range(4)]
@@ -117,10 +121,10 @@ def test_queries_on_several_streams(torch_cuda):
     for r in rays:
         want.append(launch(torch, core, torch.cuda.current_stream(), "closest", r))
         torch.cuda.synchronize()
-    streams = [torch.cuda.Stream() for _ in rays]
+    streams = [torch.cuda.Stream(), torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.default_stream()]
     out = [torch.zeros((MANY, 4), dtype=torch.int32, device="cuda") for _ in rays]
     torch.cuda.synchronize()
-    held(torch, streams[1])                          # the second one late, the others at once
+    held(torch, streams[late])                       # one late, the others at once
     for s, r, o in zip(streams, rays, out):
         core.trace_closest(r.data_ptr(), o.data_ptr(), MANY, s.cuda_stream)
     torch.cuda.synchronize()
@@ -128,7 +132,8 @@ def test_queries_on_several_streams(torch_cuda):
     core.Shutdown()
 
 
-def test_query_beside_frames(torch_cuda):
+@pytest.mark.parametrize("own", [True, False], ids=["own stream", "null stream"])
+def test_query_beside_frames(torch_cuda, own):
     """A frame that is not waited for, and a query that still waits when a frame begins."""
     torch = torch_cuda
     s = scenes.cornell_box(sphere_tris=2000)
@@ -137,7 +142,7 @@ def test_query_beside_frames(torch_cuda):
     core.SetTarget(640, 400, 1)
     view = scenes.cornell_view(640, 400)
     rays = torch.from_numpy(_random_rays(np.random.default_rng(4), MANY, -2, 2)).cuda()
-    stream = torch.cuda.Stream()
+    stream = torch.cuda.Stream() if own else torch.cuda.default_stream()
     want = launch(torch, core, torch.cuda.current_stream(), "closest", rays)
     core.Render(view, lh.LH2_RESTART)
     image = core.read_image()
@@ -178,4 +183,31 @@ def test_query_in_a_graph(torch_cuda):
     core.FinalizeInstances()
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+    core.Shutdown()
+
+
+def test_cleared_outputs_in_a_graph(torch_cuda):
+    """An any-hit query and a bounce clear their outputs on every replay, with other work between the replays."""
+    torch = torch_cuda
+    core = make(torch, True, 0, meshes()[0])
+    rays = torch.from_numpy(_random_rays(np.random.default_rng(8), 3001, -2, 2)).cuda()
+    n = len(rays)
+    want = launch(torch, core, torch.cuda.current_stream(), "any", rays).clone()
+    hits = launch(torch, core, torch.cuda.current_stream(), "closest", rays).view(torch.float32)
+    torch.cuda.synchronize()
+    found = int((hits.view(torch.int32)[:, 2] >= 0).sum())
+    mask, cnt = torch.zeros_like(want), torch.zeros(1, dtype=torch.int32, device="cuda")
+    ids = torch.arange(n, dtype=torch.int32, device="cuda")
+    out, path = torch.zeros((n + 50, 8), device="cuda"), torch.zeros(n + 50, dtype=torch.int32, device="cuda")   # room for a count that was not cleared
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        s = torch.cuda.current_stream().cuda_stream
+        core.trace_any(rays.data_ptr(), mask.data_ptr(), n, s)
+        core.bounce_diffuse(rays.data_ptr(), hits.data_ptr(), ids.data_ptr(), n, 7, 1e-4, out.data_ptr(), path.data_ptr(), cnt.data_ptr(), s)
+    for k in range(5):
+        mask.fill_(-1), cnt.fill_(50)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(mask, want) and int(cnt) == found, k
+        launch(torch, core, torch.cuda.current_stream(), "any", rays[: 100 + k])
     core.Shutdown()
