@@ -592,7 +592,8 @@ def bench_extend(a, np, torch, lh, scenes):
     prim_ms = sum(m[0] for m in ms)
     value = inco_rays / (inco_ms * 1e-3) / 1e6
 
-    # algorithmic work per incoherent ray, counted by the kernel on the same rays (untimed)
+    # algorithmic work per incoherent ray, counted on the same rays (untimed) by the variant that walks a ray with one
+    # lane to its end: the tail figures are those of that variant, not of the timed kernel's four-lane end
     keep = []
     wv.step(keep=keep)
     torch.cuda.synchronize()

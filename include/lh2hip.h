@@ -141,8 +141,11 @@ LH2HIP_API int lh2hip_trace_any(lh2hip_core* core, const Ray4* rays, uint32_t* o
  * holding a ray in them while rays remain to be fetched, [8]/[9] the same
  * once all rays are handed out, [10] ns from the first wave's start until the
  * last ray was handed out, [11] ns from the first start to the last wave's
- * end. A separate kernel variant; used to derive algorithmic bytes per ray,
- * SIMD utilisation and the share of the launch spent after the feed ran dry. */
+ * end. A separate kernel variant, which walks every ray with one lane from start
+ * to end: lh2hip_trace_closest gives four lanes to each ray of a launch of at most
+ * 131,072 and to a wave's last 16 once the feed is dry, so [8] to [11] describe a
+ * longer end than it has. Used to derive algorithmic bytes per ray, SIMD
+ * utilisation and the share of the launch spent after the feed ran dry. */
 LH2HIP_API int lh2hip_trace_closest_counted(lh2hip_core* core, const Ray4* rays, HitRecord* hits, int count, void* stream,
 	uint64_t* out12);
 

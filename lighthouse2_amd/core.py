@@ -266,7 +266,10 @@ class RenderCore:
         steps of all waves, lanes visiting a node in them, leaf steps, lanes
         testing a triangle in them, loop iterations and lanes holding a ray
         while rays remain, the same after the last ray was handed out, ns
-        from the first wave's start to the feed running dry, ns to the end)."""
+        from the first wave's start to the feed running dry, ns to the end).
+        Every ray is walked by one lane to its end: the figures after the last
+        ray was handed out are not trace_closest's, which gives a wave's last
+        16 rays four lanes each."""
         out = np.zeros(12, np.uint64)
         _check(library().lh2hip_trace_closest_counted(self._h, rays_ptr, hits_ptr, count, stream, _p(out)))
         return tuple(int(x) for x in out)

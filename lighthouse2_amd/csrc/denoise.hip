@@ -177,12 +177,12 @@ __device__ __forceinline__ uint32_t relu_mask2(uint32_t act, uint32_t g)
  * under the other's products (a block per tile: 121 us for the decoder's first
  * convolution at 1920 x 1088, 100 -> 151 us for its gradient). With fewer weights
  * three blocks a CU hide the loads better than a loop does.
- *   Measured at 1920 x 1088 (a wave per row -> now; the bytes each must move at a
- * copy's 5.06 TB/s): 16 -> 32 58 -> 42 us (40), 32 -> 32 76 -> 44 (53, partly from the
- * cache), 32 -> 32 with pooling 117 -> 65 (59), 64 -> 32 175 -> 81 (59), 32 -> 16 float
- * 49 -> 37 (53), display 71 -> 51; gradients 32 -> 32 110 -> 88 (79), 32 -> 64 187 -> 101
- * (66). Memory bounds all but the 64-channel ones, which wait for it between their
- * tiles' products as well. */
+ *   Measured within forward passes and training steps at 1920 x 1088 (kernel trace;
+ * in brackets the bytes a layer must move at a copy's 5.06 TB/s): 16 -> 32 55 us (40),
+ * 32 -> 32 66 (53), with pooling 70 (59), 64 -> 32 89 (59), 32 -> 16 float 54 (53), display
+ * 52; gradients 32 -> 32 94 (79), 16 -> 32 89 (66), 32 -> 64 104 (66). With a wave per row
+ * the whole forward pass took 715 us where it now takes 450 to 475. Memory bounds all
+ * but the 64-channel ones, which wait for it between their tiles' products as well. */
 template <int CIN, int NB, bool RELU, bool F32OUT, bool CAT, bool POOL, int IO, int MBW>
 __global__ void __launch_bounds__(256, NB == 4 || CIN == 64 ? 2 : 3) k_conv_rows(const bf16_t* __restrict__ x, const bf16_t* __restrict__ coarse,
 	const bf16_t* __restrict__ w, const float* __restrict__ bias, void* __restrict__ y, int H, int W, bf16_t* __restrict__ ypool,
@@ -800,8 +800,8 @@ hipError_t dn_conv3x3_dx_cat(const bf16_t* gy, const bf16_t* w, const bf16_t* ac
  * halves, the coarse one read from the coarse tensor (row and pixel halved).
  * The 19 layers of the network at 1088 x 1920 (1.7 GB of inputs and gradients,
  * 340 us at a copy's rate): 1,034 us and 413 us for partial sums with 9-wave
- * blocks that transposed while staging and a launch per layer, 471 and 22 us
- * now; at 256 x 256 362 us in all, now 41. */
+ * blocks that transposed while staging and a launch per layer, 466 and 22 us
+ * now; at 256 x 256 362 us in all, now 40. */
 typedef __bf16 bf8v_dw __attribute__((ext_vector_type(8)));
 typedef short s4x __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s4x lds_s4x;

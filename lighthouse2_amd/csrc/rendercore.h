@@ -228,7 +228,9 @@ private:
 	DevBuf tlasNodes, instRecs, shadeInsts;
 	TraceScene scene;
 	/* workspace of builds and layouts, kept between calls up to BUILD_WS_KEEP
-	 * bytes (a mesh of about 1.2 M triangles); used under the scene lock, on `stream` */
+	 * bytes; used under the scene lock, on `stream`. A mesh needs 46 bytes a triangle
+	 * to build and 52 per build node (at most two a triangle) to be laid out, so none
+	 * below 2.5 M triangles is given back. */
 	DevBuf buildWs, maxMatB;           /* maxMatB: one word, largest material of a mesh being set */
 	static constexpr size_t BUILD_WS_KEEP = (size_t)256 << 20;
 	void trimBuildWorkspace();

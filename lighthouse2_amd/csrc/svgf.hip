@@ -263,9 +263,9 @@ __global__ void k_prepare(const float4* __restrict__ acc, const uint4* __restric
  * square) and stages 20 x 20 pixels whatever the distance: 25.6 KB, where the
  * square of the last pass would need 64 KB. Lattices that share cache lines (same
  * rows) run one after the other on one XCD (blocks are dealt to the 8 XCDs round
- * robin). A 1920 x 1080 pass takes 111 us (the first, with its history, 161), of
- * which VALU issue is 95; it was 187 to 288 us with every tap read and decoded
- * from memory. */
+ * robin). A 1920 x 1080 pass takes 90 us within a session's frames (the first, with
+ * its history, 134), at full VALU issue; filtering frame after frame 104 and 153, at a
+ * lower clock. It was 187 to 288 us with every tap read and decoded from memory. */
 template <int STEP, bool LAST>
 __global__ void __launch_bounds__(256) k_apply(const uint4* __restrict__ features, const float4* __restrict__ prevWorldPos, const float4* __restrict__ worldPos,
 	const float4* __restrict__ deltaDepth, const float2* __restrict__ motion, const float4* __restrict__ moments,

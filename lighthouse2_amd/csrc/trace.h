@@ -27,8 +27,9 @@ struct TraceScene
 	int triBias = 16;   /* greedy loop: a leaf step when (triBias / 16) x pending-leaf lanes > node lanes */
 };
 
-/* Work counters of the counting kernel variant: node visits and triangle
- * tests per ray, and per wave the loop iterations and the lanes active in
+/* Work counters of the counting kernel variant, which walks every ray with one lane
+ * from start to end, whatever their number (without the four-lane launch of few rays
+ * and the four-lane end of a wave's last ones): node visits and triangle tests per ray, and per wave the loop iterations and the lanes active in
  * them (SIMD utilisation = lanes / (64 * iterations)). */
 struct TraceStats
 {

@@ -316,7 +316,9 @@ __device__ __forceinline__ uint32_t quad_bits(uint64_t m, int lane)
 	return ((lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32)) >> (lane & 28)) & 15u;
 }
 
-/* visit_q8 with a child per lane: the same planes, widening and tests. */
+/* visit_q8 with a child per lane: the same planes and tests, each plane widened by the
+ * rounded product of w and the span (visit_q8 fuses it into the add): both keep every
+ * box that the exact interval reaches, so hits are the same. */
 template <typename STACK>
 __device__ __forceinline__ void visit_quad(const NodeQ8* node, float w, int c, int lane, const Lane& L, STACK& st, uint32_t& ref)
 {
