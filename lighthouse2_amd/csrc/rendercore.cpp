@@ -588,6 +588,7 @@ void RenderCore::FinalizeInstances()
 void RenderCore::updateTopLevel()
 {
 	if (!instancesDirty) return;
+	requireNoJobs("scene update");     /* their passes hold pointers into what is rewritten here */
 	const int ni = (int)instances.size();
 	std::vector<InstanceRec> recs(ni);
 	std::vector<ShadeInst> sh(ni);
@@ -725,7 +726,11 @@ int RenderCore::blocksFor(int count) const
 
 const TraceScene& RenderCore::Scene()
 {
-	updateTopLevel();
+	if (instancesDirty)
+	{
+		std::unique_lock<std::shared_mutex> lockScene(sceneMutex);
+		updateTopLevel();
+	}
 	if (!sceneReady) throw CoreError(LH2HIP_ERR_STATE, "no scene: call SetGeometry, SetInstance and FinalizeInstances first");
 	return scene;
 }

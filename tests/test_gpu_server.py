@@ -317,3 +317,32 @@ def test_learned_job_needs_weights(torch_cuda):
         srv.set_denoiser(b"\0" * 16)              # wrong size
     srv.close()
     core.Shutdown()
+
+
+def test_unfinished_scene_changes_wait_for_the_jobs(torch_cuda):
+    """An instance moved but not finalised when a job is submitted: a query or a frame that would rewrite the tables under the
+    job's passes is refused until the job is done, and the job's image is that of the scene it was submitted on."""
+    torch = torch_cuda
+    s = scenes.cornell_box(sphere_tris=2000)
+    core = lh.RenderCore()
+    lh.load_scene(core, s)
+    core.SetTarget(64, 48, 1)
+    view = scenes.cornell_view(256, 192)
+    ref, _ = solo(s, view, 256, 192, 512, 3, 77)
+    srv = lh.RenderServer(core, budget_bytes=1 << 30, pass_paths=1 << 16)
+    T = np.eye(4, dtype=np.float32)
+    T[0, 3] = 0.05
+    core.SetInstance(0, s.instances[0][0], T)
+    j = srv.submit(view, 256, 192, spp=512, max_depth=3, seed=77)
+    rays, hits = torch.zeros((8, 8), device="cuda"), torch.zeros((8, 4), device="cuda")
+    with pytest.raises(lh.LH2HIPError, match="pending"):
+        core.trace_closest(rays.data_ptr(), hits.data_ptr(), 8)
+    with pytest.raises(lh.LH2HIPError, match="pending"):
+        core.Render(view, lh.LH2_RESTART)
+    srv.wait(j, timeout=120)
+    assert np.array_equal(srv.read(j), ref)
+    core.trace_closest(rays.data_ptr(), hits.data_ptr(), 8)
+    torch.cuda.synchronize()
+    core.Render(scenes.cornell_view(64, 48), lh.LH2_RESTART)
+    srv.close()
+    core.Shutdown()
