@@ -916,7 +916,8 @@ hipError_t launch_trace_dev(const TraceScene& s, int mode, const float4* rays, v
 	}
 	if (s.format == FMT_Q8) launch1<FMT_Q8>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats);
 	else launch1<FMT_F32>(s, mode, rays, out, maxCount, countDev, queue, overflow, blocks, stream, stats);
-	return clear_words(queue, TRACE_QUEUE_WORDS, stream, done);
+	const hipError_t e = hipGetLastError(), c = clear_words(queue, TRACE_QUEUE_WORDS, stream, done);
+	return e != hipSuccess ? e : c;
 }
 
 hipError_t launch_trace(const TraceScene& s, int mode, const float4* rays, void* out, int count,
